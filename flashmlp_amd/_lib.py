@@ -39,6 +39,7 @@ SIGNATURES = {
     "fmlp_act_from_name": (ctypes.c_int, [ctypes.c_char_p]),
     "fmlp_shape_supported": (ctypes.c_int, [_i64, _i64, _i64, _i64, ctypes.c_int]),
     "fmlp_shape_tuned": (ctypes.c_int, [_i64, _i64, ctypes.c_int]),
+    "fmlp_shape_dense": (ctypes.c_int, [_i64, _i64, ctypes.c_int]),
     "fmlp_fwd": (ctypes.c_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, ctypes.c_int, ctypes.c_int, _vp]),
     "fmlp_fwd_strided": (ctypes.c_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64p, _i64p, _i64p,
                                         ctypes.c_int, ctypes.c_int, _vp]),

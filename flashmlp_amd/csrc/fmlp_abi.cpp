@@ -111,6 +111,14 @@ bool fwd_tuned_shape(int64_t D, int64_t E, int io) {
   return tuned_shape(D, E, io) || ((io == FMLP_DTYPE_F16 || io == FMLP_DTYPE_BF16) && D == 256 && E % 8 == 0);
 }
 
+// Dense, 16-byte aligned tensors of these shapes run on kernels of their own: those above, and the
+// same D with E % 8 != 0, whose W1 rows are first copied to 16-byte aligned rows at the start of
+// the workspace (w1_pad_bytes; a call without room for them runs on the generic kernels, which were
+// 2.4 to 14 times slower at every E % 8 != 0 measured, from a 16-row forward to a 16-head training step).
+bool dense_shape(int64_t D, int io) {
+  return (io == FMLP_DTYPE_F16 || io == FMLP_DTYPE_BF16) && (D == 64 || D == 128 || D == 256);
+}
+
 int check_shape(int64_t H, int64_t B, int64_t D, int64_t E, int dtype) {
   if (H < 0 || B < 0 || D < 0 || E < 0)
     return fail(FMLP_ERR_INVALID_ARG, "negative dimension (H=%lld B=%lld D=%lld E=%lld)", (long long)H,
@@ -240,6 +248,8 @@ FMLP_EXPORT int fmlp_shape_supported(int64_t H, int64_t B, int64_t D, int64_t E,
 
 FMLP_EXPORT int fmlp_shape_tuned(int64_t D, int64_t E, int dtype) { return tuned_shape(D, E, io_of(dtype)) ? 1 : 0; }
 
+FMLP_EXPORT int fmlp_shape_dense(int64_t D, int64_t E, int dtype) { return E > 0 && dense_shape(D, io_of(dtype)) ? 1 : 0; }
+
 namespace {
 
 int fwd_impl(const void* x, const void* w1, const void* w2, void* o, int64_t H, int64_t B, int64_t D, int64_t E,
@@ -264,13 +274,21 @@ int fwd_impl(const void* x, const void* w1, const void* w2, void* o, int64_t H, 
   if (!rows) return ok();
   const bool dense = sx == nullptr || (is_dense3(sx, B, D) && is_dense3(sw1, D, E) && is_dense3(sw2, E, D));
   hipError_t e;
-  if (dense && fwd_tuned_shape(D, E, io) && aligned16(x) && aligned16(w1) && aligned16(w2) && aligned16(o)) {
+  const size_t pad = fmlp::w1_pad_bytes(H, D, E);
+  if (dense && dense_shape(D, io) && (pad == 0 || (ws != nullptr && ws_bytes >= pad)) && aligned16(x) &&
+      aligned16(w1) && aligned16(w2) && aligned16(o)) {
     int cus = 0;
     if ((st = num_cus_current(&cus))) return st;
-    fmlp::FwdArgs a{x, w1, w2, o, H, B, D, E, io == FMLP_DTYPE_BF16, act, (dtype & FMLP_OUT_F32) != 0, cus};
-    a.ws = ws;
-    a.ws_bytes = ws != nullptr ? ws_bytes : 0;
-    e = fmlp::launch_fwd(a, (hipStream_t)stream);
+    fmlp::FwdArgs a{x, w1, w2, o, H, B, D, E, io == FMLP_DTYPE_BF16, act, (dtype & FMLP_OUT_F32) != 0, cus,
+                    fmlp::w1_pitch(E)};
+    a.ws = ws != nullptr ? (char*)ws + pad : nullptr;
+    a.ws_bytes = ws != nullptr ? ws_bytes - pad : 0;
+    e = hipSuccess;
+    if (pad > 0) {
+      e = fmlp::launch_pad_w1(w1, ws, H, D, E, (hipStream_t)stream);
+      a.w1 = ws;
+    }
+    if (e == hipSuccess) e = fmlp::launch_fwd(a, (hipStream_t)stream);
   } else {
     fmlp::GenArgs g = gen_args(x, w1, w2, nullptr, o, nullptr, nullptr, nullptr, H, B, D, E, dtype, act);
     if (sx) {
@@ -296,10 +314,10 @@ FMLP_EXPORT int fmlp_fwd(const void* x, const void* w1, const void* w2, void* o,
 }
 
 FMLP_EXPORT size_t fmlp_fwd_workspace_bytes(int64_t H, int64_t B, int64_t D, int64_t E, int dtype) {
-  if (check_shape(H, B, D, E, dtype) != FMLP_OK || !fwd_tuned_shape(D, E, io_of(dtype))) return 0;
+  if (check_shape(H, B, D, E, dtype) != FMLP_OK || !dense_shape(D, io_of(dtype))) return 0;
   int cus = 0;
   if (num_cus_current(&cus) != FMLP_OK) return 0;
-  return fmlp::fwd_plan(H, B, D, E, cus, (size_t)-1).ws_bytes;
+  return fmlp::w1_pad_bytes(H, D, E) + fmlp::fwd_plan(H, B, D, E, cus, (size_t)-1).ws_bytes;
 }
 
 FMLP_EXPORT int fmlp_fwd_ws(const void* x, const void* w1, const void* w2, void* o, int64_t H, int64_t B, int64_t D,
@@ -318,23 +336,27 @@ FMLP_EXPORT int fmlp_fwd_strided(const void* x, const void* w1, const void* w2, 
 
 FMLP_EXPORT size_t fmlp_bwd_workspace_bytes(int64_t H, int64_t B, int64_t D, int64_t E, int dtype) {
   if (check_shape(H, B, D, E, dtype) != FMLP_OK) return 0;
-  // the generic and D = 256 dX programs alone use no workspace
-  if ((dtype & FMLP_BWD_NO_DW) && !tuned_shape(D, E, io_of(dtype))) return 0;
+  const int io = io_of(dtype);
+  const bool own = dense_shape(D, io), no_dw = (dtype & FMLP_BWD_NO_DW) != 0;
+  if (no_dw && (dtype & FMLP_BWD_NO_DX)) return 0;  // nothing to compute
+  // the generic dX programs alone use no workspace, the D = 256 ones only the padded W1
+  const size_t pad = own ? fmlp::w1_pad_bytes(H, D, E) : 0;
+  if (no_dw && !(own && D <= 128)) return pad;
   int cus = 0;
   if (num_cus_current(&cus) != FMLP_OK) return 0;
-  // the generic kernels: the fp32 partials of their dW programs' B split; dense 16-bit D = 256
-  // with E % 8 == 0 runs the D = 256 dW programs, whose split may need more
-  if (!tuned_shape(D, E, io_of(dtype))) {
-    const size_t g = fmlp::gen_plan(H, B, D, E, cus, (size_t)-1).ws_bytes;
-    if (!fwd_tuned_shape(D, E, io_of(dtype))) return g;
-    const size_t w = fmlp::plan_dw256(H, B, E, (dtype & FMLP_DW_HILO) != 0, cus, (size_t)-1).ws_bytes;
-    return w > g ? w : g;
+  // the generic kernels (also views of a shape that is not fmlp_shape_tuned): the fp32 partials
+  // of their dW programs' B split; dense 16-bit D = 256 runs the D = 256 dW programs, whose split
+  // may need more
+  size_t n = tuned_shape(D, E, io) || no_dw ? 0 : fmlp::gen_plan(H, B, D, E, cus, (size_t)-1).ws_bytes;
+  if (!own) return n;
+  if (D == 256) {
+    const size_t w = pad + fmlp::plan_dw256(H, B, E, (dtype & FMLP_DW_HILO) != 0, cus, (size_t)-1).ws_bytes;
+    return w > n ? w : n;
   }
   // the plan depends on the activation, which this query does not take: the largest over them
-  size_t n = 0;
   for (int act = 0; act < 4; ++act) {
     const size_t w =
-        plan_ws_bytes(fmlp::plan_bwd(H, B, D, E, act, (dtype & FMLP_DW_HILO) != 0, dz_mode_of(dtype), cus), dtype);
+        pad + plan_ws_bytes(fmlp::plan_bwd(H, B, D, E, act, (dtype & FMLP_DW_HILO) != 0, dz_mode_of(dtype), cus), dtype);
     if (w > n) n = w;
   }
   return n;
@@ -374,7 +396,7 @@ FMLP_EXPORT int fmlp_bwd_plan(int64_t H, int64_t B, int64_t D, int64_t E, int dt
 
 FMLP_EXPORT int fmlp_bwd_stores_dz(int64_t H, int64_t B, int64_t D, int64_t E, int dtype, int act) {
   if (check_shape(H, B, D, E, dtype) != FMLP_OK || check_act(act) != FMLP_OK) return 0;
-  if (!tuned_shape(D, E, io_of(dtype))) return 0;  // the generic kernels recompute
+  if (!dense_shape(D, io_of(dtype)) || D == 256) return 0;  // the other kernels recompute
   int cus = 0;
   if (num_cus_current(&cus) != FMLP_OK) return 0;
   if (dtype & (FMLP_BWD_NO_DX | FMLP_BWD_NO_DW)) return 0;  // a partial backward stores no dZ
@@ -411,19 +433,40 @@ int bwd_impl(const void* x, const void* w1, const void* w2, const void* dout, vo
   const bool aligned = aligned16(x) && aligned16(w1) && aligned16(w2) && aligned16(dout) && aligned16(dx) &&
                        aligned16(dw1) && aligned16(dw2);
   hipError_t e = hipSuccess;
-  if (dense && aligned && tuned_shape(D, E, io)) {
+  // E % 8 != 0: W1's padded copy at the start of the workspace (or of the static scratch); without
+  // room for it the call runs on the generic kernels
+  const size_t pad = dense && aligned && dense_shape(D, io) ? fmlp::w1_pad_bytes(H, D, E) : 0;
+  const size_t given = noalloc ? fmlp::kScratchBytes
+                               : (workspace != nullptr && aligned16(workspace) ? workspace_bytes : 0);
+  const bool own = dense && aligned && dense_shape(D, io) && (pad == 0 || given >= pad);
+  const void* w1p = w1;
+  if (own && pad > 0) {
+    void* dst = workspace;
+    if (noalloc && (e = fmlp::scratch_current_device(&dst)) != hipSuccess)
+      return fail(FMLP_ERR_HIP, "scratch lookup: %s", hipGetErrorString(e));
+    if ((e = fmlp::launch_pad_w1(w1, dst, H, D, E, (hipStream_t)stream)) != hipSuccess)
+      return fail(FMLP_ERR_HIP, "backward launch: %s", hipGetErrorString(e));
+    w1p = dst;
+  }
+  if (own && D <= 128) {
     int cus = 0;
     if ((st = num_cus_current(&cus))) return st;
     // with a scratch limit the plan only considers B splits (and the stored-dZ form) whose
     // workspace fits it; the unsplit recompute form needs none, so a plan always exists
-    fmlp::BwdPlan plan = fmlp::plan_bwd(H, B, D, E, act, (dtype & FMLP_DW_HILO) != 0, dz_mode_of(dtype), cus,
-                                        noalloc ? fmlp::kScratchBytes : (size_t)-1);
+    const bool hilo = (dtype & FMLP_DW_HILO) != 0;
+    fmlp::BwdPlan plan = fmlp::plan_bwd(H, B, D, E, act, hilo, dz_mode_of(dtype), cus,
+                                        noalloc ? fmlp::kScratchBytes - pad : (size_t)-1);
+    // E % 8 != 0 takes any workspace, as the generic kernels do: a plan that fits it
+    if (pad > 0 && plan_ws_bytes(plan, dtype) > given - pad)
+      plan = fmlp::plan_bwd(H, B, D, E, act, hilo, dz_mode_of(dtype), cus, given - pad);
     // the dW programs alone (FMLP_BWD_NO_DX) need only their fp32 partials, the dX programs
     // alone (FMLP_BWD_NO_DW) only the split ragged tiles' partials, at the workspace's start
     const size_t ws_need = plan_ws_bytes(plan, dtype);
     if (!want_dw) plan.dxs_off = 0;
     void* ws = ws_need > 0 ? workspace : nullptr;
-    if (ws_need > 0) {
+    if (ws_need > 0 && pad > 0) {
+      ws = (char*)w1p + pad;
+    } else if (ws_need > 0) {
       if (noalloc) {
         e = fmlp::scratch_current_device(&ws);
         if (e != hipSuccess) return fail(FMLP_ERR_HIP, "scratch lookup: %s", hipGetErrorString(e));
@@ -433,31 +476,29 @@ int bwd_impl(const void* x, const void* w1, const void* w2, const void* dout, vo
         if (!aligned16(workspace)) return fail(FMLP_ERR_INVALID_ARG, "workspace is not 16-byte aligned");
       }
     }
-    fmlp::BwdArgs a{x, w1, w2, dout, dx, dw1, dw2, H, B, D, E, io == FMLP_DTYPE_BF16, act, ws,
-                    (dtype & FMLP_OUT_F32) != 0, (dtype & FMLP_DW_HILO) != 0, want_dx, want_dw};
+    fmlp::BwdArgs a{x, w1p, w2, dout, dx, dw1, dw2, H, B, D, E, io == FMLP_DTYPE_BF16, act, ws,
+                    (dtype & FMLP_OUT_F32) != 0, hilo, want_dx, want_dw, fmlp::w1_pitch(E)};
     e = fmlp::launch_bwd(a, plan, (hipStream_t)stream);
-  } else if (dense && aligned && fwd_tuned_shape(D, E, io)) {
-    // dense 16-bit D = 256 with E % 8 == 0: the D = 256 dX and dW programs; as on the generic
-    // kernels, the dW programs split B only as far as the given workspace (or the static
-    // scratch) holds their partials
+  } else if (own) {
+    // dense 16-bit D = 256: the D = 256 dX and dW programs; as on the generic kernels, the dW
+    // programs split B only as far as the given workspace (or the static scratch) holds their
+    // partials
     void* ws = nullptr;
     fmlp::Dw256Plan wp{};
     if (want_dw) {
       int cus = 0;
       if ((st = num_cus_current(&cus))) return st;
-      const size_t room = noalloc ? fmlp::kScratchBytes
-                                  : (workspace != nullptr && aligned16(workspace) ? workspace_bytes : 0);
-      wp = fmlp::plan_dw256(H, B, E, (dtype & FMLP_DW_HILO) != 0, cus, room);
+      wp = fmlp::plan_dw256(H, B, E, (dtype & FMLP_DW_HILO) != 0, cus, given - pad);
       if (wp.ws_bytes > 0) {
-        ws = workspace;
-        if (noalloc) {
+        ws = pad > 0 ? (char*)w1p + pad : workspace;
+        if (noalloc && pad == 0) {
           e = fmlp::scratch_current_device(&ws);
           if (e != hipSuccess) return fail(FMLP_ERR_HIP, "scratch lookup: %s", hipGetErrorString(e));
         }
       }
     }
-    fmlp::BwdArgs a{x, w1, w2, dout, dx, dw1, dw2, H, B, D, E, io == FMLP_DTYPE_BF16, act, ws,
-                    (dtype & FMLP_OUT_F32) != 0, (dtype & FMLP_DW_HILO) != 0, want_dx, want_dw};
+    fmlp::BwdArgs a{x, w1p, w2, dout, dx, dw1, dw2, H, B, D, E, io == FMLP_DTYPE_BF16, act, ws,
+                    (dtype & FMLP_OUT_F32) != 0, (dtype & FMLP_DW_HILO) != 0, want_dx, want_dw, fmlp::w1_pitch(E)};
     if (want_dx) e = fmlp::launch_dx256(a, (hipStream_t)stream);
     if (e == hipSuccess && want_dw) e = fmlp::launch_dw256(a, wp, (hipStream_t)stream);
   } else {
@@ -483,9 +524,7 @@ int bwd_impl(const void* x, const void* w1, const void* w2, const void* dout, vo
       // path's workspace (a strided view of a tuned shape) uses what fits of it.
       int cus = 0;
       if ((st = num_cus_current(&cus))) return st;
-      const size_t room = noalloc ? fmlp::kScratchBytes
-                                  : (workspace != nullptr && aligned16(workspace) ? workspace_bytes : 0);
-      const fmlp::GenPlan gp = fmlp::gen_plan(H, B, D, E, cus, room);
+      const fmlp::GenPlan gp = fmlp::gen_plan(H, B, D, E, cus, given);
       if (gp.nS > 1) {
         void* ws = workspace;
         if (noalloc) {

@@ -30,8 +30,8 @@ constexpr int DW_BT = 32;            // rows per streamed subtile
 // and ws1[s][h][d][e], which dw_reduce_kernel sums elementwise.
 template <bool BF16, int D>
 __device__ __forceinline__ void dw_store(const f32x16 (&a1)[D / 32], const f32x16 (&a2)[D / 32], void* __restrict__ dW1,
-                                         void* __restrict__ dW2, float* __restrict__ ws, int H, int E, int h, int s,
-                                         int nS, int e0, int g, int l32, int outf32) {
+                                         void* __restrict__ dW2, float* __restrict__ ws, int H, int E, int ldw, int h,
+                                         int s, int nS, int e0, int g, int l32, int outf32) {
   constexpr int NTN = D / 32;
   if (nS == 1 && outf32) {
     float* dW2h = (float*)dW2 + (size_t)h * E * D;
@@ -45,8 +45,29 @@ __device__ __forceinline__ void dw_store(const f32x16 (&a1)[D / 32], const f32x1
           const int d = nt * 32 + l32;
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
-            dW2h[(size_t)(eb + j) * D + d] = a2[nt][4 * i4 + j];
-            dW1h[(size_t)d * E + eb + j] = a1[nt][4 * i4 + j];
+            if (eb + j < E) {
+              dW2h[(size_t)(eb + j) * D + d] = a2[nt][4 * i4 + j];
+              dW1h[(size_t)d * E + eb + j] = a1[nt][4 * i4 + j];
+            }
+          }
+        }
+      }
+    }
+  } else if (nS == 1 && (E & 3) != 0) {
+    // rows of dW1 that are not 8-byte aligned, and column groups that E cuts
+    u16* dW2h = (u16*)dW2 + (size_t)h * E * D;
+    u16* dW1h = (u16*)dW1 + (size_t)h * D * E;
+#pragma unroll
+    for (int i4 = 0; i4 < 4; ++i4) {
+      const int eb = e0 + 8 * i4 + 4 * g;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (eb + j < E) {
+#pragma unroll
+          for (int nt = 0; nt < NTN; ++nt) {
+            const int d = nt * 32 + l32;
+            dW2h[(size_t)(eb + j) * D + d] = from_f32<BF16>(a2[nt][4 * i4 + j]);
+            dW1h[(size_t)d * E + eb + j] = from_f32<BF16>(a1[nt][4 * i4 + j]);
           }
         }
       }
@@ -56,7 +77,7 @@ __device__ __forceinline__ void dw_store(const f32x16 (&a1)[D / 32], const f32x1
     u16* dW1h = (u16*)dW1 + (size_t)h * D * E;
 #pragma unroll
     for (int i4 = 0; i4 < 4; ++i4) {
-      const int eb = e0 + 8 * i4 + 4 * g;  // 4 consecutive columns eb .. eb+3 (E % 8 == 0)
+      const int eb = e0 + 8 * i4 + 4 * g;  // 4 consecutive columns eb .. eb+3 (E % 4 == 0)
       if (eb < E) {
 #pragma unroll
         for (int nt = 0; nt < NTN; ++nt) {
@@ -69,14 +90,14 @@ __device__ __forceinline__ void dw_store(const f32x16 (&a1)[D / 32], const f32x1
       }
     }
   } else {
-    // fp32 partials in the outputs' own layouts (dW2 [h][e][d], dW1 [h][d][e]), so the
-    // reduction is an elementwise sum over the nS slices
-    const size_t per = (size_t)H * E * D;
-    float* p2 = ws + ((size_t)s * H + h) * E * D;
-    float* p1 = ws + (size_t)nS * per + ((size_t)s * H + h) * D * E;
+    // fp32 partials in the outputs' own layouts (dW2 [h][e][d], dW1 [h][d][e]) with E rounded up
+    // to ldw, so the reduction is an elementwise sum over the nS slices
+    const size_t per = (size_t)H * ldw * D;
+    float* p2 = ws + ((size_t)s * H + h) * ldw * D;
+    float* p1 = ws + (size_t)nS * per + ((size_t)s * H + h) * D * ldw;
 #pragma unroll
     for (int i4 = 0; i4 < 4; ++i4) {
-      const int eb = e0 + 8 * i4 + 4 * g;  // 4 consecutive columns eb .. eb+3 (E % 8 == 0)
+      const int eb = e0 + 8 * i4 + 4 * g;  // 4 consecutive columns eb .. eb+3 (ldw % 8 == 0)
       if (eb < E) {
 #pragma unroll
         for (int nt = 0; nt < NTN; ++nt) {
@@ -84,7 +105,7 @@ __device__ __forceinline__ void dw_store(const f32x16 (&a1)[D / 32], const f32x1
 #pragma unroll
           for (int j = 0; j < 4; ++j) p2[(size_t)(eb + j) * D + d] = a2[nt][4 * i4 + j];
           const float4 v = {a1[nt][4 * i4], a1[nt][4 * i4 + 1], a1[nt][4 * i4 + 2], a1[nt][4 * i4 + 3]};
-          *(float4*)(p1 + (size_t)d * E + eb) = v;
+          *(float4*)(p1 + (size_t)d * ldw + eb) = v;
         }
       }
     }
@@ -141,7 +162,7 @@ __host__ __device__ constexpr int dx2_rows() { return DX2_ROWS / DES; }
 template <bool BF16, int D, int ACT, int DES = 1, int NW = DX2_NW>
 __device__ __forceinline__ void dx2_body(const u16* __restrict__ X, const u16* __restrict__ W1,
                                          const u16* __restrict__ W2, const u16* __restrict__ dO,
-                                         void* __restrict__ dX, int B, int E, int tiles_per_head, int outf32,
+                                         void* __restrict__ dX, int B, int E, int ldw, int tiles_per_head, int outf32,
                                          int t, int cb, int ce, float* __restrict__ pws) {
   static_assert(DES == 1 || (DES == 2 && D == 64), "E split");
   static_assert(NW == DX2_NW || (NW == 4 && D == 256 && DES == 1), "waves per program");
@@ -174,7 +195,7 @@ __device__ __forceinline__ void dx2_body(const u16* __restrict__ X, const u16* _
 
   const u16* Xh = X + (size_t)h * B * D;
   const u16* dOh = dO + (size_t)h * B * D;
-  const u16* W1h = W1 + (size_t)h * D * E;
+  const u16* W1h = W1 + (size_t)h * D * ldw;
   const u16* W2h = W2 + (size_t)h * E * D;
   const int b_wave = bt * ROWS + wp * 32;
 
@@ -186,7 +207,7 @@ __device__ __forceinline__ void dx2_body(const u16* __restrict__ X, const u16* _
     const unsigned p = k * NTP + wp * 64 + lane;
     if (p < 4u * D) {  // W1c row r, logical chunk q
       const unsigned r = p >> 2, q = (p & 3u) ^ ((r >> 2) & 3u);
-      dmaOff[k] = r * (unsigned)E * 2u + q * 16u;
+      dmaOff[k] = r * (unsigned)ldw * 2u + q * 16u;
       dmaCol[k] = (int)(q * 8u);
     } else {           // W2c block bk, row rr, logical piece q
       const unsigned pp = p - 4u * D, bk = pp >> 7, rr = (pp >> 2) & 31u;
@@ -201,7 +222,7 @@ __device__ __forceinline__ void dx2_body(const u16* __restrict__ X, const u16* _
     const int c = c0 + ci;
     const bool mine = ci < NCP;
     const int lim = mine ? e_end - c * 32 : 0;
-    const int rem = mine ? D * E * 2 - 64 * c : 0;
+    const int rem = mine ? D * ldw * 2 - 64 * c : 0;
     const i32x4 r1 = make_rsrc_words(W1h + (size_t)c * 32, rem > 0 ? rem : 0);
     const i32x4 r2 = make_rsrc_words(W2h + (size_t)c * 32 * D, clamp0(lim, 32) * D * 2);
     const int slot = RB + (ci & (NSL - 1)) * (int)SLOT + wp * 1024;
@@ -426,8 +447,8 @@ template <bool BF16, int D, int ACT, bool HILO, bool DZ = false, int ET = DW_ET>
 __device__ __forceinline__ void dw2_body(const u16* __restrict__ X, const u16* __restrict__ W1,
                                          const u16* __restrict__ W2, const u16* __restrict__ dO,
                                          void* __restrict__ dW1, void* __restrict__ dW2, float* __restrict__ ws,
-                                         int H, int B, int E, int nE, int nS, int rows_per_split, int outf32,
-                                         int t, u16* __restrict__ dzt = nullptr, int Bp = 0) {
+                                         int H, int B, int E, int ldw, int nE, int nS, int rows_per_split,
+                                         int outf32, int t, u16* __restrict__ dzt = nullptr, int Bp = 0) {
   static_assert(ET == DW_ET || (ET == 64 && D == 64 && !DZ), "E-tile width");
   constexpr int KS = D / 16, NTN = D / 32;
   constexpr int CG = ET / 32;            // column groups of waves
@@ -461,7 +482,7 @@ __device__ __forceinline__ void dw2_body(const u16* __restrict__ X, const u16* _
 
   const u16* Xh = X + (size_t)h * B * D;
   const u16* dOh = dO + (size_t)h * B * D;
-  const u16* W1h = W1 + (size_t)h * D * E;
+  const u16* W1h = W1 + (size_t)h * D * ldw;
   const u16* W2h = W2 + (size_t)h * E * D;
 
   // ---- weight tiles (once): W2T rows natural, W1T transposed with 2-byte writes ----
@@ -477,7 +498,7 @@ __device__ __forceinline__ void dw2_body(const u16* __restrict__ X, const u16* _
     {  // W1 row d, columns e_prog + 8u .. + 7  ->  W1T rows 8u + j, column d
       const int d = p / (ET / 8), u = p % (ET / 8);
       u32x4 v = {0u, 0u, 0u, 0u};
-      if (e_prog + 8 * u < E) v = *(const u32x4*)(W1h + (size_t)d * E + e_prog + 8 * u);
+      if (e_prog + 8 * u < E) v = *(const u32x4*)(W1h + (size_t)d * ldw + e_prog + 8 * u);
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         const u16 x = (u16)(v[j >> 1] >> (16 * (j & 1)));
@@ -716,7 +737,7 @@ __device__ __forceinline__ void dw2_body(const u16* __restrict__ X, const u16* _
             }
           }
       }
-      dw_store<BF16, D>(a1, a2, dW1, dW2, ws, H, E, h, s, nS, e0, g, l32, outf32);
+      dw_store<BF16, D>(a1, a2, dW1, dW2, ws, H, E, ldw, h, s, nS, e0, g, l32, outf32);
     }
   }
 }
@@ -725,8 +746,8 @@ __device__ __forceinline__ void dw2_body(const u16* __restrict__ X, const u16* _
 template <bool BF16, int D, int ACT, int DES>
 __global__ void __launch_bounds__(DX2_NT) __attribute__((amdgpu_waves_per_eu(2, 2)))
 dx2_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* __restrict__ W2,
-           const u16* __restrict__ dO, void* __restrict__ dX, int B, int E, int tiles_per_head, int outf32) {
-  dx2_body<BF16, D, ACT, DES>(X, W1, W2, dO, dX, B, E, tiles_per_head, outf32, xcd_remap(blockIdx.x, gridDim.x), 0,
+           const u16* __restrict__ dO, void* __restrict__ dX, int B, int E, int ldw, int tiles_per_head, int outf32) {
+  dx2_body<BF16, D, ACT, DES>(X, W1, W2, dO, dX, B, E, ldw, tiles_per_head, outf32, xcd_remap(blockIdx.x, gridDim.x), 0,
                               (E + 31) >> 5, nullptr);
 }
 
@@ -736,8 +757,8 @@ dx2_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* __r
 template <bool BF16, int ACT>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 dx256_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* __restrict__ W2,
-             const u16* __restrict__ dO, void* __restrict__ dX, int B, int E, int tiles_per_head, int outf32) {
-  dx2_body<BF16, 256, ACT, 1, 4>(X, W1, W2, dO, dX, B, E, tiles_per_head, outf32, xcd_remap(blockIdx.x, gridDim.x),
+             const u16* __restrict__ dO, void* __restrict__ dX, int B, int E, int ldw, int tiles_per_head, int outf32) {
+  dx2_body<BF16, 256, ACT, 1, 4>(X, W1, W2, dO, dX, B, E, ldw, tiles_per_head, outf32, xcd_remap(blockIdx.x, gridDim.x),
                                  0, (E + 31) >> 5, nullptr);
 }
 
@@ -795,7 +816,7 @@ template <bool BF16, int ACT, bool HILO>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 dw256_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* __restrict__ W2,
              const u16* __restrict__ dO, void* __restrict__ dW1, void* __restrict__ dW2, float* __restrict__ ws,
-             int H, int B, int E, int nE, int nS, int rows_per_split, int outf32) {
+             int H, int B, int E, int ldw, int nE, int nS, int rows_per_split, int outf32) {
   constexpr int D = 256, KS = D / 16, NTN = D / 32;
   constexpr int STG = 2 * DW4_SLOT;  // W1c staging tile: [256 d][128 e], 256-byte rows
   constexpr int PD = DW4_PD;
@@ -812,7 +833,7 @@ dw256_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* _
 
   const u16* Xh = X + (size_t)h * B * D;
   const u16* dOh = dO + (size_t)h * B * D;
-  const u16* W1h = W1 + (size_t)h * D * E;
+  const u16* W1h = W1 + (size_t)h * D * ldw;
   const u16* W2h = W2 + (size_t)h * E * D;
 
   // ---- subtile loads: lane-linear 16-byte pieces (pieces k4 of the X tile, then of dO) ----
@@ -847,7 +868,7 @@ dw256_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* _
   for (int k = 0; k < 256 * 16 / 256; ++k) {
     const int p = tid + 256 * k, d = p >> 4, u = p & 15;
     u32x4 v = {0u, 0u, 0u, 0u};
-    if (e_prog + 8 * u < E) v = *(const u32x4*)(W1h + (size_t)d * E + e_prog + 8 * u);
+    if (e_prog + 8 * u < E) v = *(const u32x4*)(W1h + (size_t)d * ldw + e_prog + 8 * u);
     lds_write16(STG + d * 256 + u * 16, v);
   }
   // W2 row e0 + l32, d = 16 ks + 8 g .. + 7: the B operand of dH as it lies in memory
@@ -991,15 +1012,16 @@ dw256_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* _
     asm volatile("" ::: "memory");
   }
   wait_vmcnt<0>();  // the empty requests past the range
-  dw_store<BF16, D>(a1, a2, dW1, dW2, ws, H, E, h, s, nS, e0, g, l32, outf32);
+  dw_store<BF16, D>(a1, a2, dW1, dW2, ws, H, E, ldw, h, s, nS, e0, g, l32, outf32);
 }
 
 template <bool BF16, int D, int ACT, bool HILO, bool DZ, int ET = DW_ET>
 __global__ void __launch_bounds__(DW2_NT) __attribute__((amdgpu_waves_per_eu(2, 2)))
 dw2_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* __restrict__ W2,
            const u16* __restrict__ dO, void* __restrict__ dW1, void* __restrict__ dW2, float* __restrict__ ws,
-           int H, int B, int E, int nE, int nS, int rows_per_split, int outf32, u16* __restrict__ dzt, int Bp) {
-  dw2_body<BF16, D, ACT, HILO, DZ, ET>(X, W1, W2, dO, dW1, dW2, ws, H, B, E, nE, nS, rows_per_split, outf32,
+           int H, int B, int E, int ldw, int nE, int nS, int rows_per_split, int outf32, u16* __restrict__ dzt,
+           int Bp) {
+  dw2_body<BF16, D, ACT, HILO, DZ, ET>(X, W1, W2, dO, dW1, dW2, ws, H, B, E, ldw, nE, nS, rows_per_split, outf32,
                                    xcd_remap(blockIdx.x, gridDim.x), dzt, Bp);
 }
 
@@ -1013,7 +1035,7 @@ template <bool BF16, int D, int ACT, bool HILO, int DES, int ET = DW_ET>
 __global__ void __launch_bounds__(DW2_NT) __attribute__((amdgpu_waves_per_eu(2, 2)))
 bwd_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* __restrict__ W2,
            const u16* __restrict__ dO, void* __restrict__ dX, void* __restrict__ dW1, void* __restrict__ dW2,
-           float* __restrict__ ws, int H, int B, int E, int nE, int nS, int rows_per_split, int n_dw,
+           float* __restrict__ ws, int H, int B, int E, int ldw, int nE, int nS, int rows_per_split, int n_dw,
            int dx_tiles_per_head, int dx_first, int outf32, int n_dxs, int dxs_xs, int dxs_nct,
            float* __restrict__ dxs_ws) {
   // programs: n_dw dW programs and n_dx whole-tile dX programs (in the plan's order), then
@@ -1023,19 +1045,19 @@ bwd_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* __r
   const int T = dx_tiles_per_head, nch = (E + 31) >> 5;
   if (b >= n_rest) {
     const int u = b - n_rest, hh = u / dxs_xs, cb = (u - hh * dxs_xs) * dxs_nct;
-    dx2_body<BF16, D, ACT, DES>(X, W1, W2, dO, dX, B, E, T, outf32, hh * T + T - 1, cb, min(nch, cb + dxs_nct),
+    dx2_body<BF16, D, ACT, DES>(X, W1, W2, dO, dX, B, E, ldw, T, outf32, hh * T + T - 1, cb, min(nch, cb + dxs_nct),
                                 dxs_ws + (size_t)u * dx2_rows<D, DES>() * D);
     return;
   }
   const int bw = dx_first ? b - n_dx : b;  // index among the dW programs (< 0 or >= n_dw: a dX program)
   if (bw >= 0 && bw < n_dw) {
-    dw2_body<BF16, D, ACT, HILO, false, ET>(X, W1, W2, dO, dW1, dW2, ws, H, B, E, nE, nS, rows_per_split, outf32,
+    dw2_body<BF16, D, ACT, HILO, false, ET>(X, W1, W2, dO, dW1, dW2, ws, H, B, E, ldw, nE, nS, rows_per_split, outf32,
                                             xcd_remap(bw, n_dw));
   } else {
     const int bx = dx_first ? b : b - n_dw;
     const int m = xcd_remap(bx, n_dx);
     const int t = n_dxs > 0 ? (m / (T - 1)) * T + m % (T - 1) : m;
-    dx2_body<BF16, D, ACT, DES>(X, W1, W2, dO, dX, B, E, T, outf32, t, 0, nch, nullptr);
+    dx2_body<BF16, D, ACT, DES>(X, W1, W2, dO, dX, B, E, ldw, T, outf32, t, 0, nch, nullptr);
   }
 }
 
@@ -1066,6 +1088,47 @@ dw_reduce_kernel(const float* __restrict__ ws, void* __restrict__ dW1, void* __r
     } else {
       const u32x2 v = {pack2<BF16>(acc.x, acc.y), pack2<BF16>(acc.z, acc.w)};
       *(u32x2*)((u16*)dst + i) = v;
+    }
+  }
+}
+
+// The same sum where E is no multiple of 8: the partials' rows are padded to ldw (dW2 ldw rows of
+// D per head, dW1 rows of ldw), the outputs' are not. Four padded elements per thread; dW2's
+// groups of four columns lie in one row (D % 4 == 0), dW1's are stored one by one up to E.
+template <bool BF16>
+__global__ void __launch_bounds__(256)
+dw_reduce_pad_kernel(const float* __restrict__ ws, void* __restrict__ dW1, void* __restrict__ dW2, int H, int E, int D,
+                     int ldw, int nS, int outf32) {
+  const size_t per = (size_t)H * ldw * D;
+  const size_t n4 = per / 4;
+  const size_t stride = (size_t)gridDim.x * blockDim.x;
+  for (size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x; q < 2 * n4; q += stride) {
+    const bool second = q >= n4;
+    const size_t i = (second ? q - n4 : q) * 4;
+    const size_t row = i / (second ? ldw : D);  // dW2: h ldw + e, dW1: h D + d
+    const int col = (int)(i - row * (second ? ldw : D));
+    const size_t h = row / (second ? D : ldw);
+    const int r = (int)(row - h * (second ? D : ldw));
+    const int lim = second ? E - col : (r < E ? 4 : 0);  // elements of this group that exist
+    if (lim <= 0) continue;
+    const float* src = ws + (second ? (size_t)nS * per : 0) + i;
+    float4 acc = *(const float4*)src;
+    for (int s = 1; s < nS; ++s) {
+      const float4 v = *(const float4*)(src + (size_t)s * per);
+      acc.x += v.x;
+      acc.y += v.y;
+      acc.z += v.z;
+      acc.w += v.w;
+    }
+    const float a[4] = {acc.x, acc.y, acc.z, acc.w};
+    const size_t o = second ? row * E + col : (h * E + r) * D + col;
+    void* dst = second ? dW1 : dW2;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (j < lim) {
+        if (outf32) ((float*)dst)[o + j] = a[j];
+        else ((u16*)dst)[o + j] = from_f32<BF16>(a[j]);
+      }
     }
   }
 }
@@ -1103,7 +1166,7 @@ static_assert(DXG_WPF <= DXG_WS - 1 && DXG_WPF <= dxg_zpf(2), "rings");
 template <bool BF16, int D, int TP = 1>
 __global__ void __launch_bounds__(DX2_NT) __attribute__((amdgpu_waves_per_eu(2, 2)))
 dxg_kernel(const u16* __restrict__ dzt, const u16* __restrict__ W1, void* __restrict__ dX, int B, int Bp, int E,
-           int Ep, int tiles_per_head, int n_tiles, int outf32) {
+           int ldw, int Ep, int tiles_per_head, int n_tiles, int outf32) {
   static_assert(TP == 1 || TP == 2, "256-row blocks per tile");
   constexpr int NTN = D / 32;
   constexpr int ZT = 32 * 256 * 2;      // dZ chunk bytes of one 256-row block
@@ -1143,7 +1206,7 @@ dxg_kernel(const u16* __restrict__ dzt, const u16* __restrict__ W1, void* __rest
   // W1c piece p = 64 (wave % W1W) + lane: row r = p / 4, logical chunk q = (p % 4) ^ ((r / 4) % 4)
   const unsigned pw = (unsigned)(wave % W1W) * 64u + lane;
   const unsigned wr = pw >> 2, wq = (pw & 3u) ^ ((wr >> 2) & 3u);
-  const unsigned wOff = wr * (unsigned)E * 2u + wq * 16u;
+  const unsigned wOff = wr * (unsigned)ldw * 2u + wq * 16u;
   const int wCol = (int)(wq * 8u);
 
   // step j = (tile k, chunk c) of this workgroup; steps past the last load nothing (zero-size
@@ -1159,7 +1222,7 @@ dxg_kernel(const u16* __restrict__ dzt, const u16* __restrict__ W1, void* __rest
     const int h = t / tiles_per_head, bt = t - h * tiles_per_head;
     // the tile's blocks' chunks, 8192 elements each, block after block
     q.z = dzt + ((size_t)h * Bp + (size_t)bt * TP * DX2_ROWS) * Ep;
-    q.w = W1 + (size_t)h * D * E;
+    q.w = W1 + (size_t)h * D * ldw;
     q.nb = min(TP, nblk - bt * TP);  // blocks of the tile within the head (TP = 2: the last may hold one)
   };
   auto advance = [&](Cursor& q) {
@@ -1185,7 +1248,7 @@ dxg_kernel(const u16* __restrict__ dzt, const u16* __restrict__ W1, void* __rest
   };
   auto dma_w = [&](const Cursor& q) {
     const int lim = E - q.c * 32;
-    const int rem = D * E * 2 - 64 * q.c;
+    const int rem = D * ldw * 2 - 64 * q.c;
     const i32x4 rw = make_rsrc_words(q.w, q.k < my_tiles && rem > 0 ? rem : 0);
     buf_load16_lds(rw, wCol < lim ? wOff : BUF_OOB, WOFF + (q.j & (DXG_WS - 1)) * WT + (wave % W1W) * 1024);
   };
@@ -1397,7 +1460,7 @@ BwdPlan make_plan(int64_t H, int64_t B, int64_t D, int64_t E, int act, bool hilo
   static const int et_env = env_int("FMLP_BWD_ET", 0);
   auto nE_for = [&](long long et) { return (E + et - 1) / et; };
   const long long base = H * nE_for(DW_ET);  // the stored-dZ form's dW programs (128 columns)
-  auto ws_for = [&](long long ns) { return ns > 1 ? (size_t)2 * ns * H * E * D * sizeof(float) : (size_t)0; };
+  auto ws_for = [&](long long ns) { return ns > 1 ? (size_t)2 * ns * H * w1_pitch(E) * D * sizeof(float) : (size_t)0; };
   // dX programs of 256 rows, or at D = 64 of 128 rows with E in two parts (half the time each)
   auto n_dx_for = [&](int des) { return H * ((B + DX2_ROWS / des - 1) / (DX2_ROWS / des)); };
   auto tx_for = [&](int des) {
@@ -1610,7 +1673,7 @@ Dw256Plan plan_dw256(int64_t H, int64_t B, int64_t E, bool hilo, int num_cus, si
   double best = 1e300;
   for (long long ns = 1; ns <= max_ns; ns *= 2) {
     const long long rps = rows_for_split(B, ns), eff = (B + rps - 1) / rps;
-    const size_t ws = eff > 1 ? (size_t)2 * eff * H * E * 256 * sizeof(float) : 0;
+    const size_t ws = eff > 1 ? (size_t)2 * eff * H * w1_pitch(E) * 256 * sizeof(float) : 0;
     if (ws > max_ws) continue;
     const long long progs = H * p.nE * eff, rounds = (progs + N - 1) / N;
     double cost = (double)rounds * (kFixedUs + (double)(rps / DW_BT) * t_sub);
@@ -1638,9 +1701,14 @@ constexpr size_t dw_lds_bytes() {
 template <bool BF16>
 static hipError_t launch_dw_reduce(const BwdArgs& a, int nS, hipStream_t st) {
   if (nS <= 1) return hipSuccess;
-  const size_t items = 2 * ((size_t)a.H * a.E * a.D / 4);
+  const size_t items = 2 * ((size_t)a.H * a.ldw * a.D / 4);
   size_t blocks = (items + 255) / 256;
   if (blocks > 8192) blocks = 8192;
+  if (a.ldw != a.E) {
+    hipLaunchKernelGGL(dw_reduce_pad_kernel<BF16>, dim3((unsigned)blocks), dim3(256), 0, st, (const float*)a.ws, a.dw1,
+                       a.dw2, (int)a.H, (int)a.E, (int)a.D, (int)a.ldw, nS, a.out_f32 ? 1 : 0);
+    return hipGetLastError();
+  }
   hipLaunchKernelGGL(dw_reduce_kernel<BF16>, dim3((unsigned)blocks), dim3(256), 0, st, (const float*)a.ws, a.dw1, a.dw2,
                      (int)a.H, (int)a.E, (int)a.D, nS, a.out_f32 ? 1 : 0);
   return hipGetLastError();
@@ -1665,7 +1733,7 @@ static hipError_t launch_bwd_t(const BwdArgs& a, const BwdPlan& p, hipStream_t s
       if (r != hipSuccess) return r;
       hipLaunchKernelGGL(k, dim3((unsigned)p.n_dw), dim3(DW2_NT), lds, st, (const u16*)a.x, (const u16*)a.w1,
                          (const u16*)a.w2, (const u16*)a.dout, a.dw1, a.dw2, (float*)a.ws, (int)a.H, (int)a.B,
-                         (int)a.E, p.nE, p.nS, p.rows_per_split, a.out_f32 ? 1 : 0, dzt, p.Bp);
+                         (int)a.E, (int)a.ldw, p.nE, p.nS, p.rows_per_split, a.out_f32 ? 1 : 0, dzt, p.Bp);
       return hipGetLastError();
     };
     e = a.dw_hilo ? launch_w(dw2_kernel<BF16, D, ACT, true, true>) : launch_w(dw2_kernel<BF16, D, ACT, false, true>);
@@ -1682,7 +1750,7 @@ static hipError_t launch_bwd_t(const BwdArgs& a, const BwdPlan& p, hipStream_t s
       const long long n_t = a.H * (long long)tph;
       const long long grid = TP == 1 ? p.n_xg : std::min<long long>(n_t, p.n_xg);
       hipLaunchKernelGGL(kg, dim3((unsigned)grid), dim3(DX2_NT), lds_g, st, (const u16*)dzt, (const u16*)a.w1, a.dx,
-                         (int)a.B, p.Bp, (int)a.E, Ep, tph, (int)n_t, a.out_f32 ? 1 : 0);
+                         (int)a.B, p.Bp, (int)a.E, (int)a.ldw, Ep, tph, (int)n_t, a.out_f32 ? 1 : 0);
       return hipGetLastError();
     };
     return tp_env == 1 ? launch_g(dxg_kernel<BF16, D, 1>, 1) : launch_g(dxg_kernel<BF16, D, 2>, 2);
@@ -1703,7 +1771,7 @@ static hipError_t launch_bwd_t(const BwdArgs& a, const BwdPlan& p, hipStream_t s
       if (r != hipSuccess) return r;
       hipLaunchKernelGGL(k, dim3((unsigned)(n_dw + p.n_dx + p.n_dxs)), dim3(DW2_NT), lds, st, (const u16*)a.x,
                          (const u16*)a.w1, (const u16*)a.w2, (const u16*)a.dout, a.dx, a.dw1, a.dw2, (float*)a.ws,
-                         (int)a.H, (int)a.B, (int)a.E, p.nE, p.nS, p.rows_per_split, (int)n_dw,
+                         (int)a.H, (int)a.B, (int)a.E, (int)a.ldw, p.nE, p.nS, p.rows_per_split, (int)n_dw,
                          p.dx_tiles_per_head, p.dx_first ? 1 : 0, a.out_f32 ? 1 : 0, (int)p.n_dxs, p.dxs_xs,
                          p.dxs_nct, dxs_ws);
       return hipGetLastError();
@@ -1723,7 +1791,7 @@ static hipError_t launch_bwd_t(const BwdArgs& a, const BwdPlan& p, hipStream_t s
       if (r != hipSuccess) return r;
       hipLaunchKernelGGL(k, dim3((unsigned)p.n_dw), dim3(DW2_NT), lds, st, (const u16*)a.x, (const u16*)a.w1,
                          (const u16*)a.w2, (const u16*)a.dout, a.dw1, a.dw2, (float*)a.ws, (int)a.H,
-                         (int)a.B, (int)a.E, p.nE, p.nS, p.rows_per_split, a.out_f32 ? 1 : 0, (u16*)nullptr, 0);
+                         (int)a.B, (int)a.E, (int)a.ldw, p.nE, p.nS, p.rows_per_split, a.out_f32 ? 1 : 0, (u16*)nullptr, 0);
       return hipGetLastError();
     };
     e = a.dw_hilo ? launch_w(dw2_kernel<BF16, D, ACT, true, false, ET>)
@@ -1739,7 +1807,7 @@ static hipError_t launch_bwd_t(const BwdArgs& a, const BwdPlan& p, hipStream_t s
     e = set_lds_once((const void*)k, (int)lds_x, lds_set);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(k, dim3((unsigned)n_dx_all), dim3(DX2_NT), lds_x, st, (const u16*)a.x, (const u16*)a.w1,
-                       (const u16*)a.w2, (const u16*)a.dout, a.dx, (int)a.B, (int)a.E, p.dx_tiles_per_head,
+                       (const u16*)a.w2, (const u16*)a.dout, a.dx, (int)a.B, (int)a.E, (int)a.ldw, p.dx_tiles_per_head,
                        a.out_f32 ? 1 : 0);
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
@@ -1776,7 +1844,7 @@ static hipError_t launch_dx256_t(const BwdArgs& a, hipStream_t st) {
   hipError_t e = set_lds_once((const void*)k, (int)lds, lds_set);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(256), lds, st, (const u16*)a.x, (const u16*)a.w1, (const u16*)a.w2,
-                     (const u16*)a.dout, a.dx, (int)a.B, (int)a.E, (int)tph, a.out_f32 ? 1 : 0);
+                     (const u16*)a.dout, a.dx, (int)a.B, (int)a.E, (int)a.ldw, (int)tph, a.out_f32 ? 1 : 0);
   return hipGetLastError();
 }
 
@@ -1804,7 +1872,7 @@ static hipError_t launch_dw256_t(const BwdArgs& a, const Dw256Plan& p, hipStream
   hipError_t e = set_lds_once((const void*)k, (int)lds, lds_set);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(k, dim3((unsigned)p.n), dim3(256), lds, st, (const u16*)a.x, (const u16*)a.w1, (const u16*)a.w2,
-                     (const u16*)a.dout, a.dw1, a.dw2, (float*)a.ws, (int)a.H, (int)a.B, (int)a.E, p.nE, p.nS,
+                     (const u16*)a.dout, a.dw1, a.dw2, (float*)a.ws, (int)a.H, (int)a.B, (int)a.E, (int)a.ldw, p.nE, p.nS,
                      p.rows_per_split, a.out_f32 ? 1 : 0);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   return launch_dw_reduce<BF16>(a, p.nS, st);

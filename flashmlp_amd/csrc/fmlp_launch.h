@@ -16,6 +16,15 @@ int env_int(const char* name, int dflt);
 // skip the runtime call.
 hipError_t set_lds_once(const void* kernel, int bytes, std::atomic<unsigned long long>& done);
 
+// Row pitch the tuned kernels read W1 with: E rounded up to whole 16-byte vectors of 16-bit
+// elements. Where E is no multiple of 8 the caller's W1 rows are copied to this pitch first
+// (launch_pad_w1), into w1_pad_bytes of workspace (a multiple of 256 bytes).
+inline int64_t w1_pitch(int64_t E) { return (E + 7) / 8 * 8; }
+inline size_t w1_pad_bytes(int64_t H, int64_t D, int64_t E) {
+  return E % 8 == 0 ? 0 : ((size_t)H * D * w1_pitch(E) * 2 + 255) / 256 * 256;
+}
+hipError_t launch_pad_w1(const void* w1, void* dst, int64_t H, int64_t D, int64_t E, hipStream_t st);
+
 struct FwdArgs {
   const void* x;
   const void* w1;
@@ -26,6 +35,7 @@ struct FwdArgs {
   int act;
   bool out_f32;  // outputs as fp32 (FMLP_OUT_F32)
   int num_cus;   // compute units of the current device
+  int64_t ldw;   // row pitch of w1 (w1_pitch(E))
   void* ws = nullptr;   // workspace for split tiles' partials (fwd_plan), or none
   size_t ws_bytes = 0;
 };
@@ -88,6 +98,7 @@ struct BwdArgs {
   bool dw_hilo;  // dW products with hi/lo terms of h and dZ (FMLP_DW_HILO)
   bool want_dx = true;  // false: FMLP_BWD_NO_DX (only the dW programs run)
   bool want_dw = true;  // false: FMLP_BWD_NO_DW (only the dX programs run)
+  int64_t ldw = 0;      // row pitch of w1, and of the fp32 dW partials (w1_pitch(E))
 };
 
 // io element types of the generic kernels
@@ -150,9 +161,9 @@ hipError_t launch_fwd(const FwdArgs& a, hipStream_t st);
 hipError_t launch_tile_reduce(const float* ws, void* out, bool bf16, int B, int D, int BB, int H, int T, int xs,
                               int n_split, int outf32, hipStream_t st);
 hipError_t launch_bwd(const BwdArgs& a, const BwdPlan& p, hipStream_t st);
-// dX alone at D = 256 (dense 16-bit, E % 8 == 0): the tuned dX programs
+// dX alone at D = 256 (dense 16-bit): the tuned dX programs
 hipError_t launch_dx256(const BwdArgs& a, hipStream_t st);
-// dW alone at D = 256 (dense 16-bit, E % 8 == 0): n = H nE nS programs (nE E-tiles of 128
+// dW alone at D = 256 (dense 16-bit): n = H nE nS programs (nE E-tiles of 128
 // columns, nS B ranges of rows_per_split rows), whose fp32 partials take ws_bytes of workspace
 // when nS > 1 (a split needing more than max_ws bytes is not taken)
 struct Dw256Plan {

@@ -1,7 +1,7 @@
 // _fmlp_fast: the per-call fast path of flashmlp_fwd / flashmlp_bwd (flashmlp_amd/flashmlp.py).
 //
 // A CPython module (METH_FASTCALL) over the C ABI of libflashmlp.so for the common case: 16-bit
-// inputs on one GPU, dense and 16-byte aligned, a shape the tuned kernels take. It allocates the
+// inputs on one GPU, dense and 16-byte aligned, a shape with kernels of its own. It allocates the
 // outputs and the workspace with ATen on the inputs' device, launches on torch's current HIP
 // stream of that device and returns the C ABI status with the outputs; for any other input it
 // returns None and the Python wrapper takes its general path (which also raises the reference's
@@ -34,7 +34,7 @@ bool dense16(const at::Tensor& t) {
   return t.dim() == 3 && t.is_contiguous() && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15u) == 0;
 }
 
-// the tensors the tuned kernels take as they are: 16-bit, one GPU, dense, aligned; sets the io
+// the tensors those kernels take as they are: 16-bit, one GPU, dense, aligned; sets the io
 // dtype code
 bool eligible(PyObject* const* args, int n, const at::Tensor** ts, int* code) {
   for (int i = 0; i < n; ++i) {
@@ -76,7 +76,7 @@ PyObject* fast_fwd(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const int act = (int)PyLong_AsLong(args[3]);
   if (act == -1 && PyErr_Occurred()) return nullptr;
   const int64_t H = x.size(0), B = x.size(1), D = x.size(2), E = w1.size(2);
-  if (!fmlp_shape_tuned(D, E, code)) Py_RETURN_NONE;
+  if (!fmlp_shape_dense(D, E, code)) Py_RETURN_NONE;
   c10::DeviceGuard guard(x.device());
   const hipStream_t stream = c10::hip::getCurrentHIPStream(x.device().index()).stream();
   at::Tensor o = at::empty_like(x);
@@ -112,7 +112,7 @@ PyObject* fast_bwd(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   int flags = (int)PyLong_AsLong(args[5]);
   if (flags == -1 && PyErr_Occurred()) return nullptr;
   const int64_t H = x.size(0), B = x.size(1), D = x.size(2), E = w1.size(2);
-  if (!fmlp_shape_tuned(D, E, code)) Py_RETURN_NONE;
+  if (!fmlp_shape_dense(D, E, code)) Py_RETURN_NONE;
   flags |= code;
   const bool need_dx = (flags & FMLP_BWD_NO_DX) == 0, need_dw = (flags & FMLP_BWD_NO_DW) == 0;
   c10::DeviceGuard guard(x.device());
@@ -136,10 +136,16 @@ PyObject* fast_bwd(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     } catch (const c10::OutOfMemoryError&) {
       // the stored-dZ form's workspace does not fit: the recompute form needs at most the fp32
       // dW partials (as the general path does)
-      if (flags & FMLP_BWD_RECOMPUTE) throw;
+      const bool any_ws = !fmlp_shape_tuned(D, E, code);  // such calls accept any workspace
+      if ((flags & FMLP_BWD_RECOMPUTE) && !any_ws) throw;
       flags |= FMLP_BWD_RECOMPUTE;
       n = ws_need(flags);
-      if (n) ws = bytes_on(x, n);
+      try {
+        if (n) ws = bytes_on(x, n);
+      } catch (const c10::OutOfMemoryError&) {
+        if (!any_ws) throw;
+        n = 0;
+      }
     }
   }
   const int st = fmlp_bwd(x.data_ptr(), w1.data_ptr(), w2.data_ptr(), dout.data_ptr(),

@@ -26,8 +26,8 @@ Differences from the reference, all deliberate:
   * Leaky ReLU's derivative at Z == 0 is autograd's 0.01 (flashmlp.py:33-34 uses 1.0);
   * io dtypes are fp16, bf16 and fp32 (fp32 in true fp32, where the reference's tl.dot would
     use its default reduced input precision); other dtypes raise TypeError;
-  * strided inputs are accepted: shapes with kernels of their own (16-bit io, D in {64, 128,
-    256}, E % 8 == 0) copy them to dense tensors, as the reference's reshape / contiguous does
+  * strided inputs are accepted: shapes with kernels of their own (fmlp_shape_dense: 16-bit io, D in
+    {64, 128, 256}) copy them to dense tensors, as the reference's reshape / contiguous does
     (flashmlp.py:453-459,508); every other shape reads the views in place (generic kernels),
     where the reference would copy them or fail its contiguity assertions.
 """
@@ -102,12 +102,9 @@ def _alloc_ws(nbytes: int, device: torch.device):
 
 @functools.lru_cache(maxsize=1024)
 def _own_kernels(D: int, E: int, dtype: int) -> bool:
-    # shapes with kernels of their own, which take dense 16-byte aligned tensors: the tuned
-    # kernels (fmlp_shape_tuned) and the D = 256 programs (16-bit io, E % 8 == 0); views of
-    # other shapes go to the generic kernels in place
-    if _lib.lib().fmlp_shape_tuned(D, E, dtype):
-        return True
-    return D == 256 and E % 8 == 0 and dtype in (_lib.FMLP_DTYPE_F16, _lib.FMLP_DTYPE_BF16)
+    # shapes with kernels of their own, which take dense 16-byte aligned tensors; views of other
+    # shapes go to the generic kernels in place
+    return bool(_lib.lib().fmlp_shape_dense(D, E, dtype))
 
 
 # torch's current HIP stream of a device, as the raw handle the C ABI takes, and the current
@@ -167,7 +164,7 @@ def flashmlp_fwd(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, activation
     assert E == E2, "Intermediate dimension mismatch"
     assert D == D2, "Output dimension mismatch"
 
-    if _fast is not None:  # 16-bit, one GPU, dense and aligned, a tuned shape: else None
+    if _fast is not None:  # one GPU, dense and aligned, a shape with kernels of its own: else None
         r = _fast.fwd(x, w1, w2, _act_code(activation))
         if r is not None:
             if r[0]:
@@ -257,13 +254,18 @@ def flashmlp_bwd(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, do: torch.
             try:
                 ws = _alloc_ws(ws_bytes, x.device)
             except torch.OutOfMemoryError:
-                if flags & _lib.FMLP_BWD_RECOMPUTE:
+                if flags & _lib.FMLP_BWD_RECOMPUTE and _lib.lib().fmlp_shape_tuned(D, E, dtype):
                     raise
                 # the stored-dZ form's workspace does not fit: the recompute form needs at most
                 # the fp32 dW partials (the reference's backward allocates no workspace at all)
                 flags |= _lib.FMLP_BWD_RECOMPUTE
                 ws_bytes = _ws_bytes(dev, H, B, D, E, flags)
-                ws = _alloc_ws(ws_bytes, x.device)
+                try:
+                    ws = _alloc_ws(ws_bytes, x.device)
+                except torch.OutOfMemoryError:
+                    if _lib.lib().fmlp_shape_tuned(D, E, dtype):
+                        raise
+                    ws, ws_bytes = None, 0  # any workspace is accepted
             st = L.fmlp_bwd(x.data_ptr(), w1.data_ptr(), w2.data_ptr(), do.data_ptr(), _ptr(dx),
                             _ptr(dw1), _ptr(dw2), H, B, D, E, flags, _act_code(activation),
                             ws.data_ptr() if ws is not None else None, ws_bytes, stream)
