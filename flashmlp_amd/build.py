@@ -24,7 +24,9 @@ ROOT = PKG.parent
 CSRC = PKG / "csrc"
 BUILD = PKG / "_build"
 LIB = PKG / "libflashmlp.so"
-SOURCES = ["fmlp_fwd.hip", "fmlp_bwd.hip", "fmlp_gen.hip", "fmlp_scratch.hip", "fmlp_abi.cpp"]
+# fmlp_bwd.hip is compiled once per part (file:part): the kernels of one D each, and the rest
+SOURCES = ["fmlp_bwd.hip:64", "fmlp_bwd.hip:128", "fmlp_bwd.hip:0", "fmlp_bwd.hip:32", "fmlp_fwd.hip", "fmlp_gen.hip",
+           "fmlp_scratch.hip", "fmlp_abi.cpp"]
 CEILING_SRC = "fmlp_ceiling.hip"
 CEILING_LIB = PKG / "libfmlp_ceiling.so"
 FAST_SRC = "fmlp_py.cpp"
@@ -45,8 +47,10 @@ def _hipcc() -> str:
 
 
 def _compile(src: str, verbose: bool) -> Path:
-    obj = BUILD / (src.rsplit(".", 1)[0] + ".o")
-    cmd = [_hipcc(), *COMMON, *DEVICE_FLAGS, "-x", "hip", "-c", str(CSRC / src), "-o", str(obj)]
+    src, _, part = src.partition(":")
+    obj = BUILD / (src.rsplit(".", 1)[0] + (f"_{part}" if part else "") + ".o")
+    defs = [f"-DFMLP_BWD_PART={part}"] if part else []
+    cmd = [_hipcc(), *COMMON, *DEVICE_FLAGS, *defs, "-x", "hip", "-c", str(CSRC / src), "-o", str(obj)]
     if verbose:
         print(" ".join(cmd), flush=True)
     res = subprocess.run(cmd, capture_output=True, text=True)

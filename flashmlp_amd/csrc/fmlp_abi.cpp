@@ -111,12 +111,12 @@ bool fwd_tuned_shape(int64_t D, int64_t E, int io) {
   return tuned_shape(D, E, io) || ((io == FMLP_DTYPE_F16 || io == FMLP_DTYPE_BF16) && D == 256 && E % 8 == 0);
 }
 
-// Dense, 16-byte aligned tensors of these shapes run on kernels of their own: those above, and the
-// same D with E % 8 != 0, whose W1 rows are first copied to 16-byte aligned rows at the start of
+// Dense, 16-byte aligned tensors of these shapes run on kernels of their own: those above, D = 16
+// and 32 (the same programs on 32-column tiles), and the same D with E % 8 != 0, whose W1 rows are first copied to 16-byte aligned rows at the start of
 // the workspace (w1_pad_bytes; a call without room for them runs on the generic kernels, which were
 // 2.4 to 14 times slower at every E % 8 != 0 measured, from a 16-row forward to a 16-head training step).
 bool dense_shape(int64_t D, int io) {
-  return (io == FMLP_DTYPE_F16 || io == FMLP_DTYPE_BF16) && (D == 64 || D == 128 || D == 256);
+  return (io == FMLP_DTYPE_F16 || io == FMLP_DTYPE_BF16) && (D == 16 || D == 32 || D == 64 || D == 128 || D == 256);
 }
 
 int check_shape(int64_t H, int64_t B, int64_t D, int64_t E, int dtype) {
@@ -456,8 +456,9 @@ int bwd_impl(const void* x, const void* w1, const void* w2, const void* dout, vo
     const bool hilo = (dtype & FMLP_DW_HILO) != 0;
     fmlp::BwdPlan plan = fmlp::plan_bwd(H, B, D, E, act, hilo, dz_mode_of(dtype), cus,
                                         noalloc ? fmlp::kScratchBytes - pad : (size_t)-1);
-    // E % 8 != 0 takes any workspace, as the generic kernels do: a plan that fits it
-    if (pad > 0 && plan_ws_bytes(plan, dtype) > given - pad)
+    // D < 64 and E % 8 != 0 take any workspace, as the generic kernels do: a plan that fits it
+    const bool any_ws = !tuned_shape(D, E, io);
+    if (any_ws && plan_ws_bytes(plan, dtype) > given - pad)
       plan = fmlp::plan_bwd(H, B, D, E, act, hilo, dz_mode_of(dtype), cus, given - pad);
     // the dW programs alone (FMLP_BWD_NO_DX) need only their fp32 partials, the dX programs
     // alone (FMLP_BWD_NO_DW) only the split ragged tiles' partials, at the workspace's start
@@ -471,7 +472,7 @@ int bwd_impl(const void* x, const void* w1, const void* w2, const void* dout, vo
         e = fmlp::scratch_current_device(&ws);
         if (e != hipSuccess) return fail(FMLP_ERR_HIP, "scratch lookup: %s", hipGetErrorString(e));
       } else {
-        if (workspace == nullptr || workspace_bytes < ws_need)
+        if (!any_ws && (workspace == nullptr || workspace_bytes < ws_need))
           return fail(FMLP_ERR_WORKSPACE, "workspace of %zu bytes given, %zu needed", workspace_bytes, ws_need);
         if (!aligned16(workspace)) return fail(FMLP_ERR_INVALID_ARG, "workspace is not 16-byte aligned");
       }

@@ -28,14 +28,16 @@ constexpr int DW_BT = 32;            // rows per streamed subtile
 // (32 nt + l32), rows e = e0 + 8 (i / 4) + 4 g + (i % 4). nS == 1 writes dW1, dW2 in the io
 // dtype (fp32 when outf32); otherwise fp32 partials in the outputs' layouts, ws2[s][h][e][d]
 // and ws1[s][h][d][e], which dw_reduce_kernel sums elementwise.
-template <bool BF16, int D>
+// DG < D = 32: the tensors have DG columns d.
+template <bool BF16, int D, int DG = D>
 __device__ __forceinline__ void dw_store(const f32x16 (&a1)[D / 32], const f32x16 (&a2)[D / 32], void* __restrict__ dW1,
                                          void* __restrict__ dW2, float* __restrict__ ws, int H, int E, int ldw, int h,
                                          int s, int nS, int e0, int g, int l32, int outf32) {
   constexpr int NTN = D / 32;
+  if (DG < D && l32 >= DG) return;
   if (nS == 1 && outf32) {
-    float* dW2h = (float*)dW2 + (size_t)h * E * D;
-    float* dW1h = (float*)dW1 + (size_t)h * D * E;
+    float* dW2h = (float*)dW2 + (size_t)h * E * DG;
+    float* dW1h = (float*)dW1 + (size_t)h * DG * E;
 #pragma unroll
     for (int i4 = 0; i4 < 4; ++i4) {
       const int eb = e0 + 8 * i4 + 4 * g;
@@ -46,7 +48,7 @@ __device__ __forceinline__ void dw_store(const f32x16 (&a1)[D / 32], const f32x1
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
             if (eb + j < E) {
-              dW2h[(size_t)(eb + j) * D + d] = a2[nt][4 * i4 + j];
+              dW2h[(size_t)(eb + j) * DG + d] = a2[nt][4 * i4 + j];
               dW1h[(size_t)d * E + eb + j] = a1[nt][4 * i4 + j];
             }
           }
@@ -55,8 +57,8 @@ __device__ __forceinline__ void dw_store(const f32x16 (&a1)[D / 32], const f32x1
     }
   } else if (nS == 1 && (E & 3) != 0) {
     // rows of dW1 that are not 8-byte aligned, and column groups that E cuts
-    u16* dW2h = (u16*)dW2 + (size_t)h * E * D;
-    u16* dW1h = (u16*)dW1 + (size_t)h * D * E;
+    u16* dW2h = (u16*)dW2 + (size_t)h * E * DG;
+    u16* dW1h = (u16*)dW1 + (size_t)h * DG * E;
 #pragma unroll
     for (int i4 = 0; i4 < 4; ++i4) {
       const int eb = e0 + 8 * i4 + 4 * g;
@@ -66,15 +68,15 @@ __device__ __forceinline__ void dw_store(const f32x16 (&a1)[D / 32], const f32x1
 #pragma unroll
           for (int nt = 0; nt < NTN; ++nt) {
             const int d = nt * 32 + l32;
-            dW2h[(size_t)(eb + j) * D + d] = from_f32<BF16>(a2[nt][4 * i4 + j]);
+            dW2h[(size_t)(eb + j) * DG + d] = from_f32<BF16>(a2[nt][4 * i4 + j]);
             dW1h[(size_t)d * E + eb + j] = from_f32<BF16>(a1[nt][4 * i4 + j]);
           }
         }
       }
     }
   } else if (nS == 1) {
-    u16* dW2h = (u16*)dW2 + (size_t)h * E * D;
-    u16* dW1h = (u16*)dW1 + (size_t)h * D * E;
+    u16* dW2h = (u16*)dW2 + (size_t)h * E * DG;
+    u16* dW1h = (u16*)dW1 + (size_t)h * DG * E;
 #pragma unroll
     for (int i4 = 0; i4 < 4; ++i4) {
       const int eb = e0 + 8 * i4 + 4 * g;  // 4 consecutive columns eb .. eb+3 (E % 4 == 0)
@@ -83,7 +85,7 @@ __device__ __forceinline__ void dw_store(const f32x16 (&a1)[D / 32], const f32x1
         for (int nt = 0; nt < NTN; ++nt) {
           const int d = nt * 32 + l32;
 #pragma unroll
-          for (int j = 0; j < 4; ++j) dW2h[(size_t)(eb + j) * D + d] = from_f32<BF16>(a2[nt][4 * i4 + j]);
+          for (int j = 0; j < 4; ++j) dW2h[(size_t)(eb + j) * DG + d] = from_f32<BF16>(a2[nt][4 * i4 + j]);
           u32x2 v = {pack2<BF16>(a1[nt][4 * i4 + 0], a1[nt][4 * i4 + 1]), pack2<BF16>(a1[nt][4 * i4 + 2], a1[nt][4 * i4 + 3])};
           *(u32x2*)(dW1h + (size_t)d * E + eb) = v;
         }
@@ -92,9 +94,9 @@ __device__ __forceinline__ void dw_store(const f32x16 (&a1)[D / 32], const f32x1
   } else {
     // fp32 partials in the outputs' own layouts (dW2 [h][e][d], dW1 [h][d][e]) with E rounded up
     // to ldw, so the reduction is an elementwise sum over the nS slices
-    const size_t per = (size_t)H * ldw * D;
-    float* p2 = ws + ((size_t)s * H + h) * ldw * D;
-    float* p1 = ws + (size_t)nS * per + ((size_t)s * H + h) * D * ldw;
+    const size_t per = (size_t)H * ldw * DG;
+    float* p2 = ws + ((size_t)s * H + h) * ldw * DG;
+    float* p1 = ws + (size_t)nS * per + ((size_t)s * H + h) * DG * ldw;
 #pragma unroll
     for (int i4 = 0; i4 < 4; ++i4) {
       const int eb = e0 + 8 * i4 + 4 * g;  // 4 consecutive columns eb .. eb+3 (ldw % 8 == 0)
@@ -103,7 +105,7 @@ __device__ __forceinline__ void dw_store(const f32x16 (&a1)[D / 32], const f32x1
         for (int nt = 0; nt < NTN; ++nt) {
           const int d = nt * 32 + l32;
 #pragma unroll
-          for (int j = 0; j < 4; ++j) p2[(size_t)(eb + j) * D + d] = a2[nt][4 * i4 + j];
+          for (int j = 0; j < 4; ++j) p2[(size_t)(eb + j) * DG + d] = a2[nt][4 * i4 + j];
           const float4 v = {a1[nt][4 * i4], a1[nt][4 * i4 + 1], a1[nt][4 * i4 + 2], a1[nt][4 * i4 + 3]};
           *(float4*)(p1 + (size_t)d * ldw + eb) = v;
         }
@@ -139,6 +141,11 @@ __device__ __forceinline__ constexpr unsigned sig(unsigned m) {
   return (m & ~12u) | ((m & 4u) << 1) | ((m & 8u) >> 1);
 }
 
+// waves per SIMD the two-role kernels are built for: two; at D = 32 four (two workgroups per CU):
+// there a 32 x 32 tile carries 16 activation elements for 4-8 MFMAs and both roles are bound by the
+// VALU, whose latencies more waves hide. H=32 B=4096 D=32 E=512 bf16 SiLU backward: 59 us.
+__host__ __device__ constexpr int bwd_wpe(int D) { return D <= 32 ? 4 : 2; }
+
 constexpr int DX2_NW = 8;
 constexpr int DX2_NT = DX2_NW * 64;
 constexpr int DX2_ROWS = DX2_NW * 32;
@@ -159,14 +166,15 @@ __host__ __device__ constexpr int dx2_rows() { return DX2_ROWS / DES; }
 
 // A program owns tile t's rows and the E-chunks [cb, ce); with pws set (a ragged tile split
 // over E) it stores its fp32 partial dX tile there ([rows][D]) instead of writing dX.
-template <bool BF16, int D, int ACT, int DES = 1, int NW = DX2_NW>
+template <bool BF16, int D, int ACT, int DES = 1, int NW = DX2_NW, int DG = D>
 __device__ __forceinline__ void dx2_body(const u16* __restrict__ X, const u16* __restrict__ W1,
                                          const u16* __restrict__ W2, const u16* __restrict__ dO,
                                          void* __restrict__ dX, int B, int E, int ldw, int tiles_per_head, int outf32,
                                          int t, int cb, int ce, float* __restrict__ pws) {
-  static_assert(DES == 1 || (DES == 2 && D == 64), "E split");
+  static_assert(DES == 1 || (DES == 2 && D <= 64), "E split");
+  static_assert(DG == D || (DG == 16 && D == 32), "columns in memory");
   static_assert(NW == DX2_NW || (NW == 4 && D == 256 && DES == 1), "waves per program");
-  constexpr int KS = D / 16, NTN = D / 32;
+  constexpr int KS = DG / 16, NTN = D / 32;
   constexpr unsigned SLOT = 128u * D;
   constexpr unsigned W2OFF = 64u * D;
   constexpr int NTP = NW * 64 / DES;     // threads of one E part
@@ -193,10 +201,10 @@ __device__ __forceinline__ void dx2_body(const u16* __restrict__ X, const u16* _
   // (NW = 4) every wave runs the MFMA-first order
   const bool late = NW == 8 && wave >= 4;
 
-  const u16* Xh = X + (size_t)h * B * D;
-  const u16* dOh = dO + (size_t)h * B * D;
-  const u16* W1h = W1 + (size_t)h * D * ldw;
-  const u16* W2h = W2 + (size_t)h * E * D;
+  const u16* Xh = X + (size_t)h * B * DG;
+  const u16* dOh = dO + (size_t)h * B * DG;
+  const u16* W1h = W1 + (size_t)h * DG * ldw;
+  const u16* W2h = W2 + (size_t)h * E * DG;
   const int b_wave = bt * ROWS + wp * 32;
 
   // ---- staging pieces: piece p (16 bytes at slot offset 16 p) of a chunk ----
@@ -207,12 +215,12 @@ __device__ __forceinline__ void dx2_body(const u16* __restrict__ X, const u16* _
     const unsigned p = k * NTP + wp * 64 + lane;
     if (p < 4u * D) {  // W1c row r, logical chunk q
       const unsigned r = p >> 2, q = (p & 3u) ^ ((r >> 2) & 3u);
-      dmaOff[k] = r * (unsigned)ldw * 2u + q * 16u;
+      dmaOff[k] = DG == D || r < (unsigned)DG ? r * (unsigned)ldw * 2u + q * 16u : BUF_OOB;
       dmaCol[k] = (int)(q * 8u);
     } else {           // W2c block bk, row rr, logical piece q
       const unsigned pp = p - 4u * D, bk = pp >> 7, rr = (pp >> 2) & 31u;
       const unsigned q = bk * 4u + ((pp & 3u) ^ ((rr >> 2) & 3u));
-      dmaOff[k] = rr * (D * 2u) + q * 16u;
+      dmaOff[k] = DG == D || q * 8u < (unsigned)DG ? rr * (DG * 2u) + q * 16u : BUF_OOB;
       dmaCol[k] = -1;
     }
   }
@@ -222,9 +230,9 @@ __device__ __forceinline__ void dx2_body(const u16* __restrict__ X, const u16* _
     const int c = c0 + ci;
     const bool mine = ci < NCP;
     const int lim = mine ? e_end - c * 32 : 0;
-    const int rem = mine ? D * ldw * 2 - 64 * c : 0;
+    const int rem = mine ? DG * ldw * 2 - 64 * c : 0;
     const i32x4 r1 = make_rsrc_words(W1h + (size_t)c * 32, rem > 0 ? rem : 0);
-    const i32x4 r2 = make_rsrc_words(W2h + (size_t)c * 32 * D, clamp0(lim, 32) * D * 2);
+    const i32x4 r2 = make_rsrc_words(W2h + (size_t)c * 32 * DG, clamp0(lim, 32) * DG * 2);
     const int slot = RB + (ci & (NSL - 1)) * (int)SLOT + wp * 1024;
 #pragma unroll
     for (int k = 0; k < NDMA; ++k) {
@@ -245,8 +253,8 @@ __device__ __forceinline__ void dx2_body(const u16* __restrict__ X, const u16* _
     for (int ks = 0; ks < KS; ++ks) {
       u32x4 v = {0u, 0u, 0u, 0u}, w = {0u, 0u, 0u, 0u};
       if (b < B) {
-        v = *(const u32x4*)(Xh + (size_t)b * D + ks * 16 + g * 8);
-        w = *(const u32x4*)(dOh + (size_t)b * D + ks * 16 + g * 8);
+        v = *(const u32x4*)(Xh + (size_t)b * DG + ks * 16 + g * 8);
+        w = *(const u32x4*)(dOh + (size_t)b * DG + ks * 16 + g * 8);
       }
       xr[ks] = v;
       dr[ks] = w;
@@ -373,7 +381,8 @@ __device__ __forceinline__ void dx2_body(const u16* __restrict__ X, const u16* _
     }
     valu_phase();
   }
-  g2_only(NCP - 1);
+  // (at D < 64 a part with a chunk less leaves out the product of its last step's zeros)
+  if (D >= 64 || c0 + NCP <= ce) g2_only(NCP - 1);
   wait_vmcnt<0>();  // chunk loads past the last are still landing (as zeros)
   if constexpr (DES == 2) {  // part 1 hands its partial dX tile to part 0 through LDS (the rings)
     asm volatile("" ::: "memory");
@@ -400,9 +409,9 @@ __device__ __forceinline__ void dx2_body(const u16* __restrict__ X, const u16* _
       }
   }
   if (pws != nullptr)
-    store_rows<BF16, D>(acc, pws, 0, B - bt * ROWS, wp * 32, g, l32, 1);
+    store_rows<BF16, D, DG>(acc, pws, 0, B - bt * ROWS, wp * 32, g, l32, 1);
   else
-    store_rows<BF16, D>(acc, dX, (size_t)h * B * D, B, b_wave, g, l32, outf32);
+    store_rows<BF16, D, DG>(acc, dX, (size_t)h * B * DG, B, b_wave, g, l32, outf32);
 }
 
 // ------------------------------------------------------------------------------------
@@ -443,14 +452,15 @@ __device__ __forceinline__ unsigned wt_off(unsigned r, unsigned q) {
 // w taking every fourth subtile of its set; twice the programs, each half the work, for grids
 // that leave CUs idle). Waves w and w + 4 share a SIMD; their sets differ by RS / 2, so one
 // runs the schedule half a group behind the other either way.
-template <bool BF16, int D, int ACT, bool HILO, bool DZ = false, int ET = DW_ET>
+template <bool BF16, int D, int ACT, bool HILO, bool DZ = false, int ET = DW_ET, int DG = D>
 __device__ __forceinline__ void dw2_body(const u16* __restrict__ X, const u16* __restrict__ W1,
                                          const u16* __restrict__ W2, const u16* __restrict__ dO,
                                          void* __restrict__ dW1, void* __restrict__ dW2, float* __restrict__ ws,
                                          int H, int B, int E, int ldw, int nE, int nS, int rows_per_split,
                                          int outf32, int t, u16* __restrict__ dzt = nullptr, int Bp = 0) {
   static_assert(ET == DW_ET || (ET == 64 && D == 64 && !DZ), "E-tile width");
-  constexpr int KS = D / 16, NTN = D / 32;
+  static_assert(DG == D || (DG == 16 && D == 32), "columns in memory");
+  constexpr int KS = DG / 16, NTN = D / 32;
   constexpr int CG = ET / 32;            // column groups of waves
   constexpr int RS = DW2_NW / CG;        // row sets (a set takes every RS-th subtile)
   constexpr int SUB = 64 * D;            // bytes of a [32][D] subtile
@@ -480,10 +490,10 @@ __device__ __forceinline__ void dw2_body(const u16* __restrict__ X, const u16* _
   const int nsub = (b_hi - b_lo + DW_BT - 1) / DW_BT;
   const int npair = (nsub + RS - 1) / RS;
 
-  const u16* Xh = X + (size_t)h * B * D;
-  const u16* dOh = dO + (size_t)h * B * D;
-  const u16* W1h = W1 + (size_t)h * D * ldw;
-  const u16* W2h = W2 + (size_t)h * E * D;
+  const u16* Xh = X + (size_t)h * B * DG;
+  const u16* dOh = dO + (size_t)h * B * DG;
+  const u16* W1h = W1 + (size_t)h * DG * ldw;
+  const u16* W2h = W2 + (size_t)h * E * DG;
 
   // ---- weight tiles (once): W2T rows natural, W1T transposed with 2-byte writes ----
 #pragma unroll
@@ -492,13 +502,13 @@ __device__ __forceinline__ void dw2_body(const u16* __restrict__ X, const u16* _
     {  // W2 row e_prog + r, piece q
       const int r = p / (D / 8), q = p % (D / 8);
       u32x4 v = {0u, 0u, 0u, 0u};
-      if (e_prog + r < E) v = *(const u32x4*)(W2h + (size_t)(e_prog + r) * D + q * 8);
+      if (e_prog + r < E && (DG == D || q * 8 < DG)) v = *(const u32x4*)(W2h + (size_t)(e_prog + r) * DG + q * 8);
       lds_write16(W2T_OFF + (int)wt_off<ET>(r, q), v);
     }
     {  // W1 row d, columns e_prog + 8u .. + 7  ->  W1T rows 8u + j, column d
       const int d = p / (ET / 8), u = p % (ET / 8);
       u32x4 v = {0u, 0u, 0u, 0u};
-      if (e_prog + 8 * u < E) v = *(const u32x4*)(W1h + (size_t)d * ldw + e_prog + 8 * u);
+      if (e_prog + 8 * u < E && (DG == D || d < DG)) v = *(const u32x4*)(W1h + (size_t)d * ldw + e_prog + 8 * u);
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         const u16 x = (u16)(v[j >> 1] >> (16 * (j & 1)));
@@ -513,15 +523,15 @@ __device__ __forceinline__ void dw2_body(const u16* __restrict__ X, const u16* _
   for (int k = 0; k < NPL; ++k) {
     const unsigned p = k * DW2_NT + wave * 64 + lane, pr = p % (SUB / 16), o = 16u * pr;
     const unsigned r = (o % 2048u) / 64u, q = 4u * (o / 2048u) + (((o / 16u) & 3u) ^ ((r >> 2) & 3u));
-    pieceOff[k] = r * (D * 2u) + q * 16u;
+    pieceOff[k] = DG == D || q * 8u < (unsigned)DG ? r * (DG * 2u) + q * 16u : BUF_OOB;
   }
   auto issue_pair = [&](int i, int slot) {
 #pragma unroll
     for (int k = 0; k < NPL; ++k) {
       const int region = (k * DW2_NT + wave * 64) / (SUB / 16);  // wave-uniform: 2 s X of set s, 2 s + 1 dO
       const int r0 = b_lo + (RS * i + (region >> 1)) * DW_BT;
-      const int bytes = clamp0(b_hi - r0, DW_BT) * D * 2;
-      const i32x4 rs = make_rsrc_words(((region & 1) ? dOh : Xh) + (size_t)r0 * D, bytes);
+      const int bytes = clamp0(b_hi - r0, DW_BT) * DG * 2;
+      const i32x4 rs = make_rsrc_words(((region & 1) ? dOh : Xh) + (size_t)r0 * DG, bytes);
       buf_load16_lds(rs, pieceOff[k], RING_OFF + slot * PAIR + 16 * (k * DW2_NT + wave * 64));
     }
   };
@@ -661,6 +671,11 @@ __device__ __forceinline__ void dw2_body(const u16* __restrict__ X, const u16* _
     asm volatile("" ::: "memory");
   };
 
+  // at D < 64 a subtile past the program's rows is left out (X and dO are zeros there, but an infinite
+  // weight would make NaN of them); the test costs 0.4 % at H=32 B=16384 D=128 E=1024
+  auto ag2_rows = [&](int slot, int rbase) {
+    if (D >= 64 || rbase < b_hi) ag2_phase(slot, rbase);
+  };
   const std::true_type AG{};
   const std::false_type NOAG{};
   if (npair > 0) {
@@ -678,13 +693,13 @@ __device__ __forceinline__ void dw2_body(const u16* __restrict__ X, const u16* _
     // first row of the subtile set `set` takes in group i
     auto row0 = [&](int i) { return b_lo + (RS * i + set) * DW_BT; };
     if (set < RS / 2) {
-      ag2_phase(cur, row0(0));
+      ag2_rows(cur, row0(0));
       pair_end(AG);
       for (int i = 1; i < npair; ++i) {
         rotate();
         issue_pair(i + 1, next);
         g1_phase(cur);
-        ag2_phase(cur, row0(i));
+        ag2_rows(cur, row0(i));
         pair_end(AG);
       }
     } else {
@@ -692,11 +707,11 @@ __device__ __forceinline__ void dw2_body(const u16* __restrict__ X, const u16* _
       for (int i = 1; i < npair; ++i) {
         rotate();
         issue_pair(i + 1, next);
-        ag2_phase(prev, row0(i - 1));
+        ag2_rows(prev, row0(i - 1));
         g1_phase(cur);
         pair_end(AG);
       }
-      ag2_phase(cur, row0(npair - 1));
+      ag2_rows(cur, row0(npair - 1));
     }
   } else {
     wait_vmcnt<0>();
@@ -737,17 +752,17 @@ __device__ __forceinline__ void dw2_body(const u16* __restrict__ X, const u16* _
             }
           }
       }
-      dw_store<BF16, D>(a1, a2, dW1, dW2, ws, H, E, ldw, h, s, nS, e0, g, l32, outf32);
+      dw_store<BF16, D, DG>(a1, a2, dW1, dW2, ws, H, E, ldw, h, s, nS, e0, g, l32, outf32);
     }
   }
 }
 
 // dX programs as their own launch (FMLP_BWD_UNIFIED=0, FMLP_BWD_NO_DW): 8 waves, two per SIMD.
-template <bool BF16, int D, int ACT, int DES>
-__global__ void __launch_bounds__(DX2_NT) __attribute__((amdgpu_waves_per_eu(2, 2)))
+template <bool BF16, int D, int ACT, int DES, int DG = D>
+__global__ void __launch_bounds__(DX2_NT) __attribute__((amdgpu_waves_per_eu(bwd_wpe(D), bwd_wpe(D))))
 dx2_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* __restrict__ W2,
            const u16* __restrict__ dO, void* __restrict__ dX, int B, int E, int ldw, int tiles_per_head, int outf32) {
-  dx2_body<BF16, D, ACT, DES>(X, W1, W2, dO, dX, B, E, ldw, tiles_per_head, outf32, xcd_remap(blockIdx.x, gridDim.x), 0,
+  dx2_body<BF16, D, ACT, DES, DX2_NW, DG>(X, W1, W2, dO, dX, B, E, ldw, tiles_per_head, outf32, xcd_remap(blockIdx.x, gridDim.x), 0,
                               (E + 31) >> 5, nullptr);
 }
 
@@ -1015,13 +1030,13 @@ dw256_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* _
   dw_store<BF16, D>(a1, a2, dW1, dW2, ws, H, E, ldw, h, s, nS, e0, g, l32, outf32);
 }
 
-template <bool BF16, int D, int ACT, bool HILO, bool DZ, int ET = DW_ET>
-__global__ void __launch_bounds__(DW2_NT) __attribute__((amdgpu_waves_per_eu(2, 2)))
+template <bool BF16, int D, int ACT, bool HILO, bool DZ, int ET = DW_ET, int DG = D>
+__global__ void __launch_bounds__(DW2_NT) __attribute__((amdgpu_waves_per_eu(bwd_wpe(D), bwd_wpe(D))))
 dw2_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* __restrict__ W2,
            const u16* __restrict__ dO, void* __restrict__ dW1, void* __restrict__ dW2, float* __restrict__ ws,
            int H, int B, int E, int ldw, int nE, int nS, int rows_per_split, int outf32, u16* __restrict__ dzt,
            int Bp) {
-  dw2_body<BF16, D, ACT, HILO, DZ, ET>(X, W1, W2, dO, dW1, dW2, ws, H, B, E, ldw, nE, nS, rows_per_split, outf32,
+  dw2_body<BF16, D, ACT, HILO, DZ, ET, DG>(X, W1, W2, dO, dW1, dW2, ws, H, B, E, ldw, nE, nS, rows_per_split, outf32,
                                    xcd_remap(blockIdx.x, gridDim.x), dzt, Bp);
 }
 
@@ -1031,8 +1046,8 @@ dw2_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* __r
 // use 8 waves (two per SIMD); the dynamic LDS is the dW role's (the larger). Each role's
 // tiles are remapped onto XCDs within its own range (exact when its count is a multiple of 8).
 static_assert(DW2_NT == DX2_NT, "both roles run with the same workgroup size");
-template <bool BF16, int D, int ACT, bool HILO, int DES, int ET = DW_ET>
-__global__ void __launch_bounds__(DW2_NT) __attribute__((amdgpu_waves_per_eu(2, 2)))
+template <bool BF16, int D, int ACT, bool HILO, int DES, int ET = DW_ET, int DG = D>
+__global__ void __launch_bounds__(DW2_NT) __attribute__((amdgpu_waves_per_eu(bwd_wpe(D), bwd_wpe(D))))
 bwd_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* __restrict__ W2,
            const u16* __restrict__ dO, void* __restrict__ dX, void* __restrict__ dW1, void* __restrict__ dW2,
            float* __restrict__ ws, int H, int B, int E, int ldw, int nE, int nS, int rows_per_split, int n_dw,
@@ -1045,19 +1060,19 @@ bwd_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* __r
   const int T = dx_tiles_per_head, nch = (E + 31) >> 5;
   if (b >= n_rest) {
     const int u = b - n_rest, hh = u / dxs_xs, cb = (u - hh * dxs_xs) * dxs_nct;
-    dx2_body<BF16, D, ACT, DES>(X, W1, W2, dO, dX, B, E, ldw, T, outf32, hh * T + T - 1, cb, min(nch, cb + dxs_nct),
-                                dxs_ws + (size_t)u * dx2_rows<D, DES>() * D);
+    dx2_body<BF16, D, ACT, DES, DX2_NW, DG>(X, W1, W2, dO, dX, B, E, ldw, T, outf32, hh * T + T - 1, cb, min(nch, cb + dxs_nct),
+                                dxs_ws + (size_t)u * dx2_rows<D, DES>() * DG);
     return;
   }
   const int bw = dx_first ? b - n_dx : b;  // index among the dW programs (< 0 or >= n_dw: a dX program)
   if (bw >= 0 && bw < n_dw) {
-    dw2_body<BF16, D, ACT, HILO, false, ET>(X, W1, W2, dO, dW1, dW2, ws, H, B, E, ldw, nE, nS, rows_per_split, outf32,
+    dw2_body<BF16, D, ACT, HILO, false, ET, DG>(X, W1, W2, dO, dW1, dW2, ws, H, B, E, ldw, nE, nS, rows_per_split, outf32,
                                             xcd_remap(bw, n_dw));
   } else {
     const int bx = dx_first ? b : b - n_dw;
     const int m = xcd_remap(bx, n_dx);
     const int t = n_dxs > 0 ? (m / (T - 1)) * T + m % (T - 1) : m;
-    dx2_body<BF16, D, ACT, DES>(X, W1, W2, dO, dX, B, E, ldw, T, outf32, t, 0, nch, nullptr);
+    dx2_body<BF16, D, ACT, DES, DX2_NW, DG>(X, W1, W2, dO, dX, B, E, ldw, T, outf32, t, 0, nch, nullptr);
   }
 }
 
@@ -1389,6 +1404,7 @@ dxg_kernel(const u16* __restrict__ dzt, const u16* __restrict__ W1, void* __rest
 // Constants fitted to MI355X timings of 14 shapes x activations x (order, nS); the choice the
 // estimate makes is within 2.5 % of the best measured one for each of them.
 // ------------------------------------------------------------------------------------
+#if FMLP_BWD_PART == 0
 namespace {
 
 constexpr double kPlanFixedUs = 3.0;      // per program
@@ -1453,7 +1469,12 @@ BwdPlan make_plan(int64_t H, int64_t B, int64_t D, int64_t E, int act, bool hilo
     }
   }
   BwdPlan p{};
-  const long long N = num_cus > 0 ? num_cus : 1;
+  // program slots: one per CU; at D < 64 two workgroups share a CU, each at half its rate (measured
+  // at H=32 B=4096 D=32 E=512 bf16 SiLU: planned as one per CU the backward took 63 us, nS = 2
+  // instead of 1 takes 61 us; at H=4 B=16384 E=1024 nS = 4 / 8 / 16 take 64 / 55 / 58 us)
+  const int per_cu = D < 64 ? 2 : 1;
+  const double rate = kPlanRate / per_cu;
+  const long long N = (num_cus > 0 ? num_cus : 1) * (long long)per_cu;
   // dW programs of ET E-columns: 128, or at D = 64 with the dX programs' E split also 64 (twice
   // the programs, each half the work, for grids that leave CUs idle); FMLP_BWD_ET (read once per
   // process) forces 128 or 64 where allowed
@@ -1464,11 +1485,12 @@ BwdPlan make_plan(int64_t H, int64_t B, int64_t D, int64_t E, int act, bool hilo
   // dX programs of 256 rows, or at D = 64 of 128 rows with E in two parts (half the time each)
   auto n_dx_for = [&](int des) { return H * ((B + DX2_ROWS / des - 1) / (DX2_ROWS / des)); };
   auto tx_for = [&](int des) {
-    return kPlanFixedUs + (double)(DX2_ROWS / des) * E * (3.0 * D + valu_dx(act) * kPlanValuMacs) / kPlanRate;
+    return kPlanFixedUs + (double)(DX2_ROWS / des) * E * (3.0 * D + valu_dx(act) * kPlanValuMacs) / rate;
   };
-  const int max_des = D == 64 ? 2 : 1;
+  const int max_des = D <= 64 ? 2 : 1;
+  const int min_des = D < 64 ? 2 : 1;  // D < 64 programs exist in this form only
   auto w_per_row_for = [&](long long et) {
-    return (double)et * ((hilo ? 6.0 : 4.0) * D + valu_dw(act) * kPlanValuMacs) / kPlanRate;
+    return (double)et * ((hilo ? 6.0 : 4.0) * D + valu_dw(act) * kPlanValuMacs) / rate;
   };
   const double w_per_row = w_per_row_for(DW_ET);
   // candidates nS = 1, 2, 4, ... up to B / 256 and two dW programs per CU (which keeps the fp32
@@ -1501,12 +1523,12 @@ BwdPlan make_plan(int64_t H, int64_t B, int64_t D, int64_t E, int act, bool hilo
   long long best_ns = 1;
   bool best_dx_first = false, best_dxs = false;
   int best_des = 1, best_et = DW_ET;
-  for (int des = 1; des <= max_des; ++des) {
-    if (des_env > 0 && des != des_env) continue;
+  for (int des = min_des; des <= max_des; ++des) {
+    if (des_env > 0 && des != des_env && min_des != max_des) continue;
     if (fixed_des > 0 && des != fixed_des) continue;
     const long long n_dx = n_dx_for(des), T_dx = n_dx / (H > 0 ? H : 1);
     const double tx = tx_for(des);
-    const bool rag = B % (DX2_ROWS / des) != 0 && T_dx >= 2 && dxs_xs >= 2 && dxs_env != 0 && fixed_dxs != 0;
+    const bool rag = B % (DX2_ROWS / des) != 0 && T_dx >= 2 && dxs_xs >= 2 && dxs_env != 0 && fixed_dxs != 0 && D >= 64;
     for (int et = DW_ET; et >= 64; et /= 2) {
       if (et != DW_ET && !(D == 64 && des == 2)) continue;
       if (et_env > 0 && et != et_env && (et_env == DW_ET || (D == 64 && des == 2))) continue;
@@ -1538,7 +1560,8 @@ BwdPlan make_plan(int64_t H, int64_t B, int64_t D, int64_t E, int act, bool hilo
               if (over > 0.0) t += std::max(over / (double)N, tp);
               t += kPlanLaunchUs;
             }
-            if (best_t == 0.0 || t < best_t) {
+            // (D < 64: a finer split has to win by more than the estimate's error there)
+            if (best_t == 0.0 || t < best_t * (D < 64 && eff > best_ns ? 0.9 : 1.0)) {
               best_t = t;
               best_ns = eff;
               best_dx_first = o == 2;
@@ -1571,7 +1594,7 @@ BwdPlan make_plan(int64_t H, int64_t B, int64_t D, int64_t E, int act, bool hilo
   const size_t dz_head = (size_t)nE_for(DW_ET) * DW_ET * (size_t)Bp * 2u;
   double best_dz = 0.0;
   long long best_dz_ns = 1;
-  if (dz_want != 0 && B > 0 && dz_head < ((size_t)1 << 31)) {
+  if (dz_want != 0 && D >= 64 && B > 0 && dz_head < ((size_t)1 << 31)) {
     const double t_dx = kPlanDzFixedUs + (double)H * dz_head / kPlanDzBytesPerUs;
     for (long long ns = 1; ns <= (ns_env > 0 ? 1 : cap); ns *= 2) {
       const long long want = ns_env > 0 ? (ns_env < max_ns ? ns_env : max_ns) : ns;
@@ -1691,6 +1714,8 @@ Dw256Plan plan_dw256(int64_t H, int64_t B, int64_t E, bool hilo, int num_cus, si
   return p;
 }
 
+#endif  // FMLP_BWD_PART == 0
+
 // dynamic LDS of the dW role: a 3-group ring of subtiles and the two weight tiles
 template <int D, int ET>
 constexpr size_t dw_lds_bytes() {
@@ -1714,7 +1739,7 @@ static hipError_t launch_dw_reduce(const BwdArgs& a, int nS, hipStream_t st) {
   return hipGetLastError();
 }
 
-template <bool BF16, int D, int ACT, int DES, int ET>
+template <bool BF16, int D, int ACT, int DES, int ET, int DG = D>
 static hipError_t launch_bwd_t(const BwdArgs& a, const BwdPlan& p, hipStream_t st) {
   if (p.n_dw + p.n_dx + p.n_dxs > 0x7fffffffLL || (long long)p.dx_tiles_per_head * a.H > 0x7fffffffLL)
     return hipErrorInvalidValue;
@@ -1724,7 +1749,7 @@ static hipError_t launch_bwd_t(const BwdArgs& a, const BwdPlan& p, hipStream_t s
   constexpr size_t lds = std::max<size_t>(dw_lds_bytes<D, ET>(), (size_t)DES * DX_NSLOT * 128u * D);
   static_assert(dw_lds_bytes<D, DW_ET>() == 1280u * D, "the 128-column form's LDS");
   auto reduce = [&]() { return launch_dw_reduce<BF16>(a, p.nS, st); };
-  if (p.dz && a.want_dx && a.want_dw) {  // stored-dZ form: dW programs storing dZ, their reduction, then the dX GEMM
+  if constexpr (D >= 64) if (p.dz && a.want_dx && a.want_dw) {  // stored-dZ form: dW programs storing dZ, their reduction, then the dX GEMM
     u16* dzt = (u16*)((char*)a.ws + p.dz_off);
     const int Ep = p.nE * DW_ET;
     auto launch_w = [&](auto k) {
@@ -1776,12 +1801,13 @@ static hipError_t launch_bwd_t(const BwdArgs& a, const BwdPlan& p, hipStream_t s
                          p.dxs_nct, dxs_ws);
       return hipGetLastError();
     };
-    e = a.dw_hilo ? launch_u(bwd_kernel<BF16, D, ACT, true, DES, ET>) : launch_u(bwd_kernel<BF16, D, ACT, false, DES, ET>);
+    e = a.dw_hilo ? launch_u(bwd_kernel<BF16, D, ACT, true, DES, ET, DG>)
+                  : launch_u(bwd_kernel<BF16, D, ACT, false, DES, ET, DG>);
     if (e != hipSuccess) return e;
     if (a.want_dw && (e = reduce()) != hipSuccess) return e;
     if (p.n_dxs == 0) return hipSuccess;
     // the ragged dX tiles' partials: split tile s is head s's last tile
-    return launch_tile_reduce(dxs_ws, a.dx, BF16, (int)a.B, D, DX2_ROWS / DES, (int)a.H, p.dx_tiles_per_head,
+    return launch_tile_reduce(dxs_ws, a.dx, BF16, (int)a.B, DG, DX2_ROWS / DES, (int)a.H, p.dx_tiles_per_head,
                               p.dxs_xs, (int)a.H, a.out_f32 ? 1 : 0, st);
   }
   if (p.n_dw > 0 && a.want_dw) {
@@ -1794,15 +1820,15 @@ static hipError_t launch_bwd_t(const BwdArgs& a, const BwdPlan& p, hipStream_t s
                          (int)a.B, (int)a.E, (int)a.ldw, p.nE, p.nS, p.rows_per_split, a.out_f32 ? 1 : 0, (u16*)nullptr, 0);
       return hipGetLastError();
     };
-    e = a.dw_hilo ? launch_w(dw2_kernel<BF16, D, ACT, true, false, ET>)
-                  : launch_w(dw2_kernel<BF16, D, ACT, false, false, ET>);
+    e = a.dw_hilo ? launch_w(dw2_kernel<BF16, D, ACT, true, false, ET, DG>)
+                  : launch_w(dw2_kernel<BF16, D, ACT, false, false, ET, DG>);
     if (e != hipSuccess) return e;
     if ((e = reduce()) != hipSuccess) return e;
   }
   const long long n_dx_all = (long long)p.dx_tiles_per_head * a.H;  // whole tiles only here
   if (n_dx_all > 0 && a.want_dx) {
     const size_t lds_x = (size_t)DES * DX_NSLOT * 128u * D;  // the chunk ring(s)
-    auto k = dx2_kernel<BF16, D, ACT, DES>;
+    auto k = dx2_kernel<BF16, D, ACT, DES, DG>;
     static std::atomic<unsigned long long> lds_set{0};
     e = set_lds_once((const void*)k, (int)lds_x, lds_set);
     if (e != hipSuccess) return e;
@@ -1814,25 +1840,27 @@ static hipError_t launch_bwd_t(const BwdArgs& a, const BwdPlan& p, hipStream_t s
   return hipSuccess;
 }
 
-template <bool BF16, int D, int ACT>
+template <bool BF16, int D, int ACT, int DG>
 static hipError_t launch_bwd_e(const BwdArgs& a, const BwdPlan& p, hipStream_t st) {
   if constexpr (D == 64) {
     if (p.dx_es == 2 && p.et_w == 64) return launch_bwd_t<BF16, D, ACT, 2, 64>(a, p, st);
     if (p.dx_es == 2) return launch_bwd_t<BF16, D, ACT, 2, DW_ET>(a, p, st);
   }
-  return launch_bwd_t<BF16, D, ACT, 1, DW_ET>(a, p, st);
+  if constexpr (D < 64) return launch_bwd_t<BF16, D, ACT, 2, DW_ET, DG>(a, p, st);
+  else return launch_bwd_t<BF16, D, ACT, 1, DW_ET>(a, p, st);
 }
 
-template <bool BF16, int D>
+template <bool BF16, int D, int DG = D>
 static hipError_t launch_bwd_a(const BwdArgs& a, const BwdPlan& p, hipStream_t st) {
   switch (a.act) {
-    case ACT_SILU: return launch_bwd_e<BF16, D, ACT_SILU>(a, p, st);
-    case ACT_LEAKY: return launch_bwd_e<BF16, D, ACT_LEAKY>(a, p, st);
-    case ACT_SIGMOID: return launch_bwd_e<BF16, D, ACT_SIGMOID>(a, p, st);
-    default: return launch_bwd_e<BF16, D, ACT_NONE>(a, p, st);
+    case ACT_SILU: return launch_bwd_e<BF16, D, ACT_SILU, DG>(a, p, st);
+    case ACT_LEAKY: return launch_bwd_e<BF16, D, ACT_LEAKY, DG>(a, p, st);
+    case ACT_SIGMOID: return launch_bwd_e<BF16, D, ACT_SIGMOID, DG>(a, p, st);
+    default: return launch_bwd_e<BF16, D, ACT_NONE, DG>(a, p, st);
   }
 }
 
+#if FMLP_BWD_PART == 0
 template <bool BF16, int ACT>
 static hipError_t launch_dx256_t(const BwdArgs& a, hipStream_t st) {
   const long long tph = (a.B + 127) / 128, grid = tph * a.H;
@@ -1893,13 +1921,28 @@ hipError_t launch_dw256(const BwdArgs& a, const Dw256Plan& p, hipStream_t st) {
   return a.dw_hilo ? launch_dw256_a<false, true>(a, p, st) : launch_dw256_a<false, false>(a, p, st);
 }
 
-hipError_t launch_bwd(const BwdArgs& a, const BwdPlan& p, hipStream_t st) {
-  if (a.bf16) {
-    if (a.D == 128) return launch_bwd_a<true, 128>(a, p, st);
-    return launch_bwd_a<true, 64>(a, p, st);
-  }
-  if (a.D == 128) return launch_bwd_a<false, 128>(a, p, st);
-  return launch_bwd_a<false, 64>(a, p, st);
+#endif  // FMLP_BWD_PART == 0
+
+// One object per D (build.py compiles this file once for each value of FMLP_BWD_PART; 0 holds the
+// plans, the D = 256 programs and the dispatch), so that they compile side by side.
+#if FMLP_BWD_PART == 64
+hipError_t launch_bwd_d64(const BwdArgs& a, const BwdPlan& p, hipStream_t st) {
+  return a.bf16 ? launch_bwd_a<true, 64>(a, p, st) : launch_bwd_a<false, 64>(a, p, st);
 }
+#elif FMLP_BWD_PART == 128
+hipError_t launch_bwd_d128(const BwdArgs& a, const BwdPlan& p, hipStream_t st) {
+  return a.bf16 ? launch_bwd_a<true, 128>(a, p, st) : launch_bwd_a<false, 128>(a, p, st);
+}
+#elif FMLP_BWD_PART == 32
+hipError_t launch_bwd_d32(const BwdArgs& a, const BwdPlan& p, hipStream_t st) {
+  if (a.D == 16) return a.bf16 ? launch_bwd_a<true, 32, 16>(a, p, st) : launch_bwd_a<false, 32, 16>(a, p, st);
+  return a.bf16 ? launch_bwd_a<true, 32>(a, p, st) : launch_bwd_a<false, 32>(a, p, st);
+}
+#else
+hipError_t launch_bwd(const BwdArgs& a, const BwdPlan& p, hipStream_t st) {
+  if (a.D == 128) return launch_bwd_d128(a, p, st);
+  return a.D == 64 ? launch_bwd_d64(a, p, st) : launch_bwd_d32(a, p, st);
+}
+#endif
 
 }  // namespace fmlp

@@ -59,10 +59,10 @@ __device__ __forceinline__ TileId main_tile(int m, int n_split, int H, int T) {
   const int m2 = m - first, tb = T - a - 1;
   return TileId{H - b + m2 / tb, m2 % tb};
 }
-// Waves per workgroup: D / 16 up to D = 128 (two waves per SIMD, the threads covering a chunk's
-// 4 D pieces of W1c and of W2c once); 4 at D = 256 (one wave per SIMD, whose O accumulators alone
+// Waves per workgroup: D / 16 at D = 64 and 128 (two waves per SIMD, the threads covering a chunk's
+// 4 D pieces of W1c and of W2c once); 4 at D = 32 (half the threads load W1c, half W2c) and at D = 256 (one wave per SIMD, whose O accumulators alone
 // take 128 registers; each thread loads 4 pieces per region).
-__host__ __device__ constexpr int fwd_waves(int D) { return D <= 128 ? D / 16 : 4; }
+__host__ __device__ constexpr int fwd_waves(int D) { return D > 32 && D <= 128 ? D / 16 : 4; }
 // OC: waves per SIMD the kernel is built for. Two up to D = 128 (each workgroup with an 8-slot
 // ring); at D = 64 without the E split three, each workgroup then with a 4-slot ring (32 KB) so
 // that three fit on a CU: the D = 64 kernel is VALU-issue bound (two activation elements per
@@ -74,33 +74,46 @@ __host__ __device__ constexpr int fwd_wpe(int D, int OC) { return D <= 128 ? OC 
 // loaded ahead; at D = 256 a chunk is 32 KB, so four slots, a barrier per chunk, two ahead, and
 // the same for the 4-slot rings of the higher-occupancy D = 64 builds
 constexpr int FWD_PF = 4;  // chunks loaded ahead with one barrier per chunk (D <= 128)
-__host__ __device__ constexpr bool fwd_small_ring(int D, int OC, int ES = 1) { return D > 128 || OC > 2 || ES > 2; }
+__host__ __device__ constexpr bool fwd_small_ring(int D, int OC, int ES = 1) {
+  return D > 128 || (D > 32 && OC > 2) || ES > 2;
+}
 __host__ __device__ constexpr int fwd_nslot(int D, int OC, int ES = 1) { return fwd_small_ring(D, OC, ES) ? 4 : 8; }
 __host__ __device__ constexpr int fwd_sb(int D, int OC, int ES = 1) { return fwd_small_ring(D, OC, ES) ? 1 : 2; }
 __host__ __device__ constexpr int fwd_pf(int D, int OC, int ES = 1) {
   return fwd_small_ring(D, OC, ES) ? fwd_nslot(D, OC, ES) - 2 : FWD_PF + fwd_sb(D, OC, ES) - 1;
 }
 
-template <bool BF16, int D, int ACT, int ES, int OC = 2, int NWP = fwd_waves(D)>
+// DG: columns of X, W2 and O and rows of W1 in memory (D, or 16 with D = 32: the tiles are D wide
+// with zeros past DG, but X W1 takes only the DG / 16 K steps that exist).
+// D = 32 does 16 activation elements per four MFMAs (464 VALU clocks against 128 matrix clocks per
+// 32 x 32 tile), so it is bound by the activation; four waves per SIMD (OC = 4, an 8-slot ring of
+// 32 KB each) hide the operand reads. H=32 B=4096 D=32 E=512 bf16 SiLU: forward 23 us, forward +
+// backward 720 us on the generic kernels -> 76-78 us.
+template <bool BF16, int D, int ACT, int ES, int OC = 2, int NWP = fwd_waves(D), int DG = D>
 __global__ void __launch_bounds__(NWP * ES * 64) __attribute__((amdgpu_waves_per_eu(fwd_wpe(D, OC), fwd_wpe(D, OC))))
 fwd_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* __restrict__ W2,
            void* __restrict__ O, int B, int E, int ldw, int H, int tiles_per_head, int outf32, int n_main,
            int n_split, int xs, int nct, float* __restrict__ ws) {
   constexpr int NW = NWP, NT = NW * 64;  // waves, threads of one E part
-  constexpr int KS = D / 16;           // K steps of GEMM1 (= GEMM2 operand count 2 * D/32)
+  constexpr int KS = DG / 16;          // K steps of GEMM1 (at DG = D also GEMM2's operand count 2 * D/32)
   constexpr int NTN = D / 32;          // N tiles of GEMM2
   constexpr int BB = NW * 32;          // rows per workgroup (32 per wave)
-  static_assert(ES == 1 || (ES == 2 && D == 64) || (ES == 4 && D == 64 && NWP == 2), "E split");
+  static_assert(ES == 1 || (ES == 2 && D <= 64) || (ES == 4 && D <= 64 && NWP == 2), "E split");
+  static_assert(DG == D || (DG == 16 && D == 32), "columns in memory");
   static_assert(NWP == fwd_waves(D) || (NWP == 2 && ES == 4), "waves per E part");
   constexpr unsigned SLOT = 128u * D;  // bytes per ring slot: W1c (64*D) + W2c (64*D)
   constexpr unsigned W2OFF = 64u * D;
   // SB: chunk iterations per workgroup barrier. The loads run SB - 1 chunks further ahead so
   // that a barrier covers the SB chunks read after it (measured on MI355X at cfg4: SB = 2 is
   // about 1 % faster than a barrier per chunk).
-  static_assert(OC == 2 || (D == 64 && ES == 1 && OC == 3), "occupancy");
+  static_assert(OC == 2 || (D == 64 && ES == 1 && OC == 3) || (D == 32 && ES == 1 && OC == 4), "occupancy");
   constexpr int SB = fwd_sb(D, OC, ES);
   constexpr int NSLOT = fwd_nslot(D, OC, ES), PF = fwd_pf(D, OC, ES);
-  constexpr int NPR = 4 * D / NT;  // 16-byte pieces per thread per region (W1c or W2c) of a chunk
+  // 16-byte pieces per thread per region (W1c or W2c) of a chunk; HALF: each thread loads one piece
+  // of one region, the lower half of the waves W1c's
+  constexpr bool HALF = NT > 4 * D;
+  constexpr int NPR = HALF ? 1 : 4 * D / NT;
+  constexpr int NLD = HALF ? 1 : 2 * NPR;  // loads per thread per chunk
   static_assert(SB == 1 || SB == 2, "barrier spacing");
   static_assert(PF >= 2 && PF <= NSLOT - 2 - (SB - 1) && (NSLOT & (NSLOT - 1)) == 0, "ring");
   auto rslot = [](int c) -> unsigned { return (unsigned)(c & (NSLOT - 1)); };  // ring slot of chunk c
@@ -128,15 +141,18 @@ fwd_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* __r
   }
   const int h = tile.h, bt = tile.bt;
   // chunks of this part: global chunk c0 + c for c = 0 .. NC - 1 (the last part's last chunks
-  // may lie past the range: they load as zeros and add nothing)
+  // may lie past the range: they load as zeros and add nothing). At D < 64 the parts' shares differ
+  // by at most one, and a part with a chunk less leaves the product of its last step out, so that
+  // a NaN which an infinite X makes of those zeros is not added.
   const int NC = (ce - cb + ES - 1) / ES;
-  const int c0 = cb + part * NC;
-  const int e_end = min(E, ce * 32);  // columns of W1 (rows of W2) this workgroup reads
+  const int c0 = D < 64 ? cb + part * (ce - cb) / ES : cb + part * NC;
+  const int c1 = ES > 1 && D < 64 ? cb + (part + 1) * (ce - cb) / ES : ce;
+  const int e_end = min(E, c1 * 32);  // columns of W1 (rows of W2) this workgroup reads
   const unsigned RB = (unsigned)part * NSLOT * 128u * D;  // this part's ring
 
-  const u16* Xh = X + (size_t)h * B * D;
-  const u16* W1h = W1 + (size_t)h * D * ldw;  // rows of ldw elements (E, or E padded to 8)
-  const u16* W2h = W2 + (size_t)h * E * D;
+  const u16* Xh = X + (size_t)h * B * DG;
+  const u16* W1h = W1 + (size_t)h * DG * ldw;  // rows of ldw elements (E, or E padded to 8)
+  const u16* W2h = W2 + (size_t)h * E * DG;
   const int b_wave = bt * BB + wave * 32;
 
   // ---- chunk staging: buffer-to-LDS loads, PF chunks ahead into an NSLOT-slot ring ----
@@ -144,23 +160,36 @@ fwd_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* __r
   // 16 p (row d = p / 4, columns 8 (p % 4) ..), piece p of W2c at W2OFF + 16 p (block p / 128,
   // row (p / 4) % 32, columns 32 (p / 128) + 8 (p % 4) ..). Columns past E (and every piece of a
   // chunk past the last) are out of range and land as zeros.
-  static_assert(NPR * NT == 4 * D, "the threads cover a region's pieces");
+  static_assert(HALF ? NT == 8 * D : NPR * NT == 4 * D, "the threads cover a region's pieces");
   int colq[NPR];
   unsigned dOffW1[NPR], dOffW2[NPR];
 #pragma unroll
   for (int k = 0; k < NPR; ++k) {
-    const unsigned p = (unsigned)(tid + k * NT);
+    const unsigned p = (unsigned)((HALF ? tid & (4 * D - 1) : tid) + k * NT);
     colq[k] = (int)(p & 3u) * 8;
     dOffW1[k] = (p >> 2) * (unsigned)ldw * 2u + (p & 3u) * 16u;
-    dOffW2[k] = ((p >> 2) & 31u) * (D * 2u) + (p >> 7) * 64u + (p & 3u) * 16u;
+    dOffW2[k] = ((p >> 2) & 31u) * (DG * 2u) + (p >> 7) * 64u + (p & 3u) * 16u;
+    if (DG < D) {  // columns of W2c that do not exist (rows of W1 past DG are never read)
+      if ((p & 3u) * 8u >= (unsigned)DG) dOffW2[k] = BUF_OOB;
+      if ((p >> 2) >= (unsigned)DG) dOffW1[k] = BUF_OOB;
+    }
   }
   auto dma_chunk = [&](int c) {
     const int cg = c0 + c;
     const int lim = e_end - cg * 32;
-    const int rem = D * ldw * 2 - 64 * cg;
+    const int rem = DG * ldw * 2 - 64 * cg;
     const i32x4 r1 = make_rsrc_words(W1h + (size_t)cg * 32, rem > 0 ? rem : 0);
-    const i32x4 r2 = make_rsrc_words(W2h + (size_t)cg * 32 * D, clamp0(lim, 32) * D * 2);
+    const i32x4 r2 = make_rsrc_words(W2h + (size_t)cg * 32 * DG, clamp0(lim, 32) * DG * 2);
     const int slot = (int)RB + (int)rslot(c) * (int)SLOT + wave * 1024;
+    if constexpr (HALF) {  // a wave-uniform choice of the region, no branch
+      const bool w1 = wave < NW / 2;
+      i32x4 r;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) r[i] = __builtin_amdgcn_readfirstlane(w1 ? r1[i] : r2[i]);
+      const unsigned o1 = colq[0] < lim ? dOffW1[0] : BUF_OOB;
+      buf_load16_lds(r, w1 ? o1 : dOffW2[0], slot);
+      return;
+    }
 #pragma unroll
     for (int k = 0; k < NPR; ++k) {
       buf_load16_lds(r1, colq[k] < lim ? dOffW1[k] : BUF_OOB, slot + k * NT * 16);
@@ -170,7 +199,7 @@ fwd_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* __r
   // end of a chunk: the LDS stores are retired and visible after the barrier; the loads of
   // the chunk after next stay in flight (their data is waited for where it is stored)
   auto chunk_end = [&]() {
-    wait_vmcnt<2 * NPR * (PF - 1 - SB)>();  // this wave's pieces of the SB chunks read next
+    wait_vmcnt<NLD * (PF - 1 - SB)>();  // this wave's pieces of the SB chunks read next
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
@@ -184,7 +213,7 @@ fwd_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* __r
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       u32x4 v = {0u, 0u, 0u, 0u};
-      if (b < B) v = *(const u32x4*)(Xh + (size_t)b * D + ks * 16 + g * 8);
+      if (b < B) v = *(const u32x4*)(Xh + (size_t)b * DG + ks * 16 + g * 8);
       xr[ks] = v;
     }
   }
@@ -210,7 +239,7 @@ fwd_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* __r
   // ---- prologue: chunks 0 .. PF-1 requested, chunk 0 waited for, Z^T(0) ----
 #pragma unroll
   for (int c = 0; c < PF; ++c) dma_chunk(c);
-  wait_vmcnt<2 * NPR * (PF - 2)>();  // chunks 0 and 1
+  wait_vmcnt<NLD * (PF - 2)>();  // chunks 0 and 1
   __builtin_amdgcn_s_waitcnt(0xC07F);
   asm volatile("" ::: "memory");
   __builtin_amdgcn_s_barrier();
@@ -234,7 +263,7 @@ fwd_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* __r
   auto iter = [&](auto G1, auto G2, auto SYNC, int c, St& in, St& out) {
     constexpr bool DO_G1 = decltype(G1)::value;
     constexpr bool DO_G2 = decltype(G2)::value;
-    constexpr int N1 = DO_G1 ? KS : 0, N2 = DO_G2 ? KS : 0, NOPS = N1 + N2;
+    constexpr int N1 = DO_G1 ? KS : 0, N2 = DO_G2 ? 2 * NTN : 0, NOPS = N1 + N2;
     // activation elements of step j: [16 j / NOPS, 16 (j + 1) / NOPS) (one or two per step at
     // D <= 128, one every other step at D = 256)
     const unsigned base1 = RB + rslot(c + 1) * SLOT, base2 = RB + rslot(c - 1) * SLOT;
@@ -243,8 +272,8 @@ fwd_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* __r
     dma_chunk(c + PF);
 
     // op j: G1 and G2 alternate when both are present
-    auto is_g1 = [&](int j) { return DO_G1 && (!DO_G2 || (j % 2 == 0)); };
-    auto idx = [&](int j) { return (DO_G1 && DO_G2) ? j / 2 : j; };
+    auto is_g1 = [&](int j) { return N1 == N2 ? j % 2 == 0 : !sched_is_g2(j, N1, N2); };
+    auto idx = [&](int j) { return N1 == N2 ? j / 2 : sched_index(j, N1, N2); };
     auto fetch = [&](int j) {
       const int k = idx(j);
       return is_g1(j) ? opndA(base1, k) : opndB(base2, k / NTN, k % NTN);
@@ -280,6 +309,7 @@ fwd_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* __r
     if constexpr (decltype(SYNC)::value) chunk_end();
   };
   auto last_gemm2 = [&](const St& st) {
+    if (ES > 1 && D < 64 && c0 + NC > c1) return;
     const unsigned base2 = RB + rslot(NC - 1) * SLOT;
 #pragma unroll
     for (int s = 0; s < 2; ++s)
@@ -349,9 +379,9 @@ fwd_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* __r
   // when the caller asked for them (FMLP_OUT_F32), else rounded to the io dtype; a split
   // tile's partial as fp32 rows of its workspace block ----
   if (split)
-    store_rows<BF16, D>(o, ws, (size_t)u * BB * D, B - bt * BB, wave * 32, g, l32, 1);
+    store_rows<BF16, D, DG>(o, ws, (size_t)u * BB * DG, B - bt * BB, wave * 32, g, l32, 1);
   else
-    store_rows<BF16, D>(o, O, (size_t)h * B * D, B, b_wave, g, l32, outf32);
+    store_rows<BF16, D, DG>(o, O, (size_t)h * B * DG, B, b_wave, g, l32, outf32);
 }
 
 // Sum of the split tiles' partials: O rows of split tile s = sum over p < xs of
@@ -453,7 +483,7 @@ FwdPlan fwd_plan(int64_t H, int64_t B, int64_t D, int64_t E, int num_cus, size_t
   // FMLP_FWD_SPLIT (read once per process): 0 = never, 1 = whenever E allows, else this rule
   static const int force = env_int("FMLP_FWD_SPLIT", -1);
   static const int xs_env = env_int("FMLP_FWD_XS", -1);
-  p.es = (D == 64 && E > 64 && (force == 1 || (force != 0 && R <= N))) ? 2 : 1;
+  p.es = (D <= 64 && E > 64 && (force == 1 || (force != 0 && R <= N))) ? 2 : 1;
   p.n_main = R;
   p.xs = 1;
   p.nct = (int)nch;
@@ -470,7 +500,7 @@ FwdPlan fwd_plan(int64_t H, int64_t B, int64_t D, int64_t E, int num_cus, size_t
     p.n_main = R64;
     return p;
   }
-  if (xs_env == 0 || R <= 0) return p;
+  if (xs_env == 0 || R <= 0 || D < 64) return p;  // (four D < 64 workgroups share a CU: rounds are short)
   long long cand = 0;
   int es = p.es;
   if (R > N) {
@@ -499,10 +529,10 @@ FwdPlan fwd_plan(int64_t H, int64_t B, int64_t D, int64_t E, int num_cus, size_t
   return p;
 }
 
-template <bool BF16, int D, int ACT, int ES, int OC = 2, int NWP = fwd_waves(D)>
+template <bool BF16, int D, int ACT, int ES, int OC = 2, int NWP = fwd_waves(D), int DG = D>
 static hipError_t launch_fwd_e(const FwdArgs& a, const FwdPlan& p, int tiles_per_head, hipStream_t st) {
   const size_t lds = (size_t)ES * fwd_nslot(D, OC, ES) * 128u * D;
-  auto k = fwd_kernel<BF16, D, ACT, ES, OC, NWP>;
+  auto k = fwd_kernel<BF16, D, ACT, ES, OC, NWP, DG>;
   static std::atomic<unsigned long long> lds_set{0};
   hipError_t e = set_lds_once((const void*)k, (int)lds, lds_set);
   if (e != hipSuccess) return e;
@@ -530,12 +560,12 @@ hipError_t launch_tile_reduce(const float* ws, void* out, bool bf16, int B, int 
   return hipGetLastError();
 }
 
-template <bool BF16, int D, int ACT>
+template <bool BF16, int D, int ACT, int DG = D>
 static hipError_t launch_fwd_t(const FwdArgs& a, hipStream_t st) {
   constexpr int BB0 = 32 * fwd_waves(D);
   if ((a.B + BB0 - 1) / BB0 * a.H <= 0) return hipSuccess;
   if ((a.B + 63) / 64 * a.H > 0x7fffffffLL) return hipErrorInvalidValue;
-  const FwdPlan p = fwd_plan(a.H, a.B, D, a.E, a.num_cus, a.ws != nullptr ? a.ws_bytes : 0);
+  const FwdPlan p = fwd_plan(a.H, a.B, DG, a.E, a.num_cus, a.ws != nullptr ? a.ws_bytes : 0);
   const int BB = 32 * (p.nwp > 0 ? p.nwp : fwd_waves(D));
   const int tiles_per_head = (int)((a.B + BB - 1) / BB);
   if constexpr (D == 64) {
@@ -545,16 +575,22 @@ static hipError_t launch_fwd_t(const FwdArgs& a, hipStream_t st) {
     static const int occ = env_int("FMLP_FWD_OCC", 3);
     if (occ != 2) return launch_fwd_e<BF16, D, ACT, 1, 3>(a, p, tiles_per_head, st);
   }
-  return launch_fwd_e<BF16, D, ACT, 1>(a, p, tiles_per_head, st);
+  if constexpr (D == 32) {
+    if (p.es == 4) return launch_fwd_e<BF16, D, ACT, 4, 2, 2, DG>(a, p, tiles_per_head, st);
+    if (p.es == 2) return launch_fwd_e<BF16, D, ACT, 2, 2, fwd_waves(D), DG>(a, p, tiles_per_head, st);
+    return launch_fwd_e<BF16, D, ACT, 1, 4, fwd_waves(D), DG>(a, p, tiles_per_head, st);
+  } else {
+    return launch_fwd_e<BF16, D, ACT, 1>(a, p, tiles_per_head, st);
+  }
 }
 
-template <bool BF16, int D>
+template <bool BF16, int D, int DG = D>
 static hipError_t launch_fwd_a(const FwdArgs& a, hipStream_t st) {
   switch (a.act) {
-    case ACT_SILU: return launch_fwd_t<BF16, D, ACT_SILU>(a, st);
-    case ACT_LEAKY: return launch_fwd_t<BF16, D, ACT_LEAKY>(a, st);
-    case ACT_SIGMOID: return launch_fwd_t<BF16, D, ACT_SIGMOID>(a, st);
-    default: return launch_fwd_t<BF16, D, ACT_NONE>(a, st);
+    case ACT_SILU: return launch_fwd_t<BF16, D, ACT_SILU, DG>(a, st);
+    case ACT_LEAKY: return launch_fwd_t<BF16, D, ACT_LEAKY, DG>(a, st);
+    case ACT_SIGMOID: return launch_fwd_t<BF16, D, ACT_SIGMOID, DG>(a, st);
+    default: return launch_fwd_t<BF16, D, ACT_NONE, DG>(a, st);
   }
 }
 
@@ -562,10 +598,14 @@ hipError_t launch_fwd(const FwdArgs& a, hipStream_t st) {
   if (a.bf16) {
     if (a.D == 256) return launch_fwd_a<true, 256>(a, st);
     if (a.D == 128) return launch_fwd_a<true, 128>(a, st);
+    if (a.D == 32) return launch_fwd_a<true, 32>(a, st);
+    if (a.D == 16) return launch_fwd_a<true, 32, 16>(a, st);
     return launch_fwd_a<true, 64>(a, st);
   }
   if (a.D == 256) return launch_fwd_a<false, 256>(a, st);
   if (a.D == 128) return launch_fwd_a<false, 128>(a, st);
+  if (a.D == 32) return launch_fwd_a<false, 32>(a, st);
+  if (a.D == 16) return launch_fwd_a<false, 32, 16>(a, st);
   return launch_fwd_a<false, 64>(a, st);
 }
 

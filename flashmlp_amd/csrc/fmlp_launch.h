@@ -161,6 +161,9 @@ hipError_t launch_fwd(const FwdArgs& a, hipStream_t st);
 hipError_t launch_tile_reduce(const float* ws, void* out, bool bf16, int B, int D, int BB, int H, int T, int xs,
                               int n_split, int outf32, hipStream_t st);
 hipError_t launch_bwd(const BwdArgs& a, const BwdPlan& p, hipStream_t st);
+hipError_t launch_bwd_d128(const BwdArgs& a, const BwdPlan& p, hipStream_t st);
+hipError_t launch_bwd_d64(const BwdArgs& a, const BwdPlan& p, hipStream_t st);
+hipError_t launch_bwd_d32(const BwdArgs& a, const BwdPlan& p, hipStream_t st);  // D = 32 and 16
 // dX alone at D = 256 (dense 16-bit): the tuned dX programs
 hipError_t launch_dx256(const BwdArgs& a, hipStream_t st);
 // dW alone at D = 256 (dense 16-bit): n = H nE nS programs (nE E-tiles of 128

@@ -26,8 +26,8 @@ Differences from the reference, all deliberate:
   * Leaky ReLU's derivative at Z == 0 is autograd's 0.01 (flashmlp.py:33-34 uses 1.0);
   * io dtypes are fp16, bf16 and fp32 (fp32 in true fp32, where the reference's tl.dot would
     use its default reduced input precision); other dtypes raise TypeError;
-  * strided inputs are accepted: shapes with kernels of their own (fmlp_shape_dense: 16-bit io, D in
-    {64, 128, 256}) copy them to dense tensors, as the reference's reshape / contiguous does
+  * strided inputs are accepted: shapes with kernels of their own (fmlp_shape_dense: 16-bit
+    io) copy them to dense tensors, as the reference's reshape / contiguous does
     (flashmlp.py:453-459,508); every other shape reads the views in place (generic kernels),
     where the reference would copy them or fail its contiguity assertions.
 """
