@@ -25,7 +25,7 @@ CSRC = PKG / "csrc"
 BUILD = PKG / "_build"
 LIB = PKG / "libflashmlp.so"
 # fmlp_bwd.hip is compiled once per part (file:part): the kernels of one D each, and the rest
-SOURCES = ["fmlp_bwd.hip:64", "fmlp_bwd.hip:128", "fmlp_bwd.hip:0", "fmlp_bwd.hip:32", "fmlp_fwd.hip", "fmlp_gen.hip",
+SOURCES = ["fmlp_bwd.hip:64", "fmlp_bwd.hip:128", "fmlp_bwd.hip:0", "fmlp_bwd.hip:32", "fmlp_fwd.hip", "fmlp_f32.hip", "fmlp_gen.hip",
            "fmlp_scratch.hip", "fmlp_abi.cpp"]
 CEILING_SRC = "fmlp_ceiling.hip"
 CEILING_LIB = PKG / "libfmlp_ceiling.so"

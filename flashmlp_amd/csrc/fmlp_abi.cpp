@@ -112,11 +112,20 @@ bool fwd_tuned_shape(int64_t D, int64_t E, int io) {
 }
 
 // Dense, 16-byte aligned tensors of these shapes run on kernels of their own: those above, D = 16
-// and 32 (the same programs on 32-column tiles), and the same D with E % 8 != 0, whose W1 rows are first copied to 16-byte aligned rows at the start of
+// and 32 (the same programs on 32-column tiles), fp32 with D <= 128 (fmlp_f32.hip), and the same D with
+// E % 8 != 0 (fp32: E % 4 != 0), whose W1 rows are first copied to 16-byte aligned rows at the start of
 // the workspace (w1_pad_bytes; a call without room for them runs on the generic kernels, which were
 // 2.4 to 14 times slower at every E % 8 != 0 measured, from a 16-row forward to a 16-head training step).
-bool dense_shape(int64_t D, int io) {
+bool pitch_fits(int64_t D, int64_t E, int io);
+bool dense_shape(int64_t D, int64_t E, int io) {
+  if (!pitch_fits(D, E, io)) return false;
+  if (io == FMLP_DTYPE_F32) return D == 16 || D == 32 || D == 64 || D == 128;
   return (io == FMLP_DTYPE_F16 || io == FMLP_DTYPE_BF16) && (D == 16 || D == 32 || D == 64 || D == 128 || D == 256);
+}
+// a head's padded W1 within the 32-bit byte offsets of the kernels' loads
+bool pitch_fits(int64_t D, int64_t E, int io) {
+  const int es = io == FMLP_DTYPE_F32 ? 4 : 2;
+  return D * fmlp::w1_pitch(E, es) * es <= 0x7fffffffLL;
 }
 
 int check_shape(int64_t H, int64_t B, int64_t D, int64_t E, int dtype) {
@@ -248,7 +257,7 @@ FMLP_EXPORT int fmlp_shape_supported(int64_t H, int64_t B, int64_t D, int64_t E,
 
 FMLP_EXPORT int fmlp_shape_tuned(int64_t D, int64_t E, int dtype) { return tuned_shape(D, E, io_of(dtype)) ? 1 : 0; }
 
-FMLP_EXPORT int fmlp_shape_dense(int64_t D, int64_t E, int dtype) { return E > 0 && dense_shape(D, io_of(dtype)) ? 1 : 0; }
+FMLP_EXPORT int fmlp_shape_dense(int64_t D, int64_t E, int dtype) { return E > 0 && dense_shape(D, E, io_of(dtype)) ? 1 : 0; }
 
 namespace {
 
@@ -274,21 +283,22 @@ int fwd_impl(const void* x, const void* w1, const void* w2, void* o, int64_t H, 
   if (!rows) return ok();
   const bool dense = sx == nullptr || (is_dense3(sx, B, D) && is_dense3(sw1, D, E) && is_dense3(sw2, E, D));
   hipError_t e;
-  const size_t pad = fmlp::w1_pad_bytes(H, D, E);
-  if (dense && dense_shape(D, io) && (pad == 0 || (ws != nullptr && ws_bytes >= pad)) && aligned16(x) &&
+  const size_t pad = fmlp::w1_pad_bytes(H, D, E, (int)es);
+  if (dense && dense_shape(D, E, io) && (pad == 0 || (ws != nullptr && ws_bytes >= pad)) && aligned16(x) &&
       aligned16(w1) && aligned16(w2) && aligned16(o)) {
     int cus = 0;
     if ((st = num_cus_current(&cus))) return st;
     fmlp::FwdArgs a{x, w1, w2, o, H, B, D, E, io == FMLP_DTYPE_BF16, act, (dtype & FMLP_OUT_F32) != 0, cus,
-                    fmlp::w1_pitch(E)};
+                    fmlp::w1_pitch(E, (int)es)};
     a.ws = ws != nullptr ? (char*)ws + pad : nullptr;
     a.ws_bytes = ws != nullptr ? ws_bytes - pad : 0;
     e = hipSuccess;
     if (pad > 0) {
-      e = fmlp::launch_pad_w1(w1, ws, H, D, E, (hipStream_t)stream);
+      e = fmlp::launch_pad_w1(w1, ws, H, D, E, (int)es, (hipStream_t)stream);
       a.w1 = ws;
     }
-    if (e == hipSuccess) e = fmlp::launch_fwd(a, (hipStream_t)stream);
+    if (e == hipSuccess)
+      e = io == FMLP_DTYPE_F32 ? fmlp::launch_f32_fwd(a, (hipStream_t)stream) : fmlp::launch_fwd(a, (hipStream_t)stream);
   } else {
     fmlp::GenArgs g = gen_args(x, w1, w2, nullptr, o, nullptr, nullptr, nullptr, H, B, D, E, dtype, act);
     if (sx) {
@@ -314,10 +324,12 @@ FMLP_EXPORT int fmlp_fwd(const void* x, const void* w1, const void* w2, void* o,
 }
 
 FMLP_EXPORT size_t fmlp_fwd_workspace_bytes(int64_t H, int64_t B, int64_t D, int64_t E, int dtype) {
-  if (check_shape(H, B, D, E, dtype) != FMLP_OK || !dense_shape(D, io_of(dtype))) return 0;
+  if (check_shape(H, B, D, E, dtype) != FMLP_OK || !dense_shape(D, E, io_of(dtype))) return 0;
   int cus = 0;
   if (num_cus_current(&cus) != FMLP_OK) return 0;
-  return fmlp::w1_pad_bytes(H, D, E) + fmlp::fwd_plan(H, B, D, E, cus, (size_t)-1).ws_bytes;
+  const int io = io_of(dtype);
+  const size_t pad = fmlp::w1_pad_bytes(H, D, E, (int)elem_bytes(io));
+  return io == FMLP_DTYPE_F32 ? pad : pad + fmlp::fwd_plan(H, B, D, E, cus, (size_t)-1).ws_bytes;
 }
 
 FMLP_EXPORT int fmlp_fwd_ws(const void* x, const void* w1, const void* w2, void* o, int64_t H, int64_t B, int64_t D,
@@ -337,11 +349,11 @@ FMLP_EXPORT int fmlp_fwd_strided(const void* x, const void* w1, const void* w2, 
 FMLP_EXPORT size_t fmlp_bwd_workspace_bytes(int64_t H, int64_t B, int64_t D, int64_t E, int dtype) {
   if (check_shape(H, B, D, E, dtype) != FMLP_OK) return 0;
   const int io = io_of(dtype);
-  const bool own = dense_shape(D, io), no_dw = (dtype & FMLP_BWD_NO_DW) != 0;
+  const bool own = dense_shape(D, E, io), no_dw = (dtype & FMLP_BWD_NO_DW) != 0;
   if (no_dw && (dtype & FMLP_BWD_NO_DX)) return 0;  // nothing to compute
   // the generic dX programs alone use no workspace, the D = 256 ones only the padded W1
-  const size_t pad = own ? fmlp::w1_pad_bytes(H, D, E) : 0;
-  if (no_dw && !(own && D <= 128)) return pad;
+  const size_t pad = own ? fmlp::w1_pad_bytes(H, D, E, (int)elem_bytes(io)) : 0;
+  if (no_dw && !(own && D <= 128 && io != FMLP_DTYPE_F32)) return pad;
   int cus = 0;
   if (num_cus_current(&cus) != FMLP_OK) return 0;
   // the generic kernels (also views of a shape that is not fmlp_shape_tuned): the fp32 partials
@@ -349,6 +361,10 @@ FMLP_EXPORT size_t fmlp_bwd_workspace_bytes(int64_t H, int64_t B, int64_t D, int
   // may need more
   size_t n = tuned_shape(D, E, io) || no_dw ? 0 : fmlp::gen_plan(H, B, D, E, cus, (size_t)-1).ws_bytes;
   if (!own) return n;
+  if (io == FMLP_DTYPE_F32) {
+    const size_t w = pad + fmlp::plan_f32_bwd(H, B, D, E, cus, (size_t)-1).ws_bytes;
+    return w > n ? w : n;
+  }
   if (D == 256) {
     const size_t w = pad + fmlp::plan_dw256(H, B, E, (dtype & FMLP_DW_HILO) != 0, cus, (size_t)-1).ws_bytes;
     return w > n ? w : n;
@@ -396,7 +412,7 @@ FMLP_EXPORT int fmlp_bwd_plan(int64_t H, int64_t B, int64_t D, int64_t E, int dt
 
 FMLP_EXPORT int fmlp_bwd_stores_dz(int64_t H, int64_t B, int64_t D, int64_t E, int dtype, int act) {
   if (check_shape(H, B, D, E, dtype) != FMLP_OK || check_act(act) != FMLP_OK) return 0;
-  if (!dense_shape(D, io_of(dtype)) || D == 256) return 0;  // the other kernels recompute
+  if (!dense_shape(D, E, io_of(dtype)) || D == 256 || io_of(dtype) == FMLP_DTYPE_F32) return 0;  // the other kernels recompute
   int cus = 0;
   if (num_cus_current(&cus) != FMLP_OK) return 0;
   if (dtype & (FMLP_BWD_NO_DX | FMLP_BWD_NO_DW)) return 0;  // a partial backward stores no dZ
@@ -435,20 +451,34 @@ int bwd_impl(const void* x, const void* w1, const void* w2, const void* dout, vo
   hipError_t e = hipSuccess;
   // E % 8 != 0: W1's padded copy at the start of the workspace (or of the static scratch); without
   // room for it the call runs on the generic kernels
-  const size_t pad = dense && aligned && dense_shape(D, io) ? fmlp::w1_pad_bytes(H, D, E) : 0;
+  const size_t pad = dense && aligned && dense_shape(D, E, io) ? fmlp::w1_pad_bytes(H, D, E, (int)es) : 0;
   const size_t given = noalloc ? fmlp::kScratchBytes
                                : (workspace != nullptr && aligned16(workspace) ? workspace_bytes : 0);
-  const bool own = dense && aligned && dense_shape(D, io) && (pad == 0 || given >= pad);
+  const bool own = dense && aligned && dense_shape(D, E, io) && (pad == 0 || given >= pad);
   const void* w1p = w1;
   if (own && pad > 0) {
     void* dst = workspace;
     if (noalloc && (e = fmlp::scratch_current_device(&dst)) != hipSuccess)
       return fail(FMLP_ERR_HIP, "scratch lookup: %s", hipGetErrorString(e));
-    if ((e = fmlp::launch_pad_w1(w1, dst, H, D, E, (hipStream_t)stream)) != hipSuccess)
+    if ((e = fmlp::launch_pad_w1(w1, dst, H, D, E, (int)es, (hipStream_t)stream)) != hipSuccess)
       return fail(FMLP_ERR_HIP, "backward launch: %s", hipGetErrorString(e));
     w1p = dst;
   }
-  if (own && D <= 128) {
+  if (own && io == FMLP_DTYPE_F32) {
+    int cus = 0;
+    if ((st = num_cus_current(&cus))) return st;
+    // any workspace is accepted, as on the generic kernels: B is split as far as it holds the partials
+    const fmlp::F32Plan plan = fmlp::plan_f32_bwd(H, B, D, E, cus, want_dw ? given - pad : 0);
+    void* ws = nullptr;
+    if (plan.ws_bytes > 0) {
+      ws = pad > 0 ? (char*)w1p + pad : workspace;
+      if (noalloc && pad == 0 && (e = fmlp::scratch_current_device(&ws)) != hipSuccess)
+        return fail(FMLP_ERR_HIP, "scratch lookup: %s", hipGetErrorString(e));
+    }
+    fmlp::BwdArgs a{x, w1p, w2, dout, dx, dw1, dw2, H, B, D, E, false, act, ws, true, false, want_dx, want_dw,
+                    fmlp::w1_pitch(E, (int)es)};
+    e = fmlp::launch_f32_bwd(a, plan, (hipStream_t)stream);
+  } else if (own && D <= 128) {
     int cus = 0;
     if ((st = num_cus_current(&cus))) return st;
     // with a scratch limit the plan only considers B splits (and the stored-dZ form) whose
@@ -478,7 +508,7 @@ int bwd_impl(const void* x, const void* w1, const void* w2, const void* dout, vo
       }
     }
     fmlp::BwdArgs a{x, w1p, w2, dout, dx, dw1, dw2, H, B, D, E, io == FMLP_DTYPE_BF16, act, ws,
-                    (dtype & FMLP_OUT_F32) != 0, hilo, want_dx, want_dw, fmlp::w1_pitch(E)};
+                    (dtype & FMLP_OUT_F32) != 0, hilo, want_dx, want_dw, fmlp::w1_pitch(E, (int)es)};
     e = fmlp::launch_bwd(a, plan, (hipStream_t)stream);
   } else if (own) {
     // dense 16-bit D = 256: the D = 256 dX and dW programs; as on the generic kernels, the dW
@@ -499,7 +529,7 @@ int bwd_impl(const void* x, const void* w1, const void* w2, const void* dout, vo
       }
     }
     fmlp::BwdArgs a{x, w1p, w2, dout, dx, dw1, dw2, H, B, D, E, io == FMLP_DTYPE_BF16, act, ws,
-                    (dtype & FMLP_OUT_F32) != 0, (dtype & FMLP_DW_HILO) != 0, want_dx, want_dw, fmlp::w1_pitch(E)};
+                    (dtype & FMLP_OUT_F32) != 0, (dtype & FMLP_DW_HILO) != 0, want_dx, want_dw, fmlp::w1_pitch(E, (int)es)};
     if (want_dx) e = fmlp::launch_dx256(a, (hipStream_t)stream);
     if (e == hipSuccess && want_dw) e = fmlp::launch_dw256(a, wp, (hipStream_t)stream);
   } else {

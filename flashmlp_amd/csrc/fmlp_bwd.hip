@@ -805,28 +805,6 @@ static_assert(DW4_PF <= DW4_NSLOT - 1, "a slot is reloaded only after the barrie
 static_assert(DW4_PF >= 2 && 2 * DW4_SLOT == 256 * DW_ET * 2, "the W1c staging tile fills the ring's last two slots");
 static_assert(16 % (DW4_PD + 1) == 0, "each 16-step group starts at ring slot 0");
 
-// h = act(z) and the factor f with dZ = dH f (act_fb's arithmetic, split in two so that h can be
-// computed before dH is)
-template <int ACT>
-__device__ __forceinline__ void act_hf(float z, float& h, float& f) {
-  if constexpr (ACT == ACT_SILU) {
-    const float s = sigm(z);
-    h = z * s;
-    f = __builtin_fmaf(h, 1.0f - s, s);
-  } else if constexpr (ACT == ACT_LEAKY) {
-    const bool p = z > 0.f;
-    h = p ? z : 0.01f * z;
-    f = p ? 1.0f : 0.01f;
-  } else if constexpr (ACT == ACT_SIGMOID) {
-    const float s = sigm(z);
-    h = s;
-    f = s - s * s;
-  } else {
-    h = z;
-    f = 1.0f;
-  }
-}
-
 template <bool BF16, int ACT, bool HILO>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 dw256_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* __restrict__ W2,
@@ -1405,20 +1383,6 @@ dxg_kernel(const u16* __restrict__ dzt, const u16* __restrict__ W1, void* __rest
 // estimate makes is within 2.5 % of the best measured one for each of them.
 // ------------------------------------------------------------------------------------
 #if FMLP_BWD_PART == 0
-namespace {
-
-constexpr double kPlanFixedUs = 3.0;      // per program
-constexpr double kPlanRate = 4.5e6;       // MAC equivalents per microsecond per CU
-constexpr double kPlanValuMacs = 20.0;    // MAC equivalents per VALU instruction per element
-constexpr double kPlanHbmBytesPerUs = 5.0e6;
-constexpr double kPlanLaunchUs = 4.0;
-constexpr double kPlanDzBytesPerUs = 4.9e6;  // stored-dZ form: dZ bytes per time unit (store + reload)
-constexpr double kPlanDzFixedUs = 5.0;
-
-// VALU instructions per element of the activation plane (dX role: act'; dW role: act and act')
-double valu_dx(int act) { return act == ACT_SILU ? 8.5 : act == ACT_SIGMOID ? 6.5 : act == ACT_LEAKY ? 3.0 : 1.0; }
-double valu_dw(int act) { return act == ACT_SILU ? 9.0 : act == ACT_SIGMOID ? 7.0 : act == ACT_LEAKY ? 4.0 : 1.5; }
-
 // Completion time of n1 programs of t1 dealt round-robin over N CUs, followed by n2 programs of
 // t2 each started on the first CU to come free. The n2 programs take the n2 earliest of the
 // start slots low + k t2 (the CUs done with the first role at `low`) and high + k t2 (the
@@ -1443,6 +1407,20 @@ double list_makespan(long long n1, double t1, long long n2, double t2, long long
   }
   return std::max(end1, hi + t2);
 }
+
+namespace {
+
+constexpr double kPlanFixedUs = 3.0;      // per program
+constexpr double kPlanRate = 4.5e6;       // MAC equivalents per microsecond per CU
+constexpr double kPlanValuMacs = 20.0;    // MAC equivalents per VALU instruction per element
+constexpr double kPlanHbmBytesPerUs = 5.0e6;
+constexpr double kPlanLaunchUs = 4.0;
+constexpr double kPlanDzBytesPerUs = 4.9e6;  // stored-dZ form: dZ bytes per time unit (store + reload)
+constexpr double kPlanDzFixedUs = 5.0;
+
+// VALU instructions per element of the activation plane (dX role: act'; dW role: act and act')
+double valu_dx(int act) { return act == ACT_SILU ? 8.5 : act == ACT_SIGMOID ? 6.5 : act == ACT_LEAKY ? 3.0 : 1.0; }
+double valu_dw(int act) { return act == ACT_SILU ? 9.0 : act == ACT_SIGMOID ? 7.0 : act == ACT_LEAKY ? 4.0 : 1.5; }
 
 long long rows_for_split(long long B, long long ns) {
   long long rps = (B + ns - 1) / ns;
@@ -1481,7 +1459,7 @@ BwdPlan make_plan(int64_t H, int64_t B, int64_t D, int64_t E, int act, bool hilo
   static const int et_env = env_int("FMLP_BWD_ET", 0);
   auto nE_for = [&](long long et) { return (E + et - 1) / et; };
   const long long base = H * nE_for(DW_ET);  // the stored-dZ form's dW programs (128 columns)
-  auto ws_for = [&](long long ns) { return ns > 1 ? (size_t)2 * ns * H * w1_pitch(E) * D * sizeof(float) : (size_t)0; };
+  auto ws_for = [&](long long ns) { return ns > 1 ? (size_t)2 * ns * H * w1_pitch(E, 2) * D * sizeof(float) : (size_t)0; };
   // dX programs of 256 rows, or at D = 64 of 128 rows with E in two parts (half the time each)
   auto n_dx_for = [&](int des) { return H * ((B + DX2_ROWS / des - 1) / (DX2_ROWS / des)); };
   auto tx_for = [&](int des) {
@@ -1696,7 +1674,7 @@ Dw256Plan plan_dw256(int64_t H, int64_t B, int64_t E, bool hilo, int num_cus, si
   double best = 1e300;
   for (long long ns = 1; ns <= max_ns; ns *= 2) {
     const long long rps = rows_for_split(B, ns), eff = (B + rps - 1) / rps;
-    const size_t ws = eff > 1 ? (size_t)2 * eff * H * w1_pitch(E) * 256 * sizeof(float) : 0;
+    const size_t ws = eff > 1 ? (size_t)2 * eff * H * w1_pitch(E, 2) * 256 * sizeof(float) : 0;
     if (ws > max_ws) continue;
     const long long progs = H * p.nE * eff, rounds = (progs + N - 1) / N;
     double cost = (double)rounds * (kFixedUs + (double)(rps / DW_BT) * t_sub);
@@ -1915,6 +1893,8 @@ static hipError_t launch_dw256_a(const BwdArgs& a, const Dw256Plan& p, hipStream
     default: return launch_dw256_t<BF16, ACT_NONE, HILO>(a, p, st);
   }
 }
+
+hipError_t launch_dw_reduce_f32(const BwdArgs& a, int nS, hipStream_t st) { return launch_dw_reduce<true>(a, nS, st); }
 
 hipError_t launch_dw256(const BwdArgs& a, const Dw256Plan& p, hipStream_t st) {
   if (a.bf16) return a.dw_hilo ? launch_dw256_a<true, true>(a, p, st) : launch_dw256_a<true, false>(a, p, st);

@@ -135,6 +135,36 @@ __device__ __forceinline__ void act_fb(float z, float dh, float& h, float& dz) {
   }
 }
 
+// h = act(z) and the factor f with dZ = dH f (act_fb's arithmetic, split in two so that h can be
+// computed before dH is)
+template <int ACT>
+__device__ __forceinline__ void act_hf(float z, float& h, float& f) {
+  if constexpr (ACT == ACT_SILU) {
+    const float s = sigm(z);
+    h = z * s;
+    f = __builtin_fmaf(h, 1.0f - s, s);
+  } else if constexpr (ACT == ACT_LEAKY) {
+    const bool p = z > 0.f;
+    h = p ? z : 0.01f * z;
+    f = p ? 1.0f : 0.01f;
+  } else if constexpr (ACT == ACT_SIGMOID) {
+    const float s = sigm(z);
+    h = s;
+    f = s - s * s;
+  } else {
+    h = z;
+    f = 1.0f;
+  }
+}
+
+// act'(z) alone
+template <int ACT>
+__device__ __forceinline__ float act_d(float z) {
+  float h, f;
+  act_hf<ACT>(z, h, f);
+  return f;
+}
+
 // dz only (dX programs never need h)
 template <int ACT>
 __device__ __forceinline__ float act_b(float z, float dh) {

@@ -427,35 +427,40 @@ fwd_reduce_kernel(const float* __restrict__ ws, void* __restrict__ O, int B, int
   }
 }
 
-// W1 rows of E 16-bit elements copied to rows of ldw (E rounded up to 8), zeros behind the last:
-// where E is no multiple of 8 only every eighth row starts 16-byte aligned, and the kernels load
+// W1 rows of E elements copied to rows of whole 16-byte vectors, zeros behind the last: where E is
+// no multiple of 8 (fp32: 4) most rows do not start 16-byte aligned, and the kernels load
 // 16-byte pieces of rows. One 16-byte piece per thread, read element by element (the weights are
 // small next to the rows' work: about 4 us with the launch at H=16 D=128 E=683). The generic
 // kernels, which took these E before, read every operand element from the L1 / L2 per MFMA:
 // H=16 B=4095 D=128 E=683 bf16 forward + backward 1942 -> 140 us (41 -> 574 TFLOP/s at 14u).
+template <typename T>
 __global__ void __launch_bounds__(256)
-pad_w1_kernel(const u16* __restrict__ src, u16* __restrict__ dst, long long pieces, int E, int ppr) {
+pad_w1_kernel(const T* __restrict__ src, T* __restrict__ dst, long long pieces, int E, int ppr) {
+  constexpr int N = 16 / sizeof(T);
   const long long p = (long long)blockIdx.x * 256 + threadIdx.x;
   if (p >= pieces) return;
   const long long row = p / ppr;
-  const int c = (int)(p - row * ppr) * 8;
-  const u16* s = src + row * E + c;
-  u32x4 v;
+  const int c = (int)(p - row * ppr) * N;
+  const T* s = src + row * E + c;
+  T v[N];
 #pragma unroll
-  for (int w = 0; w < 4; ++w) {
-    const unsigned lo = c + 2 * w < E ? s[2 * w] : 0u, hi = c + 2 * w + 1 < E ? s[2 * w + 1] : 0u;
-    v[w] = lo | (hi << 16);
-  }
-  *(u32x4*)(dst + p * 8) = v;
+  for (int i = 0; i < N; ++i) v[i] = c + i < E ? s[i] : (T)0;
+  u32x4 w;
+  __builtin_memcpy(&w, v, 16);
+  *(u32x4*)(dst + p * N) = w;
 }
 
-hipError_t launch_pad_w1(const void* w1, void* dst, int64_t H, int64_t D, int64_t E, hipStream_t st) {
-  const int ppr = (int)(w1_pitch(E) / 8);
+hipError_t launch_pad_w1(const void* w1, void* dst, int64_t H, int64_t D, int64_t E, int es, hipStream_t st) {
+  const int ppr = (int)(w1_pitch(E, es) * es / 16);
   const long long pieces = (long long)H * D * ppr, blocks = (pieces + 255) / 256;
   if (blocks <= 0) return hipSuccess;
   if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(pad_w1_kernel, dim3((unsigned)blocks), dim3(256), 0, st, (const u16*)w1, (u16*)dst, pieces,
-                     (int)E, ppr);
+  if (es == 4)
+    hipLaunchKernelGGL(pad_w1_kernel<unsigned>, dim3((unsigned)blocks), dim3(256), 0, st, (const unsigned*)w1,
+                       (unsigned*)dst, pieces, (int)E, ppr);
+  else
+    hipLaunchKernelGGL(pad_w1_kernel<u16>, dim3((unsigned)blocks), dim3(256), 0, st, (const u16*)w1, (u16*)dst, pieces,
+                       (int)E, ppr);
   return hipGetLastError();
 }
 

@@ -16,14 +16,14 @@ int env_int(const char* name, int dflt);
 // skip the runtime call.
 hipError_t set_lds_once(const void* kernel, int bytes, std::atomic<unsigned long long>& done);
 
-// Row pitch the tuned kernels read W1 with: E rounded up to whole 16-byte vectors of 16-bit
-// elements. Where E is no multiple of 8 the caller's W1 rows are copied to this pitch first
+// Row pitch the kernels read W1 with (elements of es bytes): E rounded up to whole 16-byte
+// vectors. Where E is no such multiple the caller's W1 rows are copied to this pitch first
 // (launch_pad_w1), into w1_pad_bytes of workspace (a multiple of 256 bytes).
-inline int64_t w1_pitch(int64_t E) { return (E + 7) / 8 * 8; }
-inline size_t w1_pad_bytes(int64_t H, int64_t D, int64_t E) {
-  return E % 8 == 0 ? 0 : ((size_t)H * D * w1_pitch(E) * 2 + 255) / 256 * 256;
+inline int64_t w1_pitch(int64_t E, int es) { return (E + 16 / es - 1) / (16 / es) * (16 / es); }
+inline size_t w1_pad_bytes(int64_t H, int64_t D, int64_t E, int es) {
+  return w1_pitch(E, es) == E ? 0 : ((size_t)H * D * w1_pitch(E, es) * es + 255) / 256 * 256;
 }
-hipError_t launch_pad_w1(const void* w1, void* dst, int64_t H, int64_t D, int64_t E, hipStream_t st);
+hipError_t launch_pad_w1(const void* w1, void* dst, int64_t H, int64_t D, int64_t E, int es, hipStream_t st);
 
 struct FwdArgs {
   const void* x;
@@ -35,7 +35,7 @@ struct FwdArgs {
   int act;
   bool out_f32;  // outputs as fp32 (FMLP_OUT_F32)
   int num_cus;   // compute units of the current device
-  int64_t ldw;   // row pitch of w1 (w1_pitch(E))
+  int64_t ldw;   // row pitch of w1 (w1_pitch)
   void* ws = nullptr;   // workspace for split tiles' partials (fwd_plan), or none
   size_t ws_bytes = 0;
 };
@@ -98,7 +98,7 @@ struct BwdArgs {
   bool dw_hilo;  // dW products with hi/lo terms of h and dZ (FMLP_DW_HILO)
   bool want_dx = true;  // false: FMLP_BWD_NO_DX (only the dW programs run)
   bool want_dw = true;  // false: FMLP_BWD_NO_DW (only the dX programs run)
-  int64_t ldw = 0;      // row pitch of w1, and of the fp32 dW partials (w1_pitch(E))
+  int64_t ldw = 0;      // row pitch of w1, and of the fp32 dW partials (w1_pitch)
 };
 
 // io element types of the generic kernels
@@ -176,6 +176,26 @@ struct Dw256Plan {
 };
 Dw256Plan plan_dw256(int64_t H, int64_t B, int64_t E, bool hilo, int num_cus, size_t max_ws);
 hipError_t launch_dw256(const BwdArgs& a, const Dw256Plan& p, hipStream_t st);
+
+// Completion time of n1 programs of t1 dealt round-robin over N slots, followed by n2 programs of
+// t2 each started on the first slot to come free (fmlp_bwd.hip).
+double list_makespan(long long n1, double t1, long long n2, double t2, long long N);
+
+// fp32 io (fmlp_f32.hip): dense tensors, D in {16, 32, 64, 128}. The backward's plan: ep E parts of
+// the dX programs (the same whatever the workspace), dW programs of 32 cg columns with B in nS
+// ranges of rows_per_split rows, whose fp32 partials take ws_bytes when nS > 1 (a split needing
+// more than max_ws bytes is not taken; nS = 1 needs none).
+struct F32Plan {
+  int ep, dx_tiles_per_head, cg, nE, nS, rows_per_split;
+  bool dx_first;
+  long long n_dx, n_dw;
+  size_t ws_bytes;
+};
+F32Plan plan_f32_bwd(int64_t H, int64_t B, int64_t D, int64_t E, int num_cus, size_t max_ws);
+hipError_t launch_f32_fwd(const FwdArgs& a, hipStream_t st);
+hipError_t launch_f32_bwd(const BwdArgs& a, const F32Plan& p, hipStream_t st);
+// sum of the fp32 programs' dW partials (fmlp_bwd.hip; nothing when nS <= 1)
+hipError_t launch_dw_reduce_f32(const BwdArgs& a, int nS, hipStream_t st);
 
 // The library's static device scratch (fmlp_bwd_noalloc): its device address on the current
 // device, looked up once per device, and its size in bytes.

@@ -1,6 +1,6 @@
 // _fmlp_fast: the per-call fast path of flashmlp_fwd / flashmlp_bwd (flashmlp_amd/flashmlp.py).
 //
-// A CPython module (METH_FASTCALL) over the C ABI of libflashmlp.so for the common case: 16-bit
+// A CPython module (METH_FASTCALL) over the C ABI of libflashmlp.so for the common case:
 // inputs on one GPU, dense and 16-byte aligned, a shape with kernels of its own. It allocates the
 // outputs and the workspace with ATen on the inputs' device, launches on torch's current HIP
 // stream of that device and returns the C ABI status with the outputs; for any other input it
@@ -26,6 +26,7 @@ int io_code(const at::Tensor& t) {
   switch (t.scalar_type()) {
     case at::kHalf: return FMLP_DTYPE_F16;
     case at::kBFloat16: return FMLP_DTYPE_BF16;
+    case at::kFloat: return FMLP_DTYPE_F32;
     default: return -1;
   }
 }
@@ -34,7 +35,7 @@ bool dense16(const at::Tensor& t) {
   return t.dim() == 3 && t.is_contiguous() && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15u) == 0;
 }
 
-// the tensors those kernels take as they are: 16-bit, one GPU, dense, aligned; sets the io
+// the tensors those kernels take as they are: one GPU, dense, aligned; sets the io
 // dtype code
 bool eligible(PyObject* const* args, int n, const at::Tensor** ts, int* code) {
   for (int i = 0; i < n; ++i) {

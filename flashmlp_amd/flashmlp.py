@@ -27,7 +27,7 @@ Differences from the reference, all deliberate:
   * io dtypes are fp16, bf16 and fp32 (fp32 in true fp32, where the reference's tl.dot would
     use its default reduced input precision); other dtypes raise TypeError;
   * strided inputs are accepted: shapes with kernels of their own (fmlp_shape_dense: 16-bit
-    io) copy them to dense tensors, as the reference's reshape / contiguous does
+    io, and fp32 with D <= 128) copy them to dense tensors, as the reference's reshape / contiguous does
     (flashmlp.py:453-459,508); every other shape reads the views in place (generic kernels),
     where the reference would copy them or fail its contiguity assertions.
 """

@@ -12,8 +12,7 @@
  * x's, flashmlp.py:87). All pointers are device pointers on the current HIP device, aligned
  * to their element size. Two kernel sets sit behind the entry points: the tuned gfx950
  * kernels for 16-bit io, D in {64, 128}, E % 8 == 0 on dense 16-byte aligned tensors
- * (fmlp_shape_tuned; with D = 16, 32 and 256 kernels of their own for the same io, E and layout, and E
- * that is no multiple of 8 through a padded copy of W1 in the workspace: fmlp_shape_dense), and
+ * (fmlp_shape_tuned) with their like for other D, fp32 io and other E (fmlp_shape_dense), and
  * generic kernels for every other supported shape, dtype and layout.
  * The library never allocates: the caller passes every buffer, including the backward
  * workspace.
@@ -127,7 +126,8 @@ int fmlp_shape_supported(int64_t H, int64_t B, int64_t D, int64_t E, int dtype);
 int fmlp_shape_tuned(int64_t D, int64_t E, int dtype);
 
 /* 1 when dense, 16-byte aligned tensors of these shapes run on kernels other than the generic ones:
- * fmlp_shape_tuned, 16-bit D = 16, 32 and 256, and the same D with E % 8 != 0 given the queried workspace (at its
+ * fmlp_shape_tuned, 16-bit D = 16, 32 and 256, fp32 with D <= 128, and the same D with E % 8 != 0
+ * (fp32: E % 4 != 0) given the queried workspace (at its
  * start W1's rows are copied to rows of E rounded up to 8; with less workspace than that copy
  * takes, as in fmlp_fwd, the call runs on the generic kernels, and any workspace is accepted, as
  * there). No counterpart in the reference. */
