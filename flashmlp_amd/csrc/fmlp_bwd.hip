@@ -169,7 +169,8 @@ __host__ __device__ constexpr int dx2_rows() { return DX2_ROWS / DES; }
 template <bool BF16, int D, int ACT, int DES = 1, int NW = DX2_NW, int DG = D>
 __device__ __forceinline__ void dx2_body(const u16* __restrict__ X, const u16* __restrict__ W1,
                                          const u16* __restrict__ W2, const u16* __restrict__ dO,
-                                         void* __restrict__ dX, int B, int E, int ldw, int tiles_per_head, int outf32,
+                                         void* __restrict__ dX, int B, int E, int ldw, long long sx, long long sdo,
+                                         int tiles_per_head, int outf32,
                                          int t, int cb, int ce, float* __restrict__ pws) {
   static_assert(DES == 1 || (DES == 2 && D <= 64), "E split");
   static_assert(DG == D || (DG == 16 && D == 32), "columns in memory");
@@ -201,8 +202,8 @@ __device__ __forceinline__ void dx2_body(const u16* __restrict__ X, const u16* _
   // (NW = 4) every wave runs the MFMA-first order
   const bool late = NW == 8 && wave >= 4;
 
-  const u16* Xh = X + (size_t)h * B * DG;
-  const u16* dOh = dO + (size_t)h * B * DG;
+  const u16* Xh = X + (size_t)h * sx;
+  const u16* dOh = dO + (size_t)h * sdo;
   const u16* W1h = W1 + (size_t)h * DG * ldw;
   const u16* W2h = W2 + (size_t)h * E * DG;
   const int b_wave = bt * ROWS + wp * 32;
@@ -456,7 +457,8 @@ template <bool BF16, int D, int ACT, bool HILO, bool DZ = false, int ET = DW_ET,
 __device__ __forceinline__ void dw2_body(const u16* __restrict__ X, const u16* __restrict__ W1,
                                          const u16* __restrict__ W2, const u16* __restrict__ dO,
                                          void* __restrict__ dW1, void* __restrict__ dW2, float* __restrict__ ws,
-                                         int H, int B, int E, int ldw, int nE, int nS, int rows_per_split,
+                                         int H, int B, int E, int ldw, long long sx, long long sdo,
+                                         int nE, int nS, int rows_per_split,
                                          int outf32, int t, u16* __restrict__ dzt = nullptr, int Bp = 0) {
   static_assert(ET == DW_ET || (ET == 64 && D == 64 && !DZ), "E-tile width");
   static_assert(DG == D || (DG == 16 && D == 32), "columns in memory");
@@ -490,8 +492,8 @@ __device__ __forceinline__ void dw2_body(const u16* __restrict__ X, const u16* _
   const int nsub = (b_hi - b_lo + DW_BT - 1) / DW_BT;
   const int npair = (nsub + RS - 1) / RS;
 
-  const u16* Xh = X + (size_t)h * B * DG;
-  const u16* dOh = dO + (size_t)h * B * DG;
+  const u16* Xh = X + (size_t)h * sx;
+  const u16* dOh = dO + (size_t)h * sdo;
   const u16* W1h = W1 + (size_t)h * DG * ldw;
   const u16* W2h = W2 + (size_t)h * E * DG;
 
@@ -761,8 +763,10 @@ __device__ __forceinline__ void dw2_body(const u16* __restrict__ X, const u16* _
 template <bool BF16, int D, int ACT, int DES, int DG = D>
 __global__ void __launch_bounds__(DX2_NT) __attribute__((amdgpu_waves_per_eu(bwd_wpe(D), bwd_wpe(D))))
 dx2_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* __restrict__ W2,
-           const u16* __restrict__ dO, void* __restrict__ dX, int B, int E, int ldw, int tiles_per_head, int outf32) {
-  dx2_body<BF16, D, ACT, DES, DX2_NW, DG>(X, W1, W2, dO, dX, B, E, ldw, tiles_per_head, outf32, xcd_remap(blockIdx.x, gridDim.x), 0,
+           const u16* __restrict__ dO, void* __restrict__ dX, int B, int E, int ldw, long long sx, long long sdo,
+           int tiles_per_head, int outf32) {
+  dx2_body<BF16, D, ACT, DES, DX2_NW, DG>(X, W1, W2, dO, dX, B, E, ldw, sx, sdo,
+                                          tiles_per_head, outf32, xcd_remap(blockIdx.x, gridDim.x), 0,
                               (E + 31) >> 5, nullptr);
 }
 
@@ -772,8 +776,10 @@ dx2_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* __r
 template <bool BF16, int ACT>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 dx256_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* __restrict__ W2,
-             const u16* __restrict__ dO, void* __restrict__ dX, int B, int E, int ldw, int tiles_per_head, int outf32) {
-  dx2_body<BF16, 256, ACT, 1, 4>(X, W1, W2, dO, dX, B, E, ldw, tiles_per_head, outf32, xcd_remap(blockIdx.x, gridDim.x),
+             const u16* __restrict__ dO, void* __restrict__ dX, int B, int E, int ldw, long long sx, long long sdo,
+             int tiles_per_head, int outf32) {
+  dx2_body<BF16, 256, ACT, 1, 4>(X, W1, W2, dO, dX, B, E, ldw, sx, sdo,
+                                 tiles_per_head, outf32, xcd_remap(blockIdx.x, gridDim.x),
                                  0, (E + 31) >> 5, nullptr);
 }
 
@@ -809,7 +815,8 @@ template <bool BF16, int ACT, bool HILO>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 dw256_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* __restrict__ W2,
              const u16* __restrict__ dO, void* __restrict__ dW1, void* __restrict__ dW2, float* __restrict__ ws,
-             int H, int B, int E, int ldw, int nE, int nS, int rows_per_split, int outf32) {
+             int H, int B, int E, int ldw, long long sx, long long sdo,
+             int nE, int nS, int rows_per_split, int outf32) {
   constexpr int D = 256, KS = D / 16, NTN = D / 32;
   constexpr int STG = 2 * DW4_SLOT;  // W1c staging tile: [256 d][128 e], 256-byte rows
   constexpr int PD = DW4_PD;
@@ -824,8 +831,8 @@ dw256_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* _
   const int b_hi = min(B, b_lo + rows_per_split);
   const int nsub = b_hi > b_lo ? (b_hi - b_lo + DW_BT - 1) / DW_BT : 0;
 
-  const u16* Xh = X + (size_t)h * B * D;
-  const u16* dOh = dO + (size_t)h * B * D;
+  const u16* Xh = X + (size_t)h * sx;
+  const u16* dOh = dO + (size_t)h * sdo;
   const u16* W1h = W1 + (size_t)h * D * ldw;
   const u16* W2h = W2 + (size_t)h * E * D;
 
@@ -1012,9 +1019,11 @@ template <bool BF16, int D, int ACT, bool HILO, bool DZ, int ET = DW_ET, int DG 
 __global__ void __launch_bounds__(DW2_NT) __attribute__((amdgpu_waves_per_eu(bwd_wpe(D), bwd_wpe(D))))
 dw2_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* __restrict__ W2,
            const u16* __restrict__ dO, void* __restrict__ dW1, void* __restrict__ dW2, float* __restrict__ ws,
-           int H, int B, int E, int ldw, int nE, int nS, int rows_per_split, int outf32, u16* __restrict__ dzt,
+           int H, int B, int E, int ldw, long long sx, long long sdo,
+           int nE, int nS, int rows_per_split, int outf32, u16* __restrict__ dzt,
            int Bp) {
-  dw2_body<BF16, D, ACT, HILO, DZ, ET, DG>(X, W1, W2, dO, dW1, dW2, ws, H, B, E, ldw, nE, nS, rows_per_split, outf32,
+  dw2_body<BF16, D, ACT, HILO, DZ, ET, DG>(X, W1, W2, dO, dW1, dW2, ws, H, B, E, ldw, sx, sdo,
+                                           nE, nS, rows_per_split, outf32,
                                    xcd_remap(blockIdx.x, gridDim.x), dzt, Bp);
 }
 
@@ -1028,7 +1037,8 @@ template <bool BF16, int D, int ACT, bool HILO, int DES, int ET = DW_ET, int DG 
 __global__ void __launch_bounds__(DW2_NT) __attribute__((amdgpu_waves_per_eu(bwd_wpe(D), bwd_wpe(D))))
 bwd_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* __restrict__ W2,
            const u16* __restrict__ dO, void* __restrict__ dX, void* __restrict__ dW1, void* __restrict__ dW2,
-           float* __restrict__ ws, int H, int B, int E, int ldw, int nE, int nS, int rows_per_split, int n_dw,
+           float* __restrict__ ws, int H, int B, int E, int ldw, long long sx, long long sdo,
+           int nE, int nS, int rows_per_split, int n_dw,
            int dx_tiles_per_head, int dx_first, int outf32, int n_dxs, int dxs_xs, int dxs_nct,
            float* __restrict__ dxs_ws) {
   // programs: n_dw dW programs and n_dx whole-tile dX programs (in the plan's order), then
@@ -1038,19 +1048,21 @@ bwd_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* __r
   const int T = dx_tiles_per_head, nch = (E + 31) >> 5;
   if (b >= n_rest) {
     const int u = b - n_rest, hh = u / dxs_xs, cb = (u - hh * dxs_xs) * dxs_nct;
-    dx2_body<BF16, D, ACT, DES, DX2_NW, DG>(X, W1, W2, dO, dX, B, E, ldw, T, outf32, hh * T + T - 1, cb, min(nch, cb + dxs_nct),
+    dx2_body<BF16, D, ACT, DES, DX2_NW, DG>(X, W1, W2, dO, dX, B, E, ldw, sx, sdo,
+                                            T, outf32, hh * T + T - 1, cb, min(nch, cb + dxs_nct),
                                 dxs_ws + (size_t)u * dx2_rows<D, DES>() * DG);
     return;
   }
   const int bw = dx_first ? b - n_dx : b;  // index among the dW programs (< 0 or >= n_dw: a dX program)
   if (bw >= 0 && bw < n_dw) {
-    dw2_body<BF16, D, ACT, HILO, false, ET, DG>(X, W1, W2, dO, dW1, dW2, ws, H, B, E, ldw, nE, nS, rows_per_split, outf32,
+    dw2_body<BF16, D, ACT, HILO, false, ET, DG>(X, W1, W2, dO, dW1, dW2, ws, H, B, E, ldw, sx, sdo,
+                                                nE, nS, rows_per_split, outf32,
                                             xcd_remap(bw, n_dw));
   } else {
     const int bx = dx_first ? b : b - n_dw;
     const int m = xcd_remap(bx, n_dx);
     const int t = n_dxs > 0 ? (m / (T - 1)) * T + m % (T - 1) : m;
-    dx2_body<BF16, D, ACT, DES, DX2_NW, DG>(X, W1, W2, dO, dX, B, E, ldw, T, outf32, t, 0, nch, nullptr);
+    dx2_body<BF16, D, ACT, DES, DX2_NW, DG>(X, W1, W2, dO, dX, B, E, ldw, sx, sdo, T, outf32, t, 0, nch, nullptr);
   }
 }
 
@@ -1736,7 +1748,8 @@ static hipError_t launch_bwd_t(const BwdArgs& a, const BwdPlan& p, hipStream_t s
       if (r != hipSuccess) return r;
       hipLaunchKernelGGL(k, dim3((unsigned)p.n_dw), dim3(DW2_NT), lds, st, (const u16*)a.x, (const u16*)a.w1,
                          (const u16*)a.w2, (const u16*)a.dout, a.dw1, a.dw2, (float*)a.ws, (int)a.H, (int)a.B,
-                         (int)a.E, (int)a.ldw, p.nE, p.nS, p.rows_per_split, a.out_f32 ? 1 : 0, dzt, p.Bp);
+                         (int)a.E, (int)a.ldw, (long long)a.sx, (long long)a.sdo,
+                         p.nE, p.nS, p.rows_per_split, a.out_f32 ? 1 : 0, dzt, p.Bp);
       return hipGetLastError();
     };
     e = a.dw_hilo ? launch_w(dw2_kernel<BF16, D, ACT, true, true>) : launch_w(dw2_kernel<BF16, D, ACT, false, true>);
@@ -1774,7 +1787,8 @@ static hipError_t launch_bwd_t(const BwdArgs& a, const BwdPlan& p, hipStream_t s
       if (r != hipSuccess) return r;
       hipLaunchKernelGGL(k, dim3((unsigned)(n_dw + p.n_dx + p.n_dxs)), dim3(DW2_NT), lds, st, (const u16*)a.x,
                          (const u16*)a.w1, (const u16*)a.w2, (const u16*)a.dout, a.dx, a.dw1, a.dw2, (float*)a.ws,
-                         (int)a.H, (int)a.B, (int)a.E, (int)a.ldw, p.nE, p.nS, p.rows_per_split, (int)n_dw,
+                         (int)a.H, (int)a.B, (int)a.E, (int)a.ldw, (long long)a.sx, (long long)a.sdo,
+                         p.nE, p.nS, p.rows_per_split, (int)n_dw,
                          p.dx_tiles_per_head, p.dx_first ? 1 : 0, a.out_f32 ? 1 : 0, (int)p.n_dxs, p.dxs_xs,
                          p.dxs_nct, dxs_ws);
       return hipGetLastError();
@@ -1795,7 +1809,8 @@ static hipError_t launch_bwd_t(const BwdArgs& a, const BwdPlan& p, hipStream_t s
       if (r != hipSuccess) return r;
       hipLaunchKernelGGL(k, dim3((unsigned)p.n_dw), dim3(DW2_NT), lds, st, (const u16*)a.x, (const u16*)a.w1,
                          (const u16*)a.w2, (const u16*)a.dout, a.dw1, a.dw2, (float*)a.ws, (int)a.H,
-                         (int)a.B, (int)a.E, (int)a.ldw, p.nE, p.nS, p.rows_per_split, a.out_f32 ? 1 : 0, (u16*)nullptr, 0);
+                         (int)a.B, (int)a.E, (int)a.ldw, (long long)a.sx, (long long)a.sdo,
+                         p.nE, p.nS, p.rows_per_split, a.out_f32 ? 1 : 0, (u16*)nullptr, 0);
       return hipGetLastError();
     };
     e = a.dw_hilo ? launch_w(dw2_kernel<BF16, D, ACT, true, false, ET, DG>)
@@ -1811,7 +1826,8 @@ static hipError_t launch_bwd_t(const BwdArgs& a, const BwdPlan& p, hipStream_t s
     e = set_lds_once((const void*)k, (int)lds_x, lds_set);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(k, dim3((unsigned)n_dx_all), dim3(DX2_NT), lds_x, st, (const u16*)a.x, (const u16*)a.w1,
-                       (const u16*)a.w2, (const u16*)a.dout, a.dx, (int)a.B, (int)a.E, (int)a.ldw, p.dx_tiles_per_head,
+                       (const u16*)a.w2, (const u16*)a.dout, a.dx, (int)a.B, (int)a.E, (int)a.ldw,
+                       (long long)a.sx, (long long)a.sdo, p.dx_tiles_per_head,
                        a.out_f32 ? 1 : 0);
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
@@ -1850,7 +1866,8 @@ static hipError_t launch_dx256_t(const BwdArgs& a, hipStream_t st) {
   hipError_t e = set_lds_once((const void*)k, (int)lds, lds_set);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(256), lds, st, (const u16*)a.x, (const u16*)a.w1, (const u16*)a.w2,
-                     (const u16*)a.dout, a.dx, (int)a.B, (int)a.E, (int)a.ldw, (int)tph, a.out_f32 ? 1 : 0);
+                     (const u16*)a.dout, a.dx, (int)a.B, (int)a.E, (int)a.ldw, (long long)a.sx, (long long)a.sdo,
+                     (int)tph, a.out_f32 ? 1 : 0);
   return hipGetLastError();
 }
 
@@ -1878,7 +1895,8 @@ static hipError_t launch_dw256_t(const BwdArgs& a, const Dw256Plan& p, hipStream
   hipError_t e = set_lds_once((const void*)k, (int)lds, lds_set);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(k, dim3((unsigned)p.n), dim3(256), lds, st, (const u16*)a.x, (const u16*)a.w1, (const u16*)a.w2,
-                     (const u16*)a.dout, a.dw1, a.dw2, (float*)a.ws, (int)a.H, (int)a.B, (int)a.E, (int)a.ldw, p.nE, p.nS,
+                     (const u16*)a.dout, a.dw1, a.dw2, (float*)a.ws, (int)a.H, (int)a.B, (int)a.E, (int)a.ldw,
+                     (long long)a.sx, (long long)a.sdo, p.nE, p.nS,
                      p.rows_per_split, a.out_f32 ? 1 : 0);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   return launch_dw_reduce<BF16>(a, p.nS, st);

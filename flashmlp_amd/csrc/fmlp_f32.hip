@@ -220,7 +220,8 @@ __device__ __forceinline__ void dw_store(const f32x16 (&a1)[D / 32], const f32x1
 template <int D, int DG, int ACT, bool BWD>
 __device__ __forceinline__ void rows_body(const float* __restrict__ X, const float* __restrict__ W1,
                                           const float* __restrict__ W2, const float* __restrict__ dO,
-                                          float* __restrict__ out, int B, int E, int ldw, int tiles_per_head, int ep,
+                                          float* __restrict__ out, int B, int E, int ldw, long long sx, long long sdo,
+                                          int tiles_per_head, int ep,
                                           int t) {
   constexpr int NW = f32_nw(D), NTN = D / 32, KJ = DG / 8;
   constexpr int SLOT = 256 * D, W2OFF = 128 * D;
@@ -228,7 +229,7 @@ __device__ __forceinline__ void rows_body(const float* __restrict__ X, const flo
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int rt = NW / ep, part = wave / rt, rtile = wave - part * rt;
   const int h = t / tiles_per_head, bt = t - h * tiles_per_head;
-  const float* Xh = X + (size_t)h * B * DG;
+  const float* Xh = X + (size_t)h * sx;
   const float* W1h = W1 + (size_t)h * DG * ldw;
   const float* W2h = W2 + (size_t)h * E * DG;
   const int b_wave = (bt * rt + rtile) * 32;
@@ -248,7 +249,7 @@ __device__ __forceinline__ void rows_body(const float* __restrict__ X, const flo
   for (int j = 0; j < KJ; ++j) {
     const size_t o = (size_t)(b_wave + l32) * DG + 8 * j + 4 * g;
     xr[j] = ok ? *(const f32x4*)(Xh + o) : f32x4{0.f, 0.f, 0.f, 0.f};
-    if constexpr (BWD) dr[j] = ok ? *(const f32x4*)(dO + (size_t)h * B * DG + o) : f32x4{0.f, 0.f, 0.f, 0.f};
+    if constexpr (BWD) dr[j] = ok ? *(const f32x4*)(dO + (size_t)h * sdo + o) : f32x4{0.f, 0.f, 0.f, 0.f};
   }
   f32x16 acc[NTN];
 #pragma unroll
@@ -328,7 +329,8 @@ template <int D, int DG, int ACT>
 __device__ __forceinline__ void dw_body(const float* __restrict__ X, const float* __restrict__ W1,
                                         const float* __restrict__ W2, const float* __restrict__ dO,
                                         float* __restrict__ dW1, float* __restrict__ dW2, float* __restrict__ ws, int H,
-                                        int B, int E, int ldw, int cg, int nE, int nS, int rows_per_split, int t) {
+                                        int B, int E, int ldw, long long sx, long long sdo,
+                                        int cg, int nE, int nS, int rows_per_split, int t) {
   constexpr int NW = f32_nw(D), NTN = D / 32, KJ = DG / 8;
   constexpr int SUB = 128 * D;  // bytes of a [32][D] tile; a set's subtile is X, then dO
   const int lane = threadIdx.x & 63, g = lane >> 5, l32 = lane & 31;
@@ -338,8 +340,8 @@ __device__ __forceinline__ void dw_body(const float* __restrict__ X, const float
   const int e0 = (et * cg + grp) * 32, e = e0 + l32;
   const int b_lo = s * rows_per_split, b_hi = min(B, b_lo + rows_per_split);
   const int nsub = b_hi > b_lo ? (b_hi - b_lo + 31) / 32 : 0, ngrp = (nsub + rs - 1) / rs;
-  const float* Xh = X + (size_t)h * B * DG;
-  const float* dOh = dO + (size_t)h * B * DG;
+  const float* Xh = X + (size_t)h * sx;
+  const float* dOh = dO + (size_t)h * sdo;
   const int slot_bytes = rs * 2 * SUB;
   const Lanes<D, NTN> lt(g, l32);
 
@@ -440,22 +442,25 @@ __device__ __forceinline__ void dw_body(const float* __restrict__ X, const float
 template <int D, int DG, int ACT>
 __global__ void __launch_bounds__(f32_nw(D) * 64) __attribute__((amdgpu_waves_per_eu(f32_nw(D) / 4, f32_nw(D) / 4)))
 f32_fwd_kernel(const float* __restrict__ X, const float* __restrict__ W1, const float* __restrict__ W2,
-               float* __restrict__ O, int B, int E, int ldw, int tiles_per_head, int ep) {
-  rows_body<D, DG, ACT, false>(X, W1, W2, nullptr, O, B, E, ldw, tiles_per_head, ep, xcd_remap(blockIdx.x, gridDim.x));
+               float* __restrict__ O, int B, int E, int ldw, long long sx, long long sdo, int tiles_per_head,
+               int ep) {
+  rows_body<D, DG, ACT, false>(X, W1, W2, nullptr, O, B, E, ldw, sx, sdo,
+                               tiles_per_head, ep, xcd_remap(blockIdx.x, gridDim.x));
 }
 
 template <int D, int DG, int ACT>
 __global__ void __launch_bounds__(f32_nw(D) * 64) __attribute__((amdgpu_waves_per_eu(f32_nw(D) / 4, f32_nw(D) / 4)))
 f32_bwd_kernel(const float* __restrict__ X, const float* __restrict__ W1, const float* __restrict__ W2,
                const float* __restrict__ dO, float* __restrict__ dX, float* __restrict__ dW1, float* __restrict__ dW2,
-               float* __restrict__ ws, int H, int B, int E, int ldw, int tiles_per_head, int ep, int n_dx, int dx_first,
+               float* __restrict__ ws, int H, int B, int E, int ldw, long long sx, long long sdo, int tiles_per_head,
+               int ep, int n_dx, int dx_first,
                int cg, int nE, int nS, int rows_per_split) {
   const int b = blockIdx.x, n_dw = (int)gridDim.x - n_dx;
   const int bx = dx_first ? b : b - n_dw;  // index among the dX programs
   if (bx >= 0 && bx < n_dx) {
-    rows_body<D, DG, ACT, true>(X, W1, W2, dO, dX, B, E, ldw, tiles_per_head, ep, xcd_remap(bx, n_dx));
+    rows_body<D, DG, ACT, true>(X, W1, W2, dO, dX, B, E, ldw, sx, sdo, tiles_per_head, ep, xcd_remap(bx, n_dx));
   } else {
-    dw_body<D, DG, ACT>(X, W1, W2, dO, dW1, dW2, ws, H, B, E, ldw, cg, nE, nS, rows_per_split,
+    dw_body<D, DG, ACT>(X, W1, W2, dO, dW1, dW2, ws, H, B, E, ldw, sx, sdo, cg, nE, nS, rows_per_split,
                         xcd_remap(dx_first ? b - n_dx : b, n_dw));
   }
 }
@@ -578,7 +583,8 @@ hipError_t fwd_t(const FwdArgs& a, hipStream_t st) {
   const hipError_t e = set_lds_once((const void*)k, kMaxLds, lds_set);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(f32_nw(D) * 64), rows_lds(D, ep), st, (const float*)a.x,
-                     (const float*)a.w1, (const float*)a.w2, (float*)a.o, (int)a.B, (int)a.E, (int)a.ldw, (int)tph, ep);
+                     (const float*)a.w1, (const float*)a.w2, (float*)a.o, (int)a.B, (int)a.E, (int)a.ldw,
+                     (long long)a.sx, 0LL, (int)tph, ep);
   return hipGetLastError();
 }
 
@@ -594,7 +600,8 @@ hipError_t bwd_t(const BwdArgs& a, const F32Plan& p, hipStream_t st) {
   const int lds = std::max(n_dx > 0 ? rows_lds(D, p.ep) : 0, n_dw > 0 ? dw_lds(D, p.cg) : 0);
   hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(f32_nw(D) * 64), lds, st, (const float*)a.x, (const float*)a.w1,
                      (const float*)a.w2, (const float*)a.dout, (float*)a.dx, (float*)a.dw1, (float*)a.dw2, (float*)a.ws,
-                     (int)a.H, (int)a.B, (int)a.E, (int)a.ldw, p.dx_tiles_per_head, p.ep, (int)n_dx, p.dx_first ? 1 : 0,
+                     (int)a.H, (int)a.B, (int)a.E, (int)a.ldw, (long long)a.sx, (long long)a.sdo,
+                     p.dx_tiles_per_head, p.ep, (int)n_dx, p.dx_first ? 1 : 0,
                      p.cg, p.nE, p.nS, p.rows_per_split);
   if ((e = hipGetLastError()) != hipSuccess || n_dw == 0) return e;
   return launch_dw_reduce_f32(a, p.nS, st);

@@ -92,7 +92,7 @@ __host__ __device__ constexpr int fwd_pf(int D, int OC, int ES = 1) {
 template <bool BF16, int D, int ACT, int ES, int OC = 2, int NWP = fwd_waves(D), int DG = D>
 __global__ void __launch_bounds__(NWP * ES * 64) __attribute__((amdgpu_waves_per_eu(fwd_wpe(D, OC), fwd_wpe(D, OC))))
 fwd_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* __restrict__ W2,
-           void* __restrict__ O, int B, int E, int ldw, int H, int tiles_per_head, int outf32, int n_main,
+           void* __restrict__ O, int B, int E, int ldw, long long sx, int H, int tiles_per_head, int outf32, int n_main,
            int n_split, int xs, int nct, float* __restrict__ ws) {
   constexpr int NW = NWP, NT = NW * 64;  // waves, threads of one E part
   constexpr int KS = DG / 16;          // K steps of GEMM1 (at DG = D also GEMM2's operand count 2 * D/32)
@@ -150,7 +150,7 @@ fwd_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* __r
   const int e_end = min(E, c1 * 32);  // columns of W1 (rows of W2) this workgroup reads
   const unsigned RB = (unsigned)part * NSLOT * 128u * D;  // this part's ring
 
-  const u16* Xh = X + (size_t)h * B * DG;
+  const u16* Xh = X + (size_t)h * sx;
   const u16* W1h = W1 + (size_t)h * DG * ldw;  // rows of ldw elements (E, or E padded to 8)
   const u16* W2h = W2 + (size_t)h * E * DG;
   const int b_wave = bt * BB + wave * 32;
@@ -543,7 +543,8 @@ static hipError_t launch_fwd_e(const FwdArgs& a, const FwdPlan& p, int tiles_per
   if (e != hipSuccess) return e;
   const long long grid = p.n_main + (long long)p.n_split * p.xs;
   hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(64 * ES * NWP), lds, st, (const u16*)a.x,
-                     (const u16*)a.w1, (const u16*)a.w2, a.o, (int)a.B, (int)a.E, (int)a.ldw, (int)a.H, tiles_per_head,
+                     (const u16*)a.w1, (const u16*)a.w2, a.o, (int)a.B, (int)a.E, (int)a.ldw,
+                     (long long)a.sx, (int)a.H, tiles_per_head,
                      a.out_f32 ? 1 : 0, (int)p.n_main, p.n_split, p.xs, p.nct, (float*)a.ws);
   if ((e = hipGetLastError()) != hipSuccess || p.n_split == 0) return e;
   return launch_tile_reduce((const float*)a.ws, a.o, BF16, (int)a.B, D, 32 * NWP, (int)a.H, tiles_per_head,

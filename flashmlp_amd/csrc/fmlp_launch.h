@@ -36,6 +36,7 @@ struct FwdArgs {
   bool out_f32;  // outputs as fp32 (FMLP_OUT_F32)
   int num_cus;   // compute units of the current device
   int64_t ldw;   // row pitch of w1 (w1_pitch)
+  int64_t sx;    // elements between the heads of x (rows dense; B D, or 0 for one X shared by all)
   void* ws = nullptr;   // workspace for split tiles' partials (fwd_plan), or none
   size_t ws_bytes = 0;
 };
@@ -99,6 +100,7 @@ struct BwdArgs {
   bool want_dx = true;  // false: FMLP_BWD_NO_DX (only the dW programs run)
   bool want_dw = true;  // false: FMLP_BWD_NO_DW (only the dX programs run)
   int64_t ldw = 0;      // row pitch of w1, and of the fp32 dW partials (w1_pitch)
+  int64_t sx = 0, sdo = 0;  // elements between the heads of x and of dout (rows dense)
 };
 
 // io element types of the generic kernels

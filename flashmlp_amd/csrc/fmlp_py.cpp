@@ -35,6 +35,13 @@ bool dense16(const at::Tensor& t) {
   return t.dim() == 3 && t.is_contiguous() && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15u) == 0;
 }
 
+// x and dout: dense 16-byte aligned rows, heads any multiple of 16 bytes apart (0: one matrix
+// expanded to every head)
+bool rows16(const at::Tensor& t) {
+  return t.dim() == 3 && t.stride(2) == 1 && t.stride(1) == t.size(2) &&
+         (t.stride(0) * (int64_t)t.element_size()) % 16 == 0 && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15u) == 0;
+}
+
 // the tensors those kernels take as they are: one GPU, dense, aligned; sets the io
 // dtype code
 bool eligible(PyObject* const* args, int n, const at::Tensor** ts, int* code) {
@@ -48,7 +55,9 @@ bool eligible(PyObject* const* args, int n, const at::Tensor** ts, int* code) {
   if (c < 0) return false;
   for (int i = 0; i < n; ++i) {
     const at::Tensor& t = *ts[i];
-    if (t.scalar_type() != x.scalar_type() || t.device() != x.device() || !dense16(t)) return false;
+    if (t.scalar_type() != x.scalar_type() || t.device() != x.device() ||
+        !(dense16(t) || ((i == 0 || i == 3) && rows16(t))))
+      return false;
   }
   *code = c;
   return true;
@@ -80,7 +89,7 @@ PyObject* fast_fwd(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (!fmlp_shape_dense(D, E, code)) Py_RETURN_NONE;
   c10::DeviceGuard guard(x.device());
   const hipStream_t stream = c10::hip::getCurrentHIPStream(x.device().index()).stream();
-  at::Tensor o = at::empty_like(x);
+  at::Tensor o = x.is_contiguous() ? at::empty_like(x) : at::empty(x.sizes(), x.options());
   size_t n = fmlp_fwd_workspace_bytes(H, B, D, E, code);
   at::Tensor ws;
   if (n) {
@@ -90,8 +99,9 @@ PyObject* fast_fwd(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
       n = 0;
     }
   }
-  const int st = fmlp_fwd_ws(x.data_ptr(), w1.data_ptr(), w2.data_ptr(), o.data_ptr(), H, B, D, E, code, act,
-                             n ? ws.data_ptr() : nullptr, n, stream);
+  const int st = fmlp_fwd_strided_ws(x.data_ptr(), w1.data_ptr(), w2.data_ptr(), o.data_ptr(), H, B, D, E,
+                                     x.strides().data(), w1.strides().data(), w2.strides().data(), code, act,
+                                     n ? ws.data_ptr() : nullptr, n, stream);
   return Py_BuildValue("(iN)", st, THPVariable_Wrap(o));
   END_HANDLE_TH_ERRORS
 }
@@ -119,7 +129,7 @@ PyObject* fast_bwd(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   c10::DeviceGuard guard(x.device());
   const hipStream_t stream = c10::hip::getCurrentHIPStream(x.device().index()).stream();
   at::Tensor dx, dw1, dw2, ws;
-  if (need_dx) dx = at::empty_like(x);
+  if (need_dx) dx = x.is_contiguous() ? at::empty_like(x) : at::empty(x.sizes(), x.options());
   if (need_dw) {
     dw1 = at::empty_like(w1);
     dw2 = at::empty_like(w2);
@@ -149,10 +159,11 @@ PyObject* fast_bwd(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
       }
     }
   }
-  const int st = fmlp_bwd(x.data_ptr(), w1.data_ptr(), w2.data_ptr(), dout.data_ptr(),
-                          need_dx ? dx.data_ptr() : nullptr, need_dw ? dw1.data_ptr() : nullptr,
-                          need_dw ? dw2.data_ptr() : nullptr, H, B, D, E, flags, act, n ? ws.data_ptr() : nullptr, n,
-                          stream);
+  const int st = fmlp_bwd_strided(x.data_ptr(), w1.data_ptr(), w2.data_ptr(), dout.data_ptr(),
+                                  need_dx ? dx.data_ptr() : nullptr, need_dw ? dw1.data_ptr() : nullptr,
+                                  need_dw ? dw2.data_ptr() : nullptr, H, B, D, E, x.strides().data(),
+                                  w1.strides().data(), w2.strides().data(), dout.strides().data(), flags, act,
+                                  n ? ws.data_ptr() : nullptr, n, stream);
   return Py_BuildValue("(iNNN)", st, wrap_or_none(dx), wrap_or_none(dw1), wrap_or_none(dw2));
   END_HANDLE_TH_ERRORS
 }

@@ -27,9 +27,11 @@ Differences from the reference, all deliberate:
   * io dtypes are fp16, bf16 and fp32 (fp32 in true fp32, where the reference's tl.dot would
     use its default reduced input precision); other dtypes raise TypeError;
   * strided inputs are accepted: shapes with kernels of their own (fmlp_shape_dense: 16-bit
-    io, and fp32 with D <= 128) copy them to dense tensors, as the reference's reshape / contiguous does
-    (flashmlp.py:453-459,508); every other shape reads the views in place (generic kernels),
-    where the reference would copy them or fail its contiguity assertions.
+    io, and fp32 with D <= 128) read an x or do of dense rows in place, whatever the distance of its
+    heads (an x expanded to every head, say), and copy other views to dense tensors, as the
+    reference's reshape / contiguous does (flashmlp.py:453-459,508); every other shape reads the
+    views in place (generic kernels), where the reference would copy them or fail its contiguity
+    assertions.
 """
 from __future__ import annotations
 
@@ -131,10 +133,19 @@ def _io_code(x: torch.Tensor, *ts: torch.Tensor):
 
 
 def _dense_all(*ts: torch.Tensor):
-    # the tuned kernels' inputs: unchanged when all are dense and 16-byte aligned
+    # the tuned kernels' weights: unchanged when all are dense and 16-byte aligned
     if all(t.is_contiguous() and t.data_ptr() % 16 == 0 for t in ts):
         return ts
     return tuple(_dense(t) for t in ts)
+
+
+def _rows(t: torch.Tensor) -> torch.Tensor:
+    # x and do of the tuned kernels: rows dense and 16-byte aligned, heads any multiple of 16
+    # bytes apart (0 for one matrix expanded to every head); anything else is copied
+    s = t.stride()
+    if s[2] == 1 and s[1] == t.shape[2] and s[0] * t.element_size() % 16 == 0 and t.data_ptr() % 16 == 0:
+        return t
+    return _dense(t)
 
 
 def _empty_as(t: torch.Tensor, shape) -> torch.Tensor:
@@ -180,14 +191,17 @@ def flashmlp_fwd(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, activation
     try:
         stream = _stream_of(dev)
         if _own_kernels(D, E, dtype):
-            x, w1, w2 = _dense_all(x, w1, w2)
+            x = _rows(x)
+            w1, w2 = _dense_all(w1, w2)
             ws_bytes = _fwd_ws_bytes(dev, H, B, D, E, dtype)
             try:
                 ws = _alloc_ws(ws_bytes, x.device)
             except torch.OutOfMemoryError:  # the kernels then run every tile whole
                 ws, ws_bytes = None, 0
-            st = L.fmlp_fwd_ws(x.data_ptr(), w1.data_ptr(), w2.data_ptr(), o.data_ptr(), H, B, D, E, dtype,
-                               _act_code(activation), ws.data_ptr() if ws is not None else None, ws_bytes, stream)
+            st = L.fmlp_fwd_strided_ws(x.data_ptr(), w1.data_ptr(), w2.data_ptr(), o.data_ptr(), H, B, D, E,
+                                       _lib.strides(x), _lib.strides(w1), _lib.strides(w2), dtype,
+                                       _act_code(activation), ws.data_ptr() if ws is not None else None, ws_bytes,
+                                       stream)
         else:
             st = L.fmlp_fwd_strided(x.data_ptr(), w1.data_ptr(), w2.data_ptr(), o.data_ptr(), H, B, D, E,
                                     _lib.strides(x), _lib.strides(w1), _lib.strides(w2), dtype,
@@ -249,7 +263,8 @@ def flashmlp_bwd(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, do: torch.
     try:
         stream = _stream_of(dev)
         if _own_kernels(D, E, dtype):
-            x, w1, w2, do = _dense_all(x, w1, w2, do)
+            x, do = _rows(x), _rows(do)
+            w1, w2 = _dense_all(w1, w2)
             ws_bytes = _ws_bytes(dev, H, B, D, E, flags)
             try:
                 ws = _alloc_ws(ws_bytes, x.device)
@@ -266,9 +281,10 @@ def flashmlp_bwd(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, do: torch.
                     if _lib.lib().fmlp_shape_tuned(D, E, dtype):
                         raise
                     ws, ws_bytes = None, 0  # any workspace is accepted
-            st = L.fmlp_bwd(x.data_ptr(), w1.data_ptr(), w2.data_ptr(), do.data_ptr(), _ptr(dx),
-                            _ptr(dw1), _ptr(dw2), H, B, D, E, flags, _act_code(activation),
-                            ws.data_ptr() if ws is not None else None, ws_bytes, stream)
+            st = L.fmlp_bwd_strided(x.data_ptr(), w1.data_ptr(), w2.data_ptr(), do.data_ptr(), _ptr(dx),
+                                    _ptr(dw1), _ptr(dw2), H, B, D, E, _lib.strides(x), _lib.strides(w1),
+                                    _lib.strides(w2), _lib.strides(do), flags, _act_code(activation),
+                                    ws.data_ptr() if ws is not None else None, ws_bytes, stream)
         else:
             # the generic kernels' dW programs split B with fp32 partials in the workspace when
             # it is given; without one (it does not fit) they run unsplit
@@ -308,6 +324,20 @@ class FlashMLPFunction(torch.autograd.Function):
         dx, dw1, dw2 = flashmlp_bwd(x, w1, w2, do, ctx.activation, accurate_dw=ctx.accurate_dw,
                                     _needs=(need_x, need_w1 or need_w2))
         return dx, (dw1 if need_w1 else None), (dw2 if need_w2 else None), None, None
+
+
+class _HeadMean(torch.autograd.Function):
+    """o.mean(dim=0) whose gradient is handed to every head as one expanded (B, D) matrix: the same
+    values as autograd's, which divides after the expansion and so writes H copies."""
+
+    @staticmethod
+    def forward(ctx, o):
+        ctx.heads = o.shape[0]
+        return o.mean(dim=0)
+
+    @staticmethod
+    def backward(ctx, g):
+        return (g / ctx.heads).unsqueeze(0).expand(ctx.heads, *g.shape)
 
 
 class FlashMLP(torch.nn.Module):
@@ -359,5 +389,5 @@ class FlashMLP(torch.nn.Module):
             o = FlashMLPFunction.apply(x, self.w1, self.w2, self.activation, self.accurate_dw)
 
         if squeeze_output:
-            o = o.mean(dim=0)
+            o = _HeadMean.apply(o) if o.requires_grad and not torch.compiler.is_compiling() else o.mean(dim=0)
         return o

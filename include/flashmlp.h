@@ -158,11 +158,17 @@ int fmlp_fwd_ws(const void* x, const void* w1, const void* w2, void* o, int64_t 
 /* fmlp_fwd with X (H,B,D), W1 (H,D,E), W2 (H,E,D) given as strided views: each *_strides is
  * three non-negative element strides (head, row, column); o stays dense. No counterpart in
  * the reference, whose wrapper copies such views through reshape / contiguous
- * (flashmlp.py:453-459): for callers holding sliced or transposed tensors. Dense strides
- * take the tuned kernels when the shape allows, other strides the generic kernels. */
+ * (flashmlp.py:453-459): for callers holding sliced or transposed tensors. Dense weights and an X
+ * of dense rows, whose heads may be any multiple of 16 bytes apart (stride 0: one X for every
+ * head), take the same kernels as dense tensors; other strides the generic kernels. */
 int fmlp_fwd_strided(const void* x, const void* w1, const void* w2, void* o, int64_t H, int64_t B, int64_t D,
                      int64_t E, const int64_t* x_strides, const int64_t* w1_strides, const int64_t* w2_strides,
                      int dtype, int act, void* stream);
+
+/* fmlp_fwd_strided with a device workspace, as fmlp_fwd_ws. No counterpart in the reference. */
+int fmlp_fwd_strided_ws(const void* x, const void* w1, const void* w2, void* o, int64_t H, int64_t B, int64_t D,
+                        int64_t E, const int64_t* x_strides, const int64_t* w1_strides, const int64_t* w2_strides,
+                        int dtype, int act, void* workspace, size_t workspace_bytes, void* stream);
 
 /* Bytes of device workspace fmlp_bwd / fmlp_bwd_strided need for these shapes and dtype flags
  * on the current device, whatever the activation (0 when none is needed). Every backward flag

@@ -1,0 +1,72 @@
+"""x and do of dense rows whose heads lie any multiple of 16 bytes apart (0: one matrix expanded to
+every head) are read in place: bit-identical to the same values passed densely, with no copy of
+them allocated; other views are copied as before.
+"""
+import pytest
+import torch
+
+import flashmlp_amd as fm
+from oracle.inputs import make_inputs
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(4, 300, 128, 256, torch.bfloat16), (4, 1025, 64, 683, torch.float16), (3, 129, 256, 264, torch.bfloat16),
+          (5, 200, 32, 96, torch.float16), (3, 77, 16, 45, torch.bfloat16), (3, 257, 64, 100, torch.float32),
+          (1, 4096, 128, 1024, torch.bfloat16), (2, 130, 256, 40, torch.float32), (12, 1024, 64, 768, torch.float16)]
+
+
+def _views(t, pad):
+    """t with its heads `pad` elements further apart than dense"""
+    H, B, D = t.shape
+    buf = torch.full((H, B * D + pad), float("nan"), dtype=t.dtype, device=t.device)
+    v = buf[:, :B * D].view(H, B, D)
+    v.copy_(t)
+    return v
+
+
+@pytest.mark.parametrize("H,B,D,E,dt", SHAPES)
+def test_views_match_dense(H, B, D, E, dt):
+    print(f"[heads] H={H} B={B} D={D} E={E} {dt}", flush=True)
+    x, w1, w2, do = (t.cuda() for t in make_inputs(H, B, D, E, dt, seed=B))
+    xe, de = x[:1].expand(H, B, D), do[:1].expand(H, B, D)
+    cases = [(xe, de), (_views(x, 8), do), (x, _views(do, 16)), (_views(x, 24), de),
+             (_views(x, 3), do),  # heads not 16-byte aligned: copied
+             (x.transpose(0, 1).contiguous().transpose(0, 1), do)]  # rows not dense: copied
+    for xv, dv in cases:
+        for kw in ({}, {"accurate_dw": True}, {"recompute": True}):
+            ref = (fm.flashmlp_fwd(xv.contiguous(), w1, w2, "silu"),
+                   *fm.flashmlp_bwd(xv.contiguous(), w1, w2, dv.contiguous(), "silu", **kw))
+            got = (fm.flashmlp_fwd(xv, w1, w2, "silu"), *fm.flashmlp_bwd(xv, w1, w2, dv, "silu", **kw))
+            for name, a, b in zip(("o", "dx", "dw1", "dw2"), got, ref):
+                assert a.is_contiguous() and torch.equal(a, b), (name, xv.stride(), dv.stride(), kw)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+def test_shared_input_module(dt):
+    # the module's 2-D input: gradients bit-identical to autograd's mean over dense copies
+    torch.manual_seed(0)
+    m = fm.FlashMLP(6, 64, 256, activation="silu", dtype=dt)
+    x = torch.randn(700, 64, device="cuda", dtype=dt, requires_grad=True)
+    g = torch.randn(700, 64, device="cuda", dtype=dt)
+    got = torch.autograd.grad(m(x), (x, m.w1, m.w2), g)
+    o = fm.FlashMLPFunction.apply(x.unsqueeze(0).expand(6, -1, -1).contiguous(), m.w1, m.w2, "silu").mean(dim=0)
+    ref = torch.autograd.grad(o, (x, m.w1, m.w2), g)
+    assert torch.equal(m(x), o)
+    for a, b in zip(got, ref):
+        assert torch.equal(a, b)
+    with torch.no_grad():
+        assert torch.equal(m(x), o)
+
+
+def test_no_copy_is_allocated():
+    H, B, D, E = 16, 4096, 128, 64
+    x = torch.randn(B, D, device="cuda", dtype=torch.bfloat16)
+    w1 = torch.randn(H, D, E, device="cuda", dtype=torch.bfloat16)
+    w2 = torch.randn(H, E, D, device="cuda", dtype=torch.bfloat16)
+    xe = x.expand(H, B, D)
+    fm.flashmlp_fwd(xe, w1, w2, "silu")
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    o = fm.flashmlp_fwd(xe, w1, w2, "silu")
+    assert torch.cuda.max_memory_allocated() - before < o.numel() * 2 * 1.5  # the output alone
