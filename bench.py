@@ -440,8 +440,15 @@ def _bwd_form(H, B, D, E, dt_name, act, accurate_dw=False, recompute=False):
 
     code = {"bf16": _lib.FMLP_DTYPE_BF16, "f16": _lib.FMLP_DTYPE_F16, "f32": _lib.FMLP_DTYPE_F32}[dt_name]
     if not _lib.lib().fmlp_shape_tuned(D, E, code):
-        # dense 16-bit D = 256 (E % 8 == 0): the D = 256 dX and dW programs
-        return "dx256+dw256" if D == 256 and dt_name != "f32" and E % 8 == 0 else "generic"
+        # dense 16-bit D = 256: the D = 256 dW programs, with dX from the dZ they store or from
+        # programs of its own; fp32 and D < 64: the dense kernels of those shapes
+        if D == 256 and dt_name != "f32":
+            code |= _lib.FMLP_BWD_RECOMPUTE if recompute else 0
+            stored = _lib.lib().fmlp_bwd_stores_dz(H, B, D, E, code, _lib.ACT_CODES[act])
+            return "dw256+dxg256" if stored else "dx256+dw256"
+        if _lib.lib().fmlp_shape_dense(D, E, code):
+            return "fp32" if dt_name == "f32" else "recompute"
+        return "generic"
     code |= (_lib.FMLP_DW_HILO if accurate_dw else 0) | (_lib.FMLP_BWD_RECOMPUTE if recompute else 0)
     return "stored-dZ" if _lib.lib().fmlp_bwd_stores_dz(H, B, D, E, code, _lib.ACT_CODES[act]) else "recompute"
 
@@ -843,6 +850,8 @@ def main():
         kernels = {"stored-dZ": "fmlp::dw2_kernel (storing dZ), fmlp::dxg_kernel",
                    "recompute": "fmlp::bwd_kernel (dW and dX programs)",
                    "generic": "fmlp::gen_dw_kernel, fmlp::gen_dx_kernel",
+                   "fp32": "fmlp::f32_bwd_kernel",
+                   "dw256+dxg256": "fmlp::dw256_kernel (storing dZ), fmlp::dxg256_kernel",
                    "dx256+dw256": "fmlp::dx256_kernel, fmlp::dw256_kernel"}[form]
         line["roofline"] = {
             "kernel": f"fmlp_bwd ({form}): {kernels}",

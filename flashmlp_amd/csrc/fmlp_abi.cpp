@@ -89,6 +89,9 @@ int dz_mode_of(int dtype) {
   return (dtype & FMLP_BWD_STORE_DZ) ? fmlp::DZ_FORCE : fmlp::DZ_AUTO;
 }
 
+// the same at D = 256, whose B split does not depend on the form
+int dz256_mode(int dtype) { return (dtype & FMLP_BWD_NO_DX) ? (int)fmlp::DZ_NEVER : dz_mode_of(dtype); }
+
 // workspace bytes a tuned backward with these flags needs under plan p: with FMLP_BWD_NO_DX the
 // dW programs' fp32 partials alone (no dZ, no split dX tiles), with FMLP_BWD_NO_DW the split
 // ragged dX tiles' partials alone (none when the plan does not split them)
@@ -388,7 +391,8 @@ FMLP_EXPORT size_t fmlp_bwd_workspace_bytes(int64_t H, int64_t B, int64_t D, int
     return w > n ? w : n;
   }
   if (D == 256) {
-    const size_t w = pad + fmlp::plan_dw256(H, B, E, (dtype & FMLP_DW_HILO) != 0, cus, (size_t)-1).ws_bytes;
+    const size_t w =
+        pad + fmlp::plan_dw256(H, B, E, (dtype & FMLP_DW_HILO) != 0, dz256_mode(dtype), cus, (size_t)-1).ws_bytes;
     return w > n ? w : n;
   }
   // the plan depends on the activation, which this query does not take: the largest over them
@@ -413,8 +417,9 @@ FMLP_EXPORT int fmlp_bwd_plan(int64_t H, int64_t B, int64_t D, int64_t E, int dt
     // D = 256: the dX programs (128 rows each) and the dW programs' split with an unlimited
     // workspace (a call splits B only as far as its workspace holds)
     const bool no_dw = (dtype & FMLP_BWD_NO_DW) != 0, no_dx = (dtype & FMLP_BWD_NO_DX) != 0;
-    const fmlp::Dw256Plan w = fmlp::plan_dw256(H, B, E, (dtype & FMLP_DW_HILO) != 0, cus, (size_t)-1);
-    const int64_t v[11] = {0, no_dw ? 1 : w.nS, 1, 0, 0, no_dw ? 0 : w.n, no_dx ? 0 : H * ((B + 127) / 128), 0,
+    const fmlp::Dw256Plan w =
+        fmlp::plan_dw256(H, B, E, (dtype & FMLP_DW_HILO) != 0, dz256_mode(dtype), cus, (size_t)-1);
+    const int64_t v[11] = {w.dz ? 1 : 0, no_dw ? 1 : w.nS, 1, 0, 0, no_dw ? 0 : w.n, no_dx ? 0 : H * ((B + 127) / 128), 0,
                            no_dw ? 0 : (int64_t)w.ws_bytes, act, 128};
     for (int i = 0; i < n_info && i < 11; ++i) info[i] = v[i];
     return ok();
@@ -435,9 +440,11 @@ FMLP_EXPORT int fmlp_bwd_plan(int64_t H, int64_t B, int64_t D, int64_t E, int dt
 FMLP_EXPORT int fmlp_bwd_stores_dz(int64_t H, int64_t B, int64_t D, int64_t E, int dtype, int act) {
   if (check_shape(H, B, D, E, dtype) != FMLP_OK || check_act(act) != FMLP_OK) return 0;
   // the other kernels recompute
-  if (!dense_shape(D, E, io_of(dtype)) || D == 256 || io_of(dtype) == FMLP_DTYPE_F32) return 0;
+  if (!dense_shape(D, E, io_of(dtype)) || io_of(dtype) == FMLP_DTYPE_F32) return 0;
   int cus = 0;
   if (num_cus_current(&cus) != FMLP_OK) return 0;
+  if (D == 256)
+    return fmlp::plan_dw256(H, B, E, (dtype & FMLP_DW_HILO) != 0, dz256_mode(dtype), cus, (size_t)-1).dz ? 1 : 0;
   if (dtype & (FMLP_BWD_NO_DX | FMLP_BWD_NO_DW)) return 0;  // a partial backward stores no dZ
   return fmlp::plan_bwd(H, B, D, E, act, (dtype & FMLP_DW_HILO) != 0, dz_mode_of(dtype), cus).dz ? 1 : 0;
 }
@@ -545,7 +552,7 @@ int bwd_impl(const void* x, const void* w1, const void* w2, const void* dout, vo
     if (want_dw) {
       int cus = 0;
       if ((st = num_cus_current(&cus))) return st;
-      wp = fmlp::plan_dw256(H, B, E, (dtype & FMLP_DW_HILO) != 0, cus, given - pad);
+      wp = fmlp::plan_dw256(H, B, E, (dtype & FMLP_DW_HILO) != 0, dz256_mode(dtype), cus, given - pad);
       if (wp.ws_bytes > 0) {
         ws = pad > 0 ? (char*)w1p + pad : workspace;
         if (noalloc && pad == 0) {
@@ -557,8 +564,9 @@ int bwd_impl(const void* x, const void* w1, const void* w2, const void* dout, vo
     fmlp::BwdArgs a{x, w1p, w2, dout, dx, dw1, dw2, H, B, D, E, io == FMLP_DTYPE_BF16, act, ws,
                     (dtype & FMLP_OUT_F32) != 0, (dtype & FMLP_DW_HILO) != 0, want_dx, want_dw,
                     fmlp::w1_pitch(E, (int)es), head_stride(sx, H, B, D), head_stride(sdo, H, B, D)};
-    if (want_dx) e = fmlp::launch_dx256(a, (hipStream_t)stream);
+    if (want_dx && !wp.dz) e = fmlp::launch_dx256(a, (hipStream_t)stream);
     if (e == hipSuccess && want_dw) e = fmlp::launch_dw256(a, wp, (hipStream_t)stream);
+    if (e == hipSuccess && wp.dz) e = fmlp::launch_dxg256(a, wp, (hipStream_t)stream);
   } else {
     fmlp::GenArgs g = gen_args(x, w1, w2, dout, nullptr, dx, dw1, dw2, H, B, D, E, dtype, act);
     g.want_dx = want_dx ? 1 : 0;

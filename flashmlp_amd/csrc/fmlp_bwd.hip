@@ -811,12 +811,13 @@ static_assert(DW4_PF <= DW4_NSLOT - 1, "a slot is reloaded only after the barrie
 static_assert(DW4_PF >= 2 && 2 * DW4_SLOT == 256 * DW_ET * 2, "the W1c staging tile fills the ring's last two slots");
 static_assert(16 % (DW4_PD + 1) == 0, "each 16-step group starts at ring slot 0");
 
-template <bool BF16, int ACT, bool HILO>
+// DZ: also stores dZ in the image dxg256_kernel reads (dw2_body's).
+template <bool BF16, int ACT, bool HILO, bool DZ>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 dw256_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* __restrict__ W2,
              const u16* __restrict__ dO, void* __restrict__ dW1, void* __restrict__ dW2, float* __restrict__ ws,
              int H, int B, int E, int ldw, long long sx, long long sdo,
-             int nE, int nS, int rows_per_split, int outf32) {
+             int nE, int nS, int rows_per_split, int outf32, u16* __restrict__ dzt, int Bp) {
   constexpr int D = 256, KS = D / 16, NTN = D / 32;
   constexpr int STG = 2 * DW4_SLOT;  // W1c staging tile: [256 d][128 e], 256-byte rows
   constexpr int PD = DW4_PD;
@@ -1004,9 +1005,19 @@ dw256_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* _
       if constexpr (HILO) a1[nt] = mfma<BF16>(dzL[s2], op, a1[nt]);
       __builtin_amdgcn_sched_barrier(0);
     }
+    if constexpr (DZ) {  // rows 16 s + 8 g .. + 7 under sig of column e0 + l32, as in dw2_body
+      const int rbase = b_lo + i * DW_BT, Ep = nE * DW_ET;
+      const unsigned blk = ((unsigned)(rbase >> 8) * (unsigned)(Ep >> 5) + (unsigned)(e0 >> 5)) * 8u +
+                           (unsigned)((rbase & 255) >> 5);
+      const Rsrc rb = make_rsrc(dzt + (size_t)h * Ep * Bp + (size_t)blk * 1024u, 2048);
+#pragma unroll
+      for (int s2 = 0; s2 < 2; ++s2)
+        __builtin_amdgcn_raw_buffer_store_b128(dzT[s2], rb, (l32 * 32 + 16 * s2 + 8 * g) * 2, 0, CPOL_NT);
+    }
     // subtile i + 1 has landed (this wave's part; the barrier publishes the others' and retires
-    // every read of slot i, which subtile i + 4 reuses)
-    wait_vmcnt<(DW4_PF - 1) * DW4_NPL>();
+    // every read of slot i, which subtile i + 4 reuses); behind its loads lie those of the next
+    // DW4_PF - 1 subtiles and (DZ) at least as many pairs of dZ stores
+    wait_vmcnt<(DW4_PF - 1) * (DW4_NPL + (DZ ? 2 : 0))>();
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
@@ -1378,6 +1389,123 @@ dxg_kernel(const u16* __restrict__ dzt, const u16* __restrict__ W1, void* __rest
 }
 
 // ------------------------------------------------------------------------------------
+// dX from the stored dZ at D = 256 (dxg256_kernel): a workgroup owns 128 rows of one head (half of
+// a 256-row dZ block), 8 waves = 2 groups of 64 rows x 4 quarters of the columns, so that the
+// four accumulator tiles and operands of a wave leave room for four waves per SIMD (two
+// workgroups per CU, whose starts and ends overlap). Per 32-column E-chunk: dZ (8 KB, read once) and
+// W1c (16 KB, L2-resident) through a 3-slot LDS ring two chunks ahead, one barrier, and 8 MFMAs
+// per wave from 8 KB of operand reads. The products and their order are dxg_kernel's, and so the
+// bits of dX those of the recomputing programs.
+// ------------------------------------------------------------------------------------
+constexpr int DXG4_ZT = 128 * 32 * 2;    // dZ chunk bytes of 128 rows
+constexpr int DXG4_WT = 64 * 256;        // W1c chunk bytes
+constexpr int DXG4_SLOT = DXG4_ZT + DXG4_WT;
+constexpr int DXG4_NSLOT = 3;
+
+template <bool BF16>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4)))
+dxg256_kernel(const u16* __restrict__ dzt, const u16* __restrict__ W1, void* __restrict__ dX, int B, int Bp, int E,
+              int ldw, int Ep, int tiles_per_head, int outf32) {
+  constexpr int D = 256;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int G = lane >> 4, i16 = lane & 15, g = lane >> 5, l32 = lane & 31;
+  const int rg = wave & 1, cq = wave >> 1;  // row group, column quarter
+  const int t = xcd_remap(blockIdx.x, gridDim.x);
+  const int h = t / tiles_per_head, ht = t - h * tiles_per_head;
+  const int NC = (E + 31) >> 5;
+  // chunk c of a 256-row block is 8192 elements, this half's the 4096 at (ht & 1) 4096
+  const u16* zb = dzt + ((size_t)h * Bp + (size_t)(ht >> 1) * DX2_ROWS) * Ep + (size_t)(ht & 1) * 4096;
+  const u16* W1h = W1 + (size_t)h * D * ldw;
+
+  // W1c piece p = tid + 512 k: row r = p / 4, chunk (p % 4) ^ ((r / 4) % 4) (the same for both k)
+  const int wr = tid >> 2, wq = (tid & 3) ^ ((wr >> 2) & 3);
+  const unsigned wOff = (unsigned)(wr * ldw * 2 + wq * 16);
+  auto dma = [&](int c) {  // chunks past the last load nothing
+    const int slot = (c % DXG4_NSLOT) * DXG4_SLOT + wave * 1024;
+    const int lim = E - c * 32, rem = D * ldw * 2 - 64 * c;
+    buf_load16_lds_nt(make_rsrc_words(zb + (size_t)c * 8192, lim > 0 ? DXG4_ZT : 0), (unsigned)tid * 16u, slot);
+    const i32x4 rw = make_rsrc_words(W1h + (size_t)c * 32, lim > 0 && rem > 0 ? rem : 0);
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+      buf_load16_lds(rw, wq * 8 < lim ? wOff + (unsigned)(k * 128 * ldw * 2) : BUF_OOB, slot + DXG4_ZT + k * 8192);
+  };
+  const int laneA = (2 * rg) * 2048 + (8 * g + (i16 >> 2)) * 64 + 32 * (G & 1) + 8 * (i16 & 3);
+  int offB[2];
+#pragma unroll
+  for (int s2 = 0; s2 < 2; ++s2)
+    offB[s2] = DXG4_ZT + cq * 4096 + l32 * 64 + (((2 * s2 + g) ^ ((l32 >> 2) & 3)) << 4);
+
+  f32x16 acc[2][2];  // [32-row block of the group][32-column tile of the quarter]
+#pragma unroll
+  for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[rb][j] = zero16();
+  dma(0);
+  dma(1);
+  for (int c = 0; c < NC; ++c) {
+    wait_vmcnt<3>();  // chunk c has landed (the three loads of chunk c + 1 may be in flight)
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();  // chunk c visible; chunk c - 1 no longer read
+    asm volatile("" ::: "memory");
+    dma(c + 2);
+    const int base = (c % DXG4_NSLOT) * DXG4_SLOT;
+    u32x4 a[2][2], b[2][2];
+#pragma unroll
+    for (int s2 = 0; s2 < 2; ++s2) {
+#pragma unroll
+      for (int rb = 0; rb < 2; ++rb)
+        a[rb][s2] = cat(lds_read_tr(base + laneA + rb * 2048 + s2 * 1024),
+                        lds_read_tr(base + laneA + rb * 2048 + s2 * 1024 + 256));
+#pragma unroll
+      for (int j = 0; j < 2; ++j) b[s2][j] = lds_read16(base + offB[s2] + j * 2048);
+    }
+#pragma unroll
+    for (int s2 = 0; s2 < 2; ++s2)
+#pragma unroll
+      for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[rb][j] = mfma<BF16>(b[s2][j], a[rb][s2], acc[rb][j]);
+  }
+  wait_vmcnt<0>();  // loads past the last chunk are still landing
+  // lane l32 holds row sig(l32) of each 32-row block, columns 32 nt + 8 q + 4 g + 0..3
+  const int row0 = ht * 128;
+  const int rows = clamp0(B - row0, 128);
+  const int es = outf32 ? 4 : 2;
+  const Rsrc ro = make_rsrc((const char*)dX + ((size_t)h * B + row0) * D * es, rows * D * es);
+#pragma unroll
+  for (int rb = 0; rb < 2; ++rb) {
+    const unsigned r = (unsigned)((2 * rg + rb) * 32) + sig((unsigned)l32);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int col = (2 * cq + j) * 32;
+      if (outf32) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const u32x4 v = {__float_as_uint(acc[rb][j][4 * q]), __float_as_uint(acc[rb][j][4 * q + 1]),
+                           __float_as_uint(acc[rb][j][4 * q + 2]), __float_as_uint(acc[rb][j][4 * q + 3])};
+          __builtin_amdgcn_raw_buffer_store_b128(v, ro, (int)((r * D + col + 8 * q + 4 * g) * 4u), 0, 0);
+        }
+      } else {
+        u32x2 v[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          v[q] = u32x2{pack2<BF16>(acc[rb][j][4 * q], acc[rb][j][4 * q + 1]),
+                       pack2<BF16>(acc[rb][j][4 * q + 2], acc[rb][j][4 * q + 3])};
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {  // one swap per pair of pieces: 8 consecutive columns per lane
+          const auto s0 = __builtin_amdgcn_permlane32_swap(v[2 * p][0], v[2 * p + 1][0], false, false);
+          const auto s1 = __builtin_amdgcn_permlane32_swap(v[2 * p][1], v[2 * p + 1][1], false, false);
+          const u32x4 w = {s0[0], s1[0], s0[1], s1[1]};
+          __builtin_amdgcn_raw_buffer_store_b128(w, ro, (int)((r * D + col + 16 * p + 8 * g) * 2u), 0, 0);
+        }
+      }
+    }
+  }
+}
+
+// ------------------------------------------------------------------------------------
 // host side
 // ------------------------------------------------------------------------------------
 // ------------------------------------------------------------------------------------
@@ -1670,7 +1798,7 @@ BwdPlan plan_bwd(int64_t H, int64_t B, int64_t D, int64_t E, int act, bool hilo,
 // rounds of programs over the CUs times a program's time (a fixed part and one per 32-row
 // subtile) plus, for nS > 1, the summing launch and the partials' traffic (written, then read).
 // FMLP_DW256_NS (read once per process) forces nS where its workspace fits.
-Dw256Plan plan_dw256(int64_t H, int64_t B, int64_t E, bool hilo, int num_cus, size_t max_ws) {
+Dw256Plan plan_dw256(int64_t H, int64_t B, int64_t E, bool hilo, int dz_mode, int num_cus, size_t max_ws) {
   constexpr double kFixedUs = 4.0, kSubUs = 1.0, kSubHiloUs = 1.4;
   static const int ns_env = env_int("FMLP_DW256_NS", 0);
   Dw256Plan p{};
@@ -1700,6 +1828,21 @@ Dw256Plan plan_dw256(int64_t H, int64_t B, int64_t E, bool hilo, int num_cus, si
       p.n = progs;
       p.ws_bytes = ws;
     }
+  }
+  // The stored-dZ form: 2u of matrix work for dX instead of 6u, for writing and reading dZ once (2
+  // bytes each per element against 1024 FLOPs saved). Whenever it fits: measured bf16 SiLU backwards,
+  // recompute -> stored: H=8 B=4096 E=1024 151 -> 124 us, H=16 B=8192 E=2048 897 -> 725, H=2 B=1024
+  // E=1024 87 -> 60, H=1 B=3000 E=64 43 -> 38, H=3 B=16 E=128 25 -> 19, H=1 B=1 E=64 20 -> 15.
+  static const int dz_env = env_int("FMLP_BWD_DZ", -1);
+  const int want = dz_mode != DZ_AUTO ? (dz_mode == DZ_FORCE ? 1 : 0) : dz_env;
+  const long long Bp = (B + DX2_ROWS - 1) / DX2_ROWS * DX2_ROWS;
+  const size_t off = (p.ws_bytes + 255) / 256 * 256;
+  const size_t dz_head = (size_t)p.nE * DW_ET * (size_t)Bp * 2u;
+  if (want != 0 && dz_head < ((size_t)1 << 31) && off + (size_t)H * dz_head <= max_ws && B > 0) {
+    p.dz = true;
+    p.Bp = (int)Bp;
+    p.dz_off = off;
+    p.ws_bytes = off + (size_t)H * dz_head;
   }
   return p;
 }
@@ -1885,21 +2028,48 @@ hipError_t launch_dx256(const BwdArgs& a, hipStream_t st) {
   return a.bf16 ? launch_dx256_a<true>(a, st) : launch_dx256_a<false>(a, st);
 }
 
-template <bool BF16, int ACT, bool HILO>
-static hipError_t launch_dw256_t(const BwdArgs& a, const Dw256Plan& p, hipStream_t st) {
+template <bool BF16, int ACT, bool HILO, bool DZ>
+static hipError_t launch_dw256_z(const BwdArgs& a, const Dw256Plan& p, hipStream_t st) {
   if (p.n <= 0) return hipSuccess;
   if (p.n > 0x7fffffffLL) return hipErrorInvalidValue;
   constexpr size_t lds = (size_t)DW4_NSLOT * DW4_SLOT;
-  auto k = dw256_kernel<BF16, ACT, HILO>;
+  auto k = dw256_kernel<BF16, ACT, HILO, DZ>;
   static std::atomic<unsigned long long> lds_set{0};
   hipError_t e = set_lds_once((const void*)k, (int)lds, lds_set);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(k, dim3((unsigned)p.n), dim3(256), lds, st, (const u16*)a.x, (const u16*)a.w1, (const u16*)a.w2,
                      (const u16*)a.dout, a.dw1, a.dw2, (float*)a.ws, (int)a.H, (int)a.B, (int)a.E, (int)a.ldw,
                      (long long)a.sx, (long long)a.sdo, p.nE, p.nS,
-                     p.rows_per_split, a.out_f32 ? 1 : 0);
+                     p.rows_per_split, a.out_f32 ? 1 : 0, (u16*)((char*)a.ws + p.dz_off), p.Bp);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   return launch_dw_reduce<BF16>(a, p.nS, st);
+}
+
+template <bool BF16, int ACT, bool HILO>
+static hipError_t launch_dw256_t(const BwdArgs& a, const Dw256Plan& p, hipStream_t st) {
+  return p.dz ? launch_dw256_z<BF16, ACT, HILO, true>(a, p, st) : launch_dw256_z<BF16, ACT, HILO, false>(a, p, st);
+}
+
+template <bool BF16>
+static hipError_t launch_dxg256_t(const BwdArgs& a, const Dw256Plan& p, hipStream_t st) {
+  const long long tph = (a.B + 127) / 128, grid = tph * a.H;
+  if (grid <= 0) return hipSuccess;
+  if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
+  constexpr int lds = DXG4_NSLOT * DXG4_SLOT;
+  static_assert(lds <= 80 * 1024, "two workgroups per CU");
+  auto k = dxg256_kernel<BF16>;
+  static std::atomic<unsigned long long> lds_set{0};
+  const hipError_t e = set_lds_once((const void*)k, lds, lds_set);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(512), lds, st, (const u16*)((const char*)a.ws + p.dz_off),
+                     (const u16*)a.w1, a.dx, (int)a.B, p.Bp, (int)a.E, (int)a.ldw, p.nE * DW_ET, (int)tph,
+                     a.out_f32 ? 1 : 0);
+  return hipGetLastError();
+}
+
+// dX from the dZ that launch_dw256 stored (p.dz)
+hipError_t launch_dxg256(const BwdArgs& a, const Dw256Plan& p, hipStream_t st) {
+  return a.bf16 ? launch_dxg256_t<true>(a, p, st) : launch_dxg256_t<false>(a, p, st);
 }
 
 template <bool BF16, bool HILO>

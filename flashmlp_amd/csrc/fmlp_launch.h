@@ -168,15 +168,21 @@ hipError_t launch_bwd_d64(const BwdArgs& a, const BwdPlan& p, hipStream_t st);
 hipError_t launch_bwd_d32(const BwdArgs& a, const BwdPlan& p, hipStream_t st);  // D = 32 and 16
 // dX alone at D = 256 (dense 16-bit): the tuned dX programs
 hipError_t launch_dx256(const BwdArgs& a, hipStream_t st);
-// dW alone at D = 256 (dense 16-bit): n = H nE nS programs (nE E-tiles of 128
-// columns, nS B ranges of rows_per_split rows), whose fp32 partials take ws_bytes of workspace
-// when nS > 1 (a split needing more than max_ws bytes is not taken)
+// dW at D = 256 (dense 16-bit): n = H nE nS programs (nE E-tiles of 128 columns, nS B ranges of
+// rows_per_split rows), whose fp32 partials are at the start of the workspace when nS > 1 (a split
+// needing more than max_ws bytes is not taken). dz (the stored-dZ form, when max_ws holds it as
+// well): the programs also store dZ at dz_off, from which launch_dxg256 computes dX. ws_bytes: all
+// of it; the split does not depend on dz_mode.
 struct Dw256Plan {
   int nE, nS, rows_per_split;
   long long n;
   size_t ws_bytes;
+  bool dz;
+  int Bp;
+  size_t dz_off;
 };
-Dw256Plan plan_dw256(int64_t H, int64_t B, int64_t E, bool hilo, int num_cus, size_t max_ws);
+Dw256Plan plan_dw256(int64_t H, int64_t B, int64_t E, bool hilo, int dz_mode, int num_cus, size_t max_ws);
+hipError_t launch_dxg256(const BwdArgs& a, const Dw256Plan& p, hipStream_t st);
 hipError_t launch_dw256(const BwdArgs& a, const Dw256Plan& p, hipStream_t st);
 
 // Completion time of n1 programs of t1 dealt round-robin over N slots, followed by n2 programs of

@@ -176,9 +176,9 @@ int fmlp_fwd_strided_ws(const void* x, const void* w1, const void* w2, void* o, 
  * FMLP_BWD_NO_DX leaves only the dW programs' partials, FMLP_BWD_NO_DW only the split ragged dX
  * tiles' partials, 0 where the plan splits none): query it with the flags of the call it is for. For
  * shapes the tuned kernels do not take, it is the fp32 partials of the generic dW programs'
- * B split (16-bit D = 256 with E % 8 == 0: the larger of that and the D = 256 dW programs'
- * split); those calls (and fmlp_bwd_strided calls whose views send a tuned shape to the
- * generic kernels) accept any workspace, NULL included, and split B only as far as it fits. */
+ * B split (16-bit D = 256: the larger of that and the D = 256 dW programs' split with the stored dZ;
+ * what other shapes of fmlp_shape_dense can use likewise); those calls (and fmlp_bwd_strided calls
+ * with views) accept any workspace, NULL included, and split B only as far as it fits. */
 size_t fmlp_bwd_workspace_bytes(int64_t H, int64_t B, int64_t D, int64_t E, int dtype);
 
 /* 1 when fmlp_bwd takes the stored-dZ form for these shapes, dtype flags and activation on the
@@ -194,9 +194,9 @@ int fmlp_bwd_stores_dz(int64_t H, int64_t B, int64_t D, int64_t E, int dtype, in
  * split-tile dX programs, workspace bytes, the activation's code, and the E-columns per dW
  * program (128 or 64). With FMLP_BWD_NO_DX or FMLP_BWD_NO_DW it describes what such a call
  * launches (the dW programs alone, or the dX programs alone over whole tiles) and the workspace
- * it needs. Also for dense 16-bit D = 256 with E % 8 == 0 (the D = 256 dX and dW
- * programs, one launch each; the split as with an unlimited workspace, which such calls take
- * only as far as their workspace holds). Returns FMLP_OK, or FMLP_ERR_UNSUPPORTED for shapes
+ * it needs. Also for dense 16-bit D = 256 with E % 8 == 0 (the D = 256 dX and dW programs, one
+ * launch each, or dX from the stored dZ; the split and the form as with an unlimited workspace,
+ * which such calls take only as far as their workspace holds). Returns FMLP_OK, or FMLP_ERR_UNSUPPORTED for shapes
  * the generic kernels take. No counterpart in the reference: a diagnostic for tests and
  * benches. */
 int fmlp_bwd_plan(int64_t H, int64_t B, int64_t D, int64_t E, int dtype, int act, int64_t* info, int n_info);

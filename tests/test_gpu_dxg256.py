@@ -1,0 +1,41 @@
+"""The stored-dZ form at D = 256 (dw256_kernel storing dZ, dxg256_kernel): the same bits as the
+recomputing programs in every output, from a workspace that starts as NaN, at the edges of the
+128-row tiles, the 256-row dZ blocks, the chunks of E and a B split."""
+import pytest
+import torch
+
+from flashmlp_amd import _lib
+from oracle.inputs import make_inputs
+from test_gpu_odd_e import _DT, _bwd
+
+pytestmark = pytest.mark.gpu
+
+CASES = [(2, 1, 8), (3, 127, 136), (2, 128, 96), (1, 129, 45), (5, 300, 264), (2, 2100, 1000), (9, 513, 32)]
+
+
+@pytest.mark.parametrize("H,B,E", CASES)
+@pytest.mark.parametrize("dt,act", [(torch.bfloat16, "silu"), (torch.float16, "leaky_relu"), (torch.float16, "sigmoid"),
+                                    (torch.bfloat16, "")], ids=["bf16-silu", "fp16-leaky", "fp16-sigmoid", "bf16-linear"])
+def test_same_bits_as_the_recompute_form(H, B, E, dt, act):
+    print(f"[dxg256] H={H} B={B} E={E} {dt} act='{act}'", flush=True)
+    L = _lib.lib()
+    D, code = 256, _DT[dt]
+    x, w1, w2, do = (t.cuda() for t in make_inputs(H, B, D, E, dt, seed=B + E))
+    assert L.fmlp_bwd_stores_dz(H, B, D, E, code, _lib.ACT_CODES[act]) == 1
+    assert L.fmlp_bwd_stores_dz(H, B, D, E, code | _lib.FMLP_BWD_RECOMPUTE, _lib.ACT_CODES[act]) == 0
+    need = H * -(-E // 128) * 128 * -(-B // 256) * 256 * 2
+    for mode in (0, _lib.FMLP_DW_HILO):
+        for out in (_lib.FMLP_OUT_F32, 0):
+            f = mode | out
+            odt = torch.float32 if out else dt
+            n = L.fmlp_bwd_workspace_bytes(H, B, D, E, code | f)
+            nr = L.fmlp_bwd_workspace_bytes(H, B, D, E, code | f | _lib.FMLP_BWD_RECOMPUTE)
+            assert n >= need and nr <= n
+            stored = _bwd(x, w1, w2, do, act, f, n, odt)
+            rec = _bwd(x, w1, w2, do, act, f | _lib.FMLP_BWD_RECOMPUTE, nr, odt)
+            for name, a, b in zip(("dx", "dw1", "dw2"), stored, rec):
+                assert torch.isfinite(a).all() and torch.equal(a, b), (name, hex(f))
+    # a workspace that holds no dZ (E % 8 != 0: W1's padded copy alone): the recompute form
+    n = (H * D * -(-E // 8) * 8 * 2 + 255) // 256 * 256 if E % 8 else 0
+    for a, b in zip(_bwd(x, w1, w2, do, act, 0, n, dt), _bwd(x, w1, w2, do, act, _lib.FMLP_BWD_RECOMPUTE, n, dt)):
+        assert torch.equal(a, b)
