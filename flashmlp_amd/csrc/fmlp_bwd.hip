@@ -1389,6 +1389,146 @@ dxg_kernel(const u16* __restrict__ dzt, const u16* __restrict__ W1, void* __rest
 }
 
 // ------------------------------------------------------------------------------------
+// The same product for grids that leave CUs idle (dxgs_kernel): dxg_kernel walks all of E with 512
+// (256) rows per workgroup, so a few tiles are one long chain of load latencies. Here a workgroup
+// owns 64 rows and its four waves a quarter of the E-chunks each, streamed through an LDS ring of
+// the wave's own (dZ 4 KB and W1c 64 D bytes per chunk, three slots, two chunks ahead) without
+// barriers; the four partial tiles are added through LDS in part order. Measured (SiLU backward,
+// dxg_kernel -> this): H=8 B=33 D=128 E=1024 40 -> 18.5 us, H=2 B=512 55 -> 34, H=4 B=1024 E=2048
+// 90 -> 55, H=1 B=4096 D=64 E=2048 77 -> 40, H=16 B=2048 E=512 (512 workgroups) 59 -> 55; H=8
+// B=8192 E=1024 (1024) 123 -> 137, hence at most two rounds of workgroups (small_dxg).
+// ------------------------------------------------------------------------------------
+constexpr int DXGS_EP = 4;      // E parts = waves
+constexpr int DXGS_ROWS = 64;
+constexpr int DXGS_NSLOT = 3;
+template <int D>
+__host__ __device__ constexpr int dxgs_slot() { return 4096 + 64 * D; }  // bytes: two dZ sub-blocks, then W1c
+template <int D>
+constexpr int dxgs_lds() {  // the rings; the partial tiles reuse them
+  return std::max(DXGS_EP * DXGS_NSLOT * dxgs_slot<D>(), DXGS_EP * 2 * (D / 32) * 4096);
+}
+
+template <bool BF16, int D>
+__global__ void __launch_bounds__(DXGS_EP * 64) __attribute__((amdgpu_waves_per_eu(1, 1)))
+dxgs_kernel(const u16* __restrict__ dzt, const u16* __restrict__ W1, void* __restrict__ dX, int B, int Bp, int E,
+            int ldw, int Ep, int tiles_per_head, int outf32) {
+  constexpr int NTN = D / 32, SLOT = dxgs_slot<D>(), NW1 = D / 16;  // 1 KB pieces of W1c
+  constexpr int NLD = 4 + NW1;                                      // loads per chunk
+  static_assert(2 * NLD < 64, "vmcnt");
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int part = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int G = lane >> 4, i16 = lane & 15, g = lane >> 5, l32 = lane & 31;
+  const int t = xcd_remap(blockIdx.x, gridDim.x);
+  const int h = t / tiles_per_head, bt = t - h * tiles_per_head;
+  const int NC = (E + 31) >> 5;
+  const int c0 = part * NC / DXGS_EP, n = (part + 1) * NC / DXGS_EP - c0;  // this part's chunks
+  // the tile is sub-blocks 2 (bt % 4) and + 1 of its 256-row dZ block; a chunk of a block is 8192 elements
+  const u16* zb = dzt + ((size_t)h * Bp + (size_t)(bt >> 2) * DX2_ROWS) * Ep + (size_t)(bt & 3) * 2048;
+  const u16* W1h = W1 + (size_t)h * D * ldw;
+  const int ring = part * DXGS_NSLOT * SLOT;
+  // W1c piece 64 k + lane: row 16 k + lane / 4, chunk (lane % 4) ^ ((row / 4) % 4) (the same for all k)
+  const int wq = (lane & 3) ^ ((lane >> 4) & 3);
+  const unsigned wOff = (unsigned)((lane >> 2) * ldw * 2 + wq * 16);
+  auto dma = [&](int k) {  // chunk k of the part; past the last nothing is loaded (the counts stay exact)
+    const int c = c0 + k, slot = ring + (k % DXGS_NSLOT) * SLOT;
+    const bool live = k < n;
+    const i32x4 rz = make_rsrc_words(zb + (size_t)c * 8192, live ? 4096 : 0);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) buf_load16_lds_nt(rz, (unsigned)(i * 1024 + lane * 16), slot + i * 1024);
+    const int lim = live ? E - c * 32 : 0, rem = D * ldw * 2 - 64 * c;
+    const i32x4 rw = make_rsrc_words(W1h + (size_t)c * 32, live && rem > 0 ? rem : 0);
+#pragma unroll
+    for (int i = 0; i < NW1; ++i)
+      buf_load16_lds(rw, wq * 8 < lim ? wOff + (unsigned)(i * 32 * ldw) : BUF_OOB, slot + 4096 + i * 1024);
+  };
+  const int laneA = (8 * g + (i16 >> 2)) * 64 + 32 * (G & 1) + 8 * (i16 & 3);
+  int offB[2];
+#pragma unroll
+  for (int s2 = 0; s2 < 2; ++s2) offB[s2] = 4096 + l32 * 64 + (((2 * s2 + g) ^ ((l32 >> 2) & 3)) << 4);
+
+  f32x16 acc[2][NTN];
+#pragma unroll
+  for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+    for (int nt = 0; nt < NTN; ++nt) acc[rb][nt] = zero16();
+  dma(0);
+  dma(1);
+  for (int k = 0; k < n; ++k) {
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // the reads of chunk k - 1, whose slot chunk k + 2 takes
+    asm volatile("" ::: "memory");
+    dma(k + 2);
+    wait_vmcnt<2 * NLD>();  // chunk k has landed
+    asm volatile("" ::: "memory");
+    const int base = ring + (k % DXGS_NSLOT) * SLOT;
+#pragma unroll
+    for (int s2 = 0; s2 < 2; ++s2) {
+      u32x4 a[2], b[NTN];
+#pragma unroll
+      for (int rb = 0; rb < 2; ++rb)
+        a[rb] = cat(lds_read_tr(base + laneA + rb * 2048 + s2 * 1024),
+                    lds_read_tr(base + laneA + rb * 2048 + s2 * 1024 + 256));
+#pragma unroll
+      for (int nt = 0; nt < NTN; ++nt) b[nt] = lds_read16(base + offB[s2] + nt * 2048);
+#pragma unroll
+      for (int nt = 0; nt < NTN; ++nt)
+#pragma unroll
+        for (int rb = 0; rb < 2; ++rb) acc[rb][nt] = mfma<BF16>(b[nt], a[rb], acc[rb][nt]);
+    }
+  }
+  wait_vmcnt<0>();  // loads past the last chunk are still landing
+  asm volatile("" ::: "memory");
+  __syncthreads();
+  // partial tiles: part p at p 2 NTN 4096, tile (rb, nt) 4 x [64 lanes][16 bytes]
+#pragma unroll
+  for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+    for (int nt = 0; nt < NTN; ++nt)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        lds_write16(((part * 2 + rb) * NTN + nt) * 4096 + (q * 64 + lane) * 16,
+                    u32x4{__float_as_uint(acc[rb][nt][4 * q]), __float_as_uint(acc[rb][nt][4 * q + 1]),
+                          __float_as_uint(acc[rb][nt][4 * q + 2]), __float_as_uint(acc[rb][nt][4 * q + 3])});
+  __syncthreads();
+  // the wave sums tiles part, part + 4, ... of the 2 NTN (rb NTN + nt) and stores them
+  const int row0 = bt * DXGS_ROWS, rows = clamp0(B - row0, DXGS_ROWS), es = outf32 ? 4 : 2;
+  const Rsrc ro = make_rsrc((const char*)dX + ((size_t)h * B + row0) * D * es, rows * D * es);
+#pragma unroll
+  for (int u = 0; u < 2 * NTN / DXGS_EP; ++u) {
+    const int tl = part + DXGS_EP * u, rb = tl / NTN, nt = tl - rb * NTN;
+    float v[16];
+#pragma unroll
+    for (int pp = 0; pp < DXGS_EP; ++pp)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const u32x4 x = lds_read16((pp * 2 * NTN + tl) * 4096 + (q * 64 + lane) * 16);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[4 * q + j] = pp == 0 ? __uint_as_float(x[j]) : v[4 * q + j] + __uint_as_float(x[j]);
+      }
+    // lane l32 holds row sig(l32) of the sub-block, columns 32 nt + 8 q + 4 g + 0..3
+    const unsigned r = (unsigned)(rb * 32) + sig((unsigned)l32);
+    if (outf32) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const u32x4 x = {__float_as_uint(v[4 * q]), __float_as_uint(v[4 * q + 1]), __float_as_uint(v[4 * q + 2]),
+                         __float_as_uint(v[4 * q + 3])};
+        __builtin_amdgcn_raw_buffer_store_b128(x, ro, (int)((r * D + 32 * nt + 8 * q + 4 * g) * 4u), 0, 0);
+      }
+    } else {
+      u32x2 w[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) w[q] = u32x2{pack2<BF16>(v[4 * q], v[4 * q + 1]), pack2<BF16>(v[4 * q + 2], v[4 * q + 3])};
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        const auto s0 = __builtin_amdgcn_permlane32_swap(w[2 * p][0], w[2 * p + 1][0], false, false);
+        const auto s1 = __builtin_amdgcn_permlane32_swap(w[2 * p][1], w[2 * p + 1][1], false, false);
+        const u32x4 x = {s0[0], s1[0], s0[1], s1[1]};
+        __builtin_amdgcn_raw_buffer_store_b128(x, ro, (int)((r * D + 32 * nt + 16 * p + 8 * g) * 2u), 0, 0);
+      }
+    }
+  }
+}
+
+// ------------------------------------------------------------------------------------
 // dX from the stored dZ at D = 256 (dxg256_kernel): a workgroup owns 128 rows of one head (half of
 // a 256-row dZ block), 8 waves = 2 groups of 64 rows x 4 quarters of the columns, so that the
 // four accumulator tiles and operands of a wave leave room for four waves per SIMD (two
@@ -1557,6 +1697,7 @@ constexpr double kPlanHbmBytesPerUs = 5.0e6;
 constexpr double kPlanLaunchUs = 4.0;
 constexpr double kPlanDzBytesPerUs = 4.9e6;  // stored-dZ form: dZ bytes per time unit (store + reload)
 constexpr double kPlanDzFixedUs = 5.0;
+constexpr double kPlanDxgsBytesPerUs = 4.2e6;
 
 // VALU instructions per element of the activation plane (dX role: act'; dW role: act and act')
 double valu_dx(int act) { return act == ACT_SILU ? 8.5 : act == ACT_SIGMOID ? 6.5 : act == ACT_LEAKY ? 3.0 : 1.0; }
@@ -1567,6 +1708,9 @@ long long rows_for_split(long long B, long long ns) {
   rps = (rps + DW_BT - 1) / DW_BT * DW_BT;
   return rps < DW_BT ? (long long)DW_BT : rps;
 }
+
+// the dX GEMM for grids that leave CUs idle: at most two rounds of its 64-row workgroups
+bool small_dxg(int64_t H, int64_t B, long long N) { return H * ((B + DXGS_ROWS - 1) / DXGS_ROWS) <= 2 * N; }
 
 BwdPlan make_plan(int64_t H, int64_t B, int64_t D, int64_t E, int act, bool hilo, int dz_mode, int num_cus,
                   size_t max_ws) {
@@ -1713,7 +1857,11 @@ BwdPlan make_plan(int64_t H, int64_t B, int64_t D, int64_t E, int act, bool hilo
   double best_dz = 0.0;
   long long best_dz_ns = 1;
   if (dz_want != 0 && D >= 64 && B > 0 && dz_head < ((size_t)1 << 31)) {
-    const double t_dx = kPlanDzFixedUs + (double)H * dz_head / kPlanDzBytesPerUs;
+    double t_dx = kPlanDzFixedUs + (double)H * dz_head / kPlanDzBytesPerUs;
+    // dxgs_kernel reads the head's whole W1 for every 64 rows (fitted on 14 small grids: the form picked
+    // is the faster one or within 5 % of it, H=8 B=1024 D=128 E=1024 recompute 37 / stored 46 us and
+    // H=4 B=1024 E=2048 66 / 55 us among them)
+    if (small_dxg(H, B, N)) t_dx += (double)H * ((B + DXGS_ROWS - 1) / DXGS_ROWS) * E * D * 2.0 / kPlanDxgsBytesPerUs;
     for (long long ns = 1; ns <= (ns_env > 0 ? 1 : cap); ns *= 2) {
       const long long want = ns_env > 0 ? (ns_env < max_ns ? ns_env : max_ns) : ns;
       const long long rps = rows_for_split(B, want), eff = B > rps ? (B + rps - 1) / rps : 1;
@@ -1759,6 +1907,9 @@ BwdPlan make_plan(int64_t H, int64_t B, int64_t D, int64_t E, int act, bool hilo
     // dxg_kernel is persistent: one workgroup per CU (a multiple of 8, the XCD count), at most
     // one per tile
     p.n_xg = (int)std::min<long long>(p.n_dx, std::max<long long>(8, N / 8 * 8));
+    // FMLP_DXGS (read once per process) forces the small-grid GEMM on (1) or off (0)
+    static const int dxgs_env = env_int("FMLP_DXGS", -1);
+    p.dxgs = dxgs_env >= 0 ? dxgs_env == 1 : small_dxg(H, B, N);
   }
   return p;
 }
@@ -1898,6 +2049,17 @@ static hipError_t launch_bwd_t(const BwdArgs& a, const BwdPlan& p, hipStream_t s
     e = a.dw_hilo ? launch_w(dw2_kernel<BF16, D, ACT, true, true>) : launch_w(dw2_kernel<BF16, D, ACT, false, true>);
     if (e != hipSuccess) return e;
     if ((e = reduce()) != hipSuccess) return e;
+    if (p.dxgs) {
+      const long long tph = (a.B + DXGS_ROWS - 1) / DXGS_ROWS, grid = tph * a.H;
+      if (grid <= 0) return hipSuccess;
+      auto k = dxgs_kernel<BF16, D>;
+      static std::atomic<unsigned long long> lds_set{0};
+      if ((e = set_lds_once((const void*)k, dxgs_lds<D>(), lds_set)) != hipSuccess) return e;
+      hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(DXGS_EP * 64), dxgs_lds<D>(), st, (const u16*)dzt,
+                         (const u16*)a.w1, a.dx, (int)a.B, p.Bp, (int)a.E, (int)a.ldw, Ep, (int)tph,
+                         a.out_f32 ? 1 : 0);
+      return hipGetLastError();
+    }
     // FMLP_DXG_TP (read once per process): 256-row blocks per dX GEMM tile, 2 (default) or 1
     static const int tp_env = env_int("FMLP_DXG_TP", 2);
     auto launch_g = [&](auto kg, int TP) {

@@ -78,6 +78,7 @@ struct BwdPlan {
   bool dz;             // stored-dZ form
   int Bp;              // B rounded up to 256 (dZ tiles), stored-dZ form
   int n_xg;            // dxg_kernel workgroups (persistent), stored-dZ form
+  bool dxgs;           // stored-dZ form: the dX GEMM for small grids (dxgs_kernel)
   size_t dz_off;       // byte offset of dZ in the workspace, stored-dZ form
   size_t ws_bytes;     // fp32 partials when nS > 1, then dZ (H nE 128 Bp io elements) when dz
   size_t dw_ws_bytes;  // the fp32 partials alone (at offset 0): what the dW programs need by themselves
