@@ -31,12 +31,13 @@ namespace fmlp {
 //   W2c  [D/32][32][32]    block nt, row e = W2[h][32c + e][32nt .. 32nt+31]
 // Waves per workgroup: one 32-row M-tile each, so that the workgroup's threads cover a chunk's
 // 4 D pieces of W1c and of W2c exactly once (NT == 4 D); two waves per SIMD either way.
-// ES = 2 (E split, D = 64 only, for grids that leave CUs idle): the workgroup holds two such
+// ES = 2 (E split, D = 64, for grids that leave CUs idle): the workgroup holds two such
 // sets of waves on the same rows, each walking half of the E-chunks through a ring of its own
 // (one workgroup per CU, two waves per SIMD instead of one); the two partial O tiles are added
 // through LDS at the end. ES = 4 with NWP = 2 (D = 64, smaller grids still): 64-row tiles, four
 // sets of two waves, each walking a quarter of the E-chunks through a 4-slot ring of its own;
-// the partial tiles are added in part order.
+// the partial tiles are added in part order. ES = 2 with NWP = 4 at D = 128: 128-row tiles, two sets of
+// four waves, 4-slot rings, for grids that leave half the CUs idle (small_grid).
 // Split tiles (fwd_plan): the last n_split tiles in row-block-major order (tile (h, bt) at
 // bt H + h; the ragged last tiles of the heads first) are split; the first n_main workgroups
 // each own one of the other tiles, enumerated head by head (split_tile / main_tile); every later
@@ -72,10 +73,10 @@ __host__ __device__ constexpr int fwd_waves(int D) { return D > 32 && D <= 128 ?
 __host__ __device__ constexpr int fwd_wpe(int D, int OC) { return D <= 128 ? OC : 1; }
 // ring geometry: slots (chunks of 128 D bytes), chunk iterations per workgroup barrier and chunks
 // loaded ahead; at D = 256 a chunk is 32 KB, so four slots, a barrier per chunk, two ahead, and
-// the same for the 4-slot rings of the higher-occupancy D = 64 builds
+// the same for the 4-slot rings of the higher-occupancy D = 64 builds and of the E parts at D = 128
 constexpr int FWD_PF = 4;  // chunks loaded ahead with one barrier per chunk (D <= 128)
 __host__ __device__ constexpr bool fwd_small_ring(int D, int OC, int ES = 1) {
-  return D > 128 || (D > 32 && OC > 2) || ES > 2;
+  return D > 128 || (D > 32 && OC > 2) || ES > 2 || (D > 64 && ES > 1);
 }
 __host__ __device__ constexpr int fwd_nslot(int D, int OC, int ES = 1) { return fwd_small_ring(D, OC, ES) ? 4 : 8; }
 __host__ __device__ constexpr int fwd_sb(int D, int OC, int ES = 1) { return fwd_small_ring(D, OC, ES) ? 1 : 2; }
@@ -98,9 +99,10 @@ fwd_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* __r
   constexpr int KS = DG / 16;          // K steps of GEMM1 (at DG = D also GEMM2's operand count 2 * D/32)
   constexpr int NTN = D / 32;          // N tiles of GEMM2
   constexpr int BB = NW * 32;          // rows per workgroup (32 per wave)
-  static_assert(ES == 1 || (ES == 2 && D <= 64) || (ES == 4 && D <= 64 && NWP == 2), "E split");
+  static_assert(ES == 1 || (ES == 2 && D <= 64) || (ES == 2 && D == 128 && NWP == 4) ||
+                (ES == 4 && D <= 64 && NWP == 2), "E split");
   static_assert(DG == D || (DG == 16 && D == 32), "columns in memory");
-  static_assert(NWP == fwd_waves(D) || (NWP == 2 && ES == 4), "waves per E part");
+  static_assert(NWP == fwd_waves(D) || (NWP == 2 && ES == 4) || (D == 128 && ES == 2), "waves per E part");
   constexpr unsigned SLOT = 128u * D;  // bytes per ring slot: W1c (64*D) + W2c (64*D)
   constexpr unsigned W2OFF = 64u * D;
   // SB: chunk iterations per workgroup barrier. The loads run SB - 1 chunks further ahead so
@@ -141,12 +143,12 @@ fwd_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* __r
   }
   const int h = tile.h, bt = tile.bt;
   // chunks of this part: global chunk c0 + c for c = 0 .. NC - 1 (the last part's last chunks
-  // may lie past the range: they load as zeros and add nothing). At D < 64 the parts' shares differ
-  // by at most one, and a part with a chunk less leaves the product of its last step out, so that
-  // a NaN which an infinite X makes of those zeros is not added.
+  // may lie past the range: they load as zeros and add nothing). Except at D = 64 the parts' shares
+  // differ by at most one, and a part with a chunk less leaves the product of its last step out, so
+  // that a NaN which an infinite X makes of those zeros is not added.
   const int NC = (ce - cb + ES - 1) / ES;
-  const int c0 = D < 64 ? cb + part * (ce - cb) / ES : cb + part * NC;
-  const int c1 = ES > 1 && D < 64 ? cb + (part + 1) * (ce - cb) / ES : ce;
+  const int c0 = D != 64 ? cb + part * (ce - cb) / ES : cb + part * NC;
+  const int c1 = ES > 1 && D != 64 ? cb + (part + 1) * (ce - cb) / ES : ce;
   const int e_end = min(E, c1 * 32);  // columns of W1 (rows of W2) this workgroup reads
   const unsigned RB = (unsigned)part * NSLOT * 128u * D;  // this part's ring
 
@@ -309,7 +311,7 @@ fwd_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* __r
     if constexpr (decltype(SYNC)::value) chunk_end();
   };
   auto last_gemm2 = [&](const St& st) {
-    if (ES > 1 && D < 64 && c0 + NC > c1) return;
+    if (ES > 1 && D != 64 && c0 + NC > c1) return;
     const unsigned base2 = RB + rslot(NC - 1) * SLOT;
 #pragma unroll
     for (int s = 0; s < 2; ++s)
@@ -476,9 +478,48 @@ hipError_t launch_pad_w1(const void* w1, void* dst, int64_t H, int64_t D, int64_
 // set with the in-workgroup split); the parts' fp32 partials go to the caller's workspace and
 // a second launch sums them. At D = 64 the full round then runs with the in-workgroup split
 // (one tile per CU). Measured on MI355X at H=8 B=4097 D=64 E=2048: 43.9 us unsplit, 33.0 us
-// for the split launch. Small grids (fewer tiles than CUs) gain nothing from it: their tiles'
-// time is mostly fixed latency (12.5 vs 11.4 us at H=12 B=1024 D=64 E=768, before the sum).
+// for the split launch. At D = 64 small grids (fewer tiles than CUs) gain nothing from it: their
+// tiles' time is mostly fixed latency (12.5 vs 11.4 us at H=12 B=1024 D=64 E=768, before the sum).
+// At D = 128 and 256 a tile's chunk takes 0.7 / 0.85 us, so there (small_grid) grids that leave half
+// the CUs idle are split.
 // FMLP_FWD_XS=0 (read once per process) turns the cross-workgroup split off.
+// D = 128 and 256, at most N / 2 tiles of BB rows: D = 128 takes 128-row tiles of two E parts per
+// workgroup; every tile is then split over xs workgroups where the chunks saved are worth more than
+// the sum's launch and the partials (H B D fp32 per part, written and read at about 2 MB/us).
+// A lone round of whole tiles costs its chunks one after the other, however few tiles there are.
+// Forward, bf16 SiLU, whole tiles -> 128-row tiles -> split over workgroups: D = 128 H=1 B=33 E=2048
+// 48.6 -> 29.1 -> 8.9 us, H=8 B=512 E=2048 50.6 -> 30.8 -> 19.0, H=8 B=1024 E=1024 27.9 -> 18.4 -> not
+// split, H=8 B=2048 E=512 16.9 -> 12.2, E=128 8.3 -> 7.5; D = 256 H=1 B=33 E=1024 31.7 -> 9.8 split, H=8
+// B=1024 E=2048 60.8 -> 34.7, H=8 B=2048 E=1024 34.6 either way (not split).
+static void small_grid(FwdPlan& p, int64_t H, int64_t B, int64_t D, int64_t nch, long long N, size_t max_ws,
+                       bool parts, bool across) {
+  const double chunk_us = D == 128 ? 0.71 : 0.85;
+  long long BB = 32 * fwd_waves((int)D), R = p.n_main;
+  if (parts && D == 128 && nch >= 2) {
+    BB = 128;
+    R = H * ((B + BB - 1) / BB);
+    p.es = 2;
+    p.nwp = 4;
+    p.n_main = R;
+  }
+  if (!across) return;
+  const auto time = [&](long long nct) { return chunk_us * (double)((nct + p.es - 1) / p.es); };
+  double best = time(nch) - 1.0;  // the estimate's margin
+  const long long cap = std::min<long long>(std::min<long long>(N / R, nch / (2 * p.es)), FWD_XS_MAX);
+  for (long long want = 2; want <= cap; ++want) {
+    const long long nct = (nch + want - 1) / want, xs = (nch + nct - 1) / nct;
+    const size_t ws = (size_t)R * (size_t)xs * (size_t)BB * (size_t)D * sizeof(float);
+    const double t = time(nct) + 3.0 + (double)(H * B * D * xs) * 4.0 / 2.0e6;
+    if (xs < 2 || ws > max_ws || t >= best) continue;
+    best = t;
+    p.n_main = 0;
+    p.n_split = (int)R;
+    p.xs = (int)xs;
+    p.nct = (int)nct;
+    p.ws_bytes = ws;
+  }
+}
+
 FwdPlan fwd_plan(int64_t H, int64_t B, int64_t D, int64_t E, int num_cus, size_t max_ws) {
   FwdPlan p{};
   const long long BB = 32 * fwd_waves((int)D), T = (B + BB - 1) / BB, R = H * T, N = num_cus > 0 ? num_cus : 1;
@@ -503,6 +544,10 @@ FwdPlan fwd_plan(int64_t H, int64_t B, int64_t D, int64_t E, int num_cus, size_t
     p.es = 4;
     p.nwp = 2;
     p.n_main = R64;
+    return p;
+  }
+  if (D >= 128 && R > 0 && 2 * R <= N) {
+    small_grid(p, H, B, D, nch, N, max_ws, force != 0, xs_env != 0);
     return p;
   }
   if (xs_env == 0 || R <= 0 || D < 64) return p;  // (four D < 64 workgroups share a CU: rounds are short)
@@ -586,6 +631,9 @@ static hipError_t launch_fwd_t(const FwdArgs& a, hipStream_t st) {
     if (p.es == 2) return launch_fwd_e<BF16, D, ACT, 2, 2, fwd_waves(D), DG>(a, p, tiles_per_head, st);
     return launch_fwd_e<BF16, D, ACT, 1, 4, fwd_waves(D), DG>(a, p, tiles_per_head, st);
   } else {
+    if constexpr (D == 128) {
+      if (p.es == 2) return launch_fwd_e<BF16, D, ACT, 2, 2, 4>(a, p, tiles_per_head, st);
+    }
     return launch_fwd_e<BF16, D, ACT, 1>(a, p, tiles_per_head, st);
   }
 }

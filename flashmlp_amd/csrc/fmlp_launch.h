@@ -48,7 +48,7 @@ struct FwdArgs {
 // needing more than max_ws bytes is not taken.
 struct FwdPlan {
   int es;
-  int nwp = 0;  // waves per E part (32 rows each): 0 = fwd_waves(D); 2 = 64-row tiles (D = 64, es = 4)
+  int nwp = 0;  // waves per E part (32 rows each): 0 = fwd_waves(D); 2 = 64-row tiles (D <= 64, es = 4); 4 = 128-row tiles (D = 128, es = 2)
   long long n_main;
   int n_split, xs, nct;
   size_t ws_bytes;
