@@ -503,6 +503,7 @@ static void small_grid(FwdPlan& p, int64_t H, int64_t B, int64_t D, int64_t nch,
     p.n_main = R;
   }
   if (!across) return;
+  const FwdPlan whole = p;
   const auto time = [&](long long nct) { return chunk_us * (double)((nct + p.es - 1) / p.es); };
   double best = time(nch) - 1.0;  // the estimate's margin
   const long long cap = std::min<long long>(std::min<long long>(N / R, nch / (2 * p.es)), FWD_XS_MAX);
@@ -510,7 +511,7 @@ static void small_grid(FwdPlan& p, int64_t H, int64_t B, int64_t D, int64_t nch,
     const long long nct = (nch + want - 1) / want, xs = (nch + nct - 1) / nct;
     const size_t ws = (size_t)R * (size_t)xs * (size_t)BB * (size_t)D * sizeof(float);
     const double t = time(nct) + 3.0 + (double)(H * B * D * xs) * 4.0 / 2.0e6;
-    if (xs < 2 || ws > max_ws || t >= best) continue;
+    if (xs < 2 || t >= best) continue;
     best = t;
     p.n_main = 0;
     p.n_split = (int)R;
@@ -518,6 +519,7 @@ static void small_grid(FwdPlan& p, int64_t H, int64_t B, int64_t D, int64_t nch,
     p.nct = (int)nct;
     p.ws_bytes = ws;
   }
+  if (p.ws_bytes > max_ws) p = whole;  // a smaller workspace: fmlp_fwd's result
 }
 
 FwdPlan fwd_plan(int64_t H, int64_t B, int64_t D, int64_t E, int num_cus, size_t max_ws) {

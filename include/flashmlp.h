@@ -148,7 +148,8 @@ size_t fmlp_fwd_workspace_bytes(int64_t H, int64_t B, int64_t D, int64_t E, int 
 /* fmlp_fwd with a device workspace (16-byte aligned, or NULL). No counterpart in the reference,
  * whose forward allocates only o: with at least fmlp_fwd_workspace_bytes() bytes, a grid whose
  * last round of tiles would leave most CUs idle (a short last round after full ones, e.g. a
- * ragged B just past a multiple of the CU count) splits those tiles over E across workgroups.
+ * ragged B just past a multiple of the CU count; at D >= 128 also a grid of few tiles) splits
+ * those tiles over E across workgroups.
  * The parts' fp32 partials go through the workspace and a second launch sums them in a fixed
  * order. With a smaller workspace or NULL it is fmlp_fwd. The workspace is scratch for the
  * duration of the call on `stream`. */

@@ -43,6 +43,9 @@ def test_small_grid_forward(H, B, D, E, dt, act):
         o = _fwd(L, xd, w1d, w2d, act, code, dt, ws, nb, fill_nan=True)
         assert torch.equal(o, s.to(dt))
         assert torch.equal(o, _fwd(L, xd, w1d, w2d, act, code, dt, ws, nb))
+    if n and E % 8 == 0:  # a workspace too small for every part: fmlp_fwd's bits
+        ws = torch.empty(n - 16, dtype=torch.uint8, device="cuda")
+        assert torch.equal(_fwd(L, xd, w1d, w2d, act, code, dt, ws, n - 16), _fwd(L, xd, w1d, w2d, act, code, dt))
 
 
 @pytest.mark.parametrize("D,E", [(128, 96), (128, 2016), (256, 96), (256, 2016)])
