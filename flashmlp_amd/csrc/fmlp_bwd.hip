@@ -1535,7 +1535,10 @@ dxgs_kernel(const u16* __restrict__ dzt, const u16* __restrict__ W1, void* __res
 // workgroups per CU, whose starts and ends overlap). Per 32-column E-chunk: dZ (8 KB, read once) and
 // W1c (16 KB, L2-resident) through a 3-slot LDS ring two chunks ahead, one barrier, and 8 MFMAs
 // per wave from 8 KB of operand reads. The products and their order are dxg_kernel's, and so the
-// bits of dX those of the recomputing programs.
+// bits of dX those of the recomputing programs. Small grids (xs > 1, plan_dw256): a tile's chunks over
+// xs workgroups, whose fp32 partial tiles launch_tile_reduce sums in part order.
+// A lone workgroup takes 0.55 us per chunk: H=1 B=33 E=2048 bf16 36.0 -> 5.6 us + 1.6-3 for the sum, H=1 B=1000
+// E=2048 40.4 -> 11.5 + 4 (kernel trace).
 // ------------------------------------------------------------------------------------
 constexpr int DXG4_ZT = 128 * 32 * 2;    // dZ chunk bytes of 128 rows
 constexpr int DXG4_WT = 64 * 256;        // W1c chunk bytes
@@ -1545,15 +1548,16 @@ constexpr int DXG4_NSLOT = 3;
 template <bool BF16>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4)))
 dxg256_kernel(const u16* __restrict__ dzt, const u16* __restrict__ W1, void* __restrict__ dX, int B, int Bp, int E,
-              int ldw, int Ep, int tiles_per_head, int outf32) {
+              int ldw, int Ep, int tiles_per_head, int H, int outf32, int xs, int nct, float* __restrict__ part) {
   constexpr int D = 256;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int G = lane >> 4, i16 = lane & 15, g = lane >> 5, l32 = lane & 31;
   const int rg = wave & 1, cq = wave >> 1;  // row group, column quarter
   const int t = xcd_remap(blockIdx.x, gridDim.x);
-  const int h = t / tiles_per_head, ht = t - h * tiles_per_head;
-  const int NC = (E + 31) >> 5;
+  const int tile = t / xs;  // xs > 1: tiles in row-block-major order, as launch_tile_reduce takes them
+  const int h = xs > 1 ? tile % H : tile / tiles_per_head, ht = xs > 1 ? tile / H : tile - h * tiles_per_head;
+  const int c0 = (t - tile * xs) * nct, c1 = min((E + 31) >> 5, c0 + nct);  // this workgroup's chunks
   // chunk c of a 256-row block is 8192 elements, this half's the 4096 at (ht & 1) 4096
   const u16* zb = dzt + ((size_t)h * Bp + (size_t)(ht >> 1) * DX2_ROWS) * Ep + (size_t)(ht & 1) * 4096;
   const u16* W1h = W1 + (size_t)h * D * ldw;
@@ -1563,7 +1567,7 @@ dxg256_kernel(const u16* __restrict__ dzt, const u16* __restrict__ W1, void* __r
   const unsigned wOff = (unsigned)(wr * ldw * 2 + wq * 16);
   auto dma = [&](int c) {  // chunks past the last load nothing
     const int slot = (c % DXG4_NSLOT) * DXG4_SLOT + wave * 1024;
-    const int lim = E - c * 32, rem = D * ldw * 2 - 64 * c;
+    const int lim = c < c1 ? E - c * 32 : 0, rem = D * ldw * 2 - 64 * c;
     buf_load16_lds_nt(make_rsrc_words(zb + (size_t)c * 8192, lim > 0 ? DXG4_ZT : 0), (unsigned)tid * 16u, slot);
     const i32x4 rw = make_rsrc_words(W1h + (size_t)c * 32, lim > 0 && rem > 0 ? rem : 0);
 #pragma unroll
@@ -1581,9 +1585,9 @@ dxg256_kernel(const u16* __restrict__ dzt, const u16* __restrict__ W1, void* __r
   for (int rb = 0; rb < 2; ++rb)
 #pragma unroll
     for (int j = 0; j < 2; ++j) acc[rb][j] = zero16();
-  dma(0);
-  dma(1);
-  for (int c = 0; c < NC; ++c) {
+  dma(c0);
+  dma(c0 + 1);
+  for (int c = c0; c < c1; ++c) {
     wait_vmcnt<3>();  // chunk c has landed (the three loads of chunk c + 1 may be in flight)
     __builtin_amdgcn_s_waitcnt(0xC07F);
     asm volatile("" ::: "memory");
@@ -1612,15 +1616,17 @@ dxg256_kernel(const u16* __restrict__ dzt, const u16* __restrict__ W1, void* __r
   // lane l32 holds row sig(l32) of each 32-row block, columns 32 nt + 8 q + 4 g + 0..3
   const int row0 = ht * 128;
   const int rows = clamp0(B - row0, 128);
-  const int es = outf32 ? 4 : 2;
-  const Rsrc ro = make_rsrc((const char*)dX + ((size_t)h * B + row0) * D * es, rows * D * es);
+  const bool f32 = outf32 || xs > 1;
+  const int es = f32 ? 4 : 2;
+  const Rsrc ro = make_rsrc(xs > 1 ? (const char*)(part + (size_t)t * (128 * D))
+                                   : (const char*)dX + ((size_t)h * B + row0) * D * es, rows * D * es);
 #pragma unroll
   for (int rb = 0; rb < 2; ++rb) {
     const unsigned r = (unsigned)((2 * rg + rb) * 32) + sig((unsigned)l32);
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const int col = (2 * cq + j) * 32;
-      if (outf32) {
+      if (f32) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           const u32x4 v = {__float_as_uint(acc[rb][j][4 * q]), __float_as_uint(acc[rb][j][4 * q + 1]),
@@ -1994,6 +2000,26 @@ Dw256Plan plan_dw256(int64_t H, int64_t B, int64_t E, bool hilo, int dz_mode, in
     p.Bp = (int)Bp;
     p.dz_off = off;
     p.ws_bytes = off + (size_t)H * dz_head;
+    // the dX GEMM's tiles split over E where they leave half the CUs idle and the chunks saved outweigh
+    // the sum's launch and the partials (fwd_plan's estimate of both; a chunk takes 0.55 us)
+    constexpr double kChunkUs = 0.55;
+    const long long T = (B + 127) / 128, R = H * T, nch = (E + 31) / 32;
+    p.xg_xs = 1;
+    p.xg_nct = (int)nch;
+    double best = 0.8 * kChunkUs * (double)nch;  // by a fifth: the estimate's error, and a launch more on the host
+    const long long cap = std::min<long long>(std::min<long long>(2 * R <= N ? N / R : 1, nch / 4), 16);
+    const size_t xoff = (p.ws_bytes + 255) / 256 * 256;
+    for (long long want = 2; want <= cap; ++want) {
+      const long long nct = (nch + want - 1) / want, xs = (nch + nct - 1) / nct;
+      const size_t need = xoff + (size_t)R * (size_t)xs * (128 * 256 * sizeof(float));
+      const double t = kChunkUs * (double)nct + 3.0 + (double)(H * B * xs) * (256 * 4.0 / 2.0e6);
+      if (xs < 2 || need > max_ws || t >= best) continue;
+      best = t;
+      p.xg_xs = (int)xs;
+      p.xg_nct = (int)nct;
+      p.xg_off = xoff;
+      p.ws_bytes = need;
+    }
   }
   return p;
 }
@@ -2214,19 +2240,22 @@ static hipError_t launch_dw256_t(const BwdArgs& a, const Dw256Plan& p, hipStream
 
 template <bool BF16>
 static hipError_t launch_dxg256_t(const BwdArgs& a, const Dw256Plan& p, hipStream_t st) {
-  const long long tph = (a.B + 127) / 128, grid = tph * a.H;
+  const long long tph = (a.B + 127) / 128, grid = tph * a.H * p.xg_xs;
   if (grid <= 0) return hipSuccess;
   if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
   constexpr int lds = DXG4_NSLOT * DXG4_SLOT;
   static_assert(lds <= 80 * 1024, "two workgroups per CU");
   auto k = dxg256_kernel<BF16>;
   static std::atomic<unsigned long long> lds_set{0};
-  const hipError_t e = set_lds_once((const void*)k, lds, lds_set);
+  hipError_t e = set_lds_once((const void*)k, lds, lds_set);
   if (e != hipSuccess) return e;
+  float* part = (float*)((char*)a.ws + p.xg_off);
   hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(512), lds, st, (const u16*)((const char*)a.ws + p.dz_off),
-                     (const u16*)a.w1, a.dx, (int)a.B, p.Bp, (int)a.E, (int)a.ldw, p.nE * DW_ET, (int)tph,
-                     a.out_f32 ? 1 : 0);
-  return hipGetLastError();
+                     (const u16*)a.w1, a.dx, (int)a.B, p.Bp, (int)a.E, (int)a.ldw, p.nE * DW_ET, (int)tph, (int)a.H,
+                     a.out_f32 ? 1 : 0, p.xg_xs, p.xg_nct, part);
+  if ((e = hipGetLastError()) != hipSuccess || p.xg_xs == 1) return e;
+  return launch_tile_reduce(part, a.dx, BF16, (int)a.B, 256, 128, (int)a.H, (int)tph, p.xg_xs, (int)(tph * a.H),
+                            a.out_f32 ? 1 : 0, st);
 }
 
 // dX from the dZ that launch_dw256 stored (p.dz)

@@ -181,6 +181,8 @@ struct Dw256Plan {
   bool dz;
   int Bp;
   size_t dz_off;
+  int xg_xs, xg_nct;  // dz: parts of E per dX tile and chunks per part (fp32 partials at xg_off when > 1)
+  size_t xg_off;
 };
 Dw256Plan plan_dw256(int64_t H, int64_t B, int64_t E, bool hilo, int dz_mode, int num_cus, size_t max_ws);
 hipError_t launch_dxg256(const BwdArgs& a, const Dw256Plan& p, hipStream_t st);

@@ -39,3 +39,27 @@ def test_same_bits_as_the_recompute_form(H, B, E, dt, act):
     n = (H * D * -(-E // 8) * 8 * 2 + 255) // 256 * 256 if E % 8 else 0
     for a, b in zip(_bwd(x, w1, w2, do, act, 0, n, dt), _bwd(x, w1, w2, do, act, _lib.FMLP_BWD_RECOMPUTE, n, dt)):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("H,B,E", [(1, 33, 2048), (1, 1000, 2048), (3, 129, 1500), (2, 300, 1355)])
+@pytest.mark.parametrize("dt,act", [(torch.bfloat16, "silu"), (torch.float16, "sigmoid")], ids=["bf16", "fp16"])
+def test_tiles_split_over_e(H, B, E, dt, act):
+    # grids that leave the chip idle: the recompute form's sums in another order, also from a
+    # workspace too short for every part
+    print(f"[dxg256-split] H={H} B={B} E={E} {dt} act='{act}'", flush=True)
+    L = _lib.lib()
+    D, code = 256, _DT[dt]
+    x, w1, w2, do = (t.cuda() for t in make_inputs(H, B, D, E, dt, seed=B + E))
+    f = _lib.FMLP_OUT_F32
+    n = L.fmlp_bwd_workspace_bytes(H, B, D, E, code | f)
+    sums = _bwd(x, w1, w2, do, act, f, n, torch.float32)
+    rec = _bwd(x, w1, w2, do, act, f | _lib.FMLP_BWD_RECOMPUTE, n, torch.float32)
+    assert all(torch.isfinite(t).all() for t in sums)
+    assert not torch.equal(sums[0], rec[0]), "the case must split its tiles"
+    assert ((sums[0] - rec[0]).norm() / rec[0].norm()).item() <= 1e-6  # the same dZ bits, E / 2 additions regrouped
+    assert torch.equal(sums[1], rec[1]) and torch.equal(sums[2], rec[2])
+    for flags in (0, _lib.FMLP_DW_HILO):  # dX does not depend on the dW mode; repeats agree
+        nf = L.fmlp_bwd_workspace_bytes(H, B, D, E, code | flags)
+        assert torch.equal(_bwd(x, w1, w2, do, act, flags, nf, dt)[0], sums[0].to(dt))
+    short = _bwd(x, w1, w2, do, act, f, n - 16, torch.float32)  # fewer parts, or none
+    assert ((short[0] - rec[0]).norm() / rec[0].norm()).item() <= 1e-6
