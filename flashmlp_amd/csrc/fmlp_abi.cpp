@@ -102,9 +102,9 @@ size_t plan_ws_bytes(const fmlp::BwdPlan& p, int dtype) {
 }
 size_t elem_bytes(int io) { return io == FMLP_DTYPE_F32 ? 4 : 2; }
 
-// The tuned kernels (fmlp_fwd.hip, fmlp_bwd.hip) take 16-bit io, D in {64, 128} and
-// E % 8 == 0 on dense, 16-byte aligned tensors; everything else within check_shape runs on the
-// generic kernels (fmlp_gen.hip).
+// The shapes of fmlp_shape_tuned: 16-bit io, D in {64, 128} and E % 8 == 0. dense_shape below has
+// every shape with kernels of its own; the rest of check_shape runs on the generic kernels
+// (fmlp_gen.hip).
 bool tuned_shape(int64_t D, int64_t E, int io) {
   return (io == FMLP_DTYPE_F16 || io == FMLP_DTYPE_BF16) && (D == 64 || D == 128) && E % 8 == 0;
 }
