@@ -1790,7 +1790,7 @@ BwdPlan make_plan(int64_t H, int64_t B, int64_t D, int64_t E, int act, bool hilo
   double best_t = 0.0;
   long long best_ns = 1;
   bool best_dx_first = false, best_dxs = false;
-  int best_des = 1, best_et = DW_ET;
+  int best_des = min_des, best_et = DW_ET;  // what is left when a forced B split fits no workspace
   for (int des = min_des; des <= max_des; ++des) {
     if (des_env > 0 && des != des_env && min_des != max_des) continue;
     if (fixed_des > 0 && des != fixed_des) continue;

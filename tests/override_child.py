@@ -9,9 +9,12 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 if ROOT not in sys.path:
     sys.path.insert(0, ROOT)
 
+import ctypes  # noqa: E402
+
 import torch  # noqa: E402
 
 import flashmlp_amd as fm  # noqa: E402
+from flashmlp_amd import _lib  # noqa: E402
 from oracle import emulate, reference  # noqa: E402
 from oracle.inputs import make_inputs  # noqa: E402
 
@@ -37,9 +40,32 @@ def _rel(a, b):
     return ((a - b).norm() / b.norm().clamp_min(1e-30)).item()
 
 
+# H, B, D, E: backwards of narrow heads given no workspace, which a forced B split does not fit
+NO_WORKSPACE = [(2, 1100, 32, 136), (2, 1100, 16, 40)]
+
+
+def _no_workspace(env):
+    bad = 0
+    for H, B, D, E in NO_WORKSPACE:
+        x, w1, w2, do = make_inputs(H, B, D, E, torch.bfloat16, seed=B + D)
+        xg, w1g, w2g, dog = (t.cuda() for t in (x, w1, w2, do))
+        outs = [torch.full_like(t, float("nan")) for t in (xg, w1g, w2g)]
+        st = _lib.lib().fmlp_bwd(*(ctypes.c_void_p(t.data_ptr()) for t in (xg, w1g, w2g, dog, *outs)), H, B, D, E,
+                                 _lib.FMLP_DTYPE_BF16, _lib.ACT_CODES["silu"], None, 0,
+                                 ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+        _lib.check(st, "backward")
+        torch.cuda.synchronize()
+        rel = [_rel(g.cpu(), r) for g, r in zip(outs, reference.autograd_grads(x, w1, w2, do, "silu")[1:])]
+        ok = max(rel) <= 1e-2  # (NaN fails too)
+        bad += not ok
+        print(f"[{env}] no workspace H={H} B={B} D={D} E={E}: dx, dw1, dw2 normwise {rel} {'ok' if ok else 'MISS'}",
+              flush=True)
+    return bad
+
+
 def main():
     env = " ".join(f"{k}={v}" for k, v in sorted(os.environ.items()) if k.startswith("FMLP_"))
-    bad = 0
+    bad = _no_workspace(env)
     for i, (H, B, D, E, dt, act, kw) in enumerate(CASES):
         x, w1, w2, do = make_inputs(H, B, D, E, dt, seed=300 + i)
         xg, w1g, w2g, dog = (t.cuda() for t in (x, w1, w2, do))
