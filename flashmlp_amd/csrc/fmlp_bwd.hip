@@ -673,11 +673,6 @@ __device__ __forceinline__ void dw2_body(const u16* __restrict__ X, const u16* _
     asm volatile("" ::: "memory");
   };
 
-  // at D < 64 a subtile past the program's rows is left out (X and dO are zeros there, but an infinite
-  // weight would make NaN of them); the test costs 0.4 % at H=32 B=16384 D=128 E=1024
-  auto ag2_rows = [&](int slot, int rbase) {
-    if (D >= 64 || rbase < b_hi) ag2_phase(slot, rbase);
-  };
   const std::true_type AG{};
   const std::false_type NOAG{};
   if (npair > 0) {
@@ -692,28 +687,38 @@ __device__ __forceinline__ void dw2_body(const u16* __restrict__ X, const u16* _
     };
     issue_pair(1, next);
     g1_phase(cur);
-    // first row of the subtile set `set` takes in group i
+    // first row of the subtile set `set` takes in group i; the last group may have none left for it. Such a
+    // subtile is left out: X and dO are zeros there, but an infinite weight would make NaN of them. Only
+    // the end of the walk knows of it (a test in every iteration costs 0.4 % at H=32 B=16384 D=128 E=1024).
     auto row0 = [&](int i) { return b_lo + (RS * i + set) * DW_BT; };
+    const bool whole = row0(npair - 1) < b_hi;
     if (set < RS / 2) {
-      ag2_rows(cur, row0(0));
-      pair_end(AG);
-      for (int i = 1; i < npair; ++i) {
+      // (with two row sets this is set 0, which always has one)
+      const int n = RS == 2 || whole ? npair : npair - 1;
+      if (RS == 2 || n > 0) {
+        ag2_phase(cur, row0(0));
+        pair_end(AG);
+      } else {
+        pair_end(NOAG);
+      }
+      for (int i = 1; i < n; ++i) {
         rotate();
         issue_pair(i + 1, next);
         g1_phase(cur);
-        ag2_rows(cur, row0(i));
+        ag2_phase(cur, row0(i));
         pair_end(AG);
       }
+      if (RS > 2 && n > 0 && n < npair) pair_end(NOAG);  // the barrier of the other sets' last group
     } else {
       pair_end(NOAG);
       for (int i = 1; i < npair; ++i) {
         rotate();
         issue_pair(i + 1, next);
-        ag2_rows(prev, row0(i - 1));
+        ag2_phase(prev, row0(i - 1));
         g1_phase(cur);
         pair_end(AG);
       }
-      ag2_rows(cur, row0(npair - 1));
+      if (whole) ag2_phase(cur, row0(npair - 1));
     }
   } else {
     wait_vmcnt<0>();

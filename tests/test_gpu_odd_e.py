@@ -136,3 +136,27 @@ def test_workspace_between_the_copy_and_the_plan():
     for (b, o), r in zip(bufs, gen):
         _check_guards(b, o.numel())
         assert _rel(o, r) <= 1e-4
+
+
+@pytest.mark.parametrize("H,B,D,E", [(2, 96, 128, 45), (2, 32, 64, 683), (2, 96, 64, 45), (1, 1056, 128, 683),
+                                     (3, 160, 64, 100), (2, 96, 256, 45)])
+def test_infinite_weights_stay_where_the_generic_kernels_have_them(H, B, D, E):
+    """A row range with an odd number of 32-row subtiles: the row sets without one of their own must not
+    add the NaN that an infinite weight makes of the zeros behind the last row."""
+    dt, act = torch.float16, "sigmoid"
+    print(f"[odd E] infinite w1 H={H} B={B} D={D} E={E}", flush=True)
+    L = _lib.lib()
+    x, w1, w2, do = (t.cuda() for t in make_inputs(H, B, D, E, dt, seed=3))
+    w1[H - 1, 5, 3] = float("inf")
+    f32 = _lib.FMLP_OUT_F32
+    gen = _bwd(x, w1, w2, do, act, f32, 0, torch.float32)
+    assert gen[2].isfinite().all() and not gen[0].isfinite().all()
+    for flags in (0, _lib.FMLP_BWD_RECOMPUTE, _lib.FMLP_BWD_STORE_DZ, _lib.FMLP_DW_HILO, _lib.FMLP_BWD_NO_DX):
+        n = L.fmlp_bwd_workspace_bytes(H, B, D, E, _DT[dt] | f32 | flags)
+        own = _bwd(x, w1, w2, do, act, f32 | flags, n, torch.float32)
+        for name, a, r in zip(("dx", "dw1", "dw2"), own, gen):
+            if a is not None:
+                fin = r.isfinite()
+                assert torch.equal(a.isfinite(), fin), (hex(flags), name)
+                # (HILO carries h and dZ with twice the bits: the io type's rounding apart)
+                assert _rel(a[fin], r[fin]) <= (5e-3 if flags & _lib.FMLP_DW_HILO else 1e-4), (hex(flags), name)
