@@ -44,21 +44,25 @@ namespace fmlp {
 // workgroup owns one of xs E-ranges of nct chunks of split tile (b - n_main) / xs and stores its
 // fp32 partial O tile to ws (one [BB][D] block per workgroup), which fwd_reduce_kernel sums in
 // part order and rounds.
+// Each workgroup finds its tile by integer divisions, a chain of some 25 dependent instructions each before
+// the first load can be issued: unsigned ones (no sign to fix), and one instead of two where no tile is split.
+// H=8 B=33 D=64 E=512 bf16 SiLU, one short round of workgroups: 6.41 -> 6.33 us a call.
 struct TileId {
   int h, bt;
 };
 // split tile s of n_split (H heads, T tiles per head)
 __device__ __forceinline__ TileId split_tile(int s, int n_split, int H, int T) {
-  const int t = H * T - n_split + s;
-  return TileId{t % H, t / H};
+  const unsigned t = (unsigned)(H * T - n_split + s);
+  return TileId{(int)(t % (unsigned)H), (int)(t / (unsigned)H)};
 }
 // whole tile m: rem = n_split = a H + b leaves heads h < H - b with T - a tiles, the others T - a - 1
-__device__ __forceinline__ TileId main_tile(int m, int n_split, int H, int T) {
-  const int a = n_split / H, b = n_split - a * H;
-  const int first = (H - b) * (T - a);
-  if (m < first) return TileId{m / (T - a), m % (T - a)};
-  const int m2 = m - first, tb = T - a - 1;
-  return TileId{H - b + m2 / tb, m2 % tb};
+__device__ __forceinline__ TileId main_tile(unsigned m, int n_split, int H, int T) {
+  if (n_split == 0) return TileId{(int)(m / (unsigned)T), (int)(m % (unsigned)T)};
+  const unsigned a = (unsigned)n_split / (unsigned)H, b = n_split - a * H;
+  const unsigned first = (H - b) * (T - a);
+  if (m < first) return TileId{(int)(m / (T - a)), (int)(m % (T - a))};
+  const unsigned m2 = m - first, tb = T - a - 1;
+  return TileId{(int)(H - b + m2 / tb), (int)(m2 % tb)};
 }
 // Waves per workgroup: D / 16 at D = 64 and 128 (two waves per SIMD, the threads covering a chunk's
 // 4 D pieces of W1c and of W2c once); 4 at D = 32 (half the threads load W1c, half W2c) and at D = 256 (one wave per SIMD, whose O accumulators alone
@@ -136,7 +140,7 @@ fwd_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* __r
     tile = main_tile(xcd_remap(bid, n_main), n_split, H, tiles_per_head);
   } else {
     u = bid - n_main;
-    const int s = u / xs;
+    const int s = (int)((unsigned)u / (unsigned)xs);
     tile = split_tile(s, n_split, H, tiles_per_head);
     cb = (u - s * xs) * nct;
     ce = min(ce, cb + nct);
