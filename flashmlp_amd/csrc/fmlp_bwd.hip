@@ -382,8 +382,9 @@ __device__ __forceinline__ void dx2_body(const u16* __restrict__ X, const u16* _
     }
     valu_phase();
   }
-  // (at D < 64 a part with a chunk less leaves out the product of its last step's zeros)
-  if (D >= 64 || c0 + NCP <= ce) g2_only(NCP - 1);
+  __builtin_amdgcn_sched_barrier(0);
+  // a part with a chunk less leaves out the product of its last step's zeros, of which an infinite X makes NaN
+  if (DES == 1 || part == 0 || NC % DES == 0) g2_only(NCP - 1);
   wait_vmcnt<0>();  // chunk loads past the last are still landing (as zeros)
   if constexpr (DES == 2) {  // part 1 hands its partial dX tile to part 0 through LDS (the rings)
     asm volatile("" ::: "memory");

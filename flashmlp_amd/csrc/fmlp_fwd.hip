@@ -94,12 +94,16 @@ __host__ __device__ constexpr int fwd_pf(int D, int OC, int ES = 1) {
 // 32 x 32 tile), so it is bound by the activation; four waves per SIMD (OC = 4, an 8-slot ring of
 // 32 KB each) hide the operand reads. H=32 B=4096 D=32 E=512 bf16 SiLU: forward 23 us, forward +
 // backward 720 us on the generic kernels -> 76-78 us.
-template <bool BF16, int D, int ACT, int ES, int OC = 2, int NWP = fwd_waves(D), int DG = D>
+// CUT: the E parts' chunk counts may differ. A template argument, as the test at the end of the walk costs the
+// D = 64 calls that do not need it 0.04-0.1 us (H=8 B=33 E=512: 6.31 us without, 6.36-6.42 with); the other D
+// are always built with it.
+template <bool BF16, int D, int ACT, int ES, int OC = 2, int NWP = fwd_waves(D), int DG = D, bool CUT = (ES > 1)>
 __global__ void __launch_bounds__(NWP * ES * 64) __attribute__((amdgpu_waves_per_eu(fwd_wpe(D, OC), fwd_wpe(D, OC))))
 fwd_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* __restrict__ W2,
            void* __restrict__ O, int B, int E, int ldw, long long sx, int H, int tiles_per_head, int outf32, int n_main,
            int n_split, int xs, int nct, float* __restrict__ ws) {
   constexpr int NW = NWP, NT = NW * 64;  // waves, threads of one E part
+  static_assert(!CUT || ES > 1, "one part has every chunk");
   constexpr int KS = DG / 16;          // K steps of GEMM1 (at DG = D also GEMM2's operand count 2 * D/32)
   constexpr int NTN = D / 32;          // N tiles of GEMM2
   constexpr int BB = NW * 32;          // rows per workgroup (32 per wave)
@@ -146,13 +150,12 @@ fwd_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* __r
     ce = min(ce, cb + nct);
   }
   const int h = tile.h, bt = tile.bt;
-  // chunks of this part: global chunk c0 + c for c = 0 .. NC - 1 (the last part's last chunks
-  // may lie past the range: they load as zeros and add nothing). Except at D = 64 the parts' shares
-  // differ by at most one, and a part with a chunk less leaves the product of its last step out, so
-  // that a NaN which an infinite X makes of those zeros is not added.
+  // chunks of this part: global chunk c0 + c for c = 0 .. NC - 1. Where the count does not divide (CUT) the
+  // parts' shares differ by one; the last chunk of a part with one less loads as zeros, and its product is left
+  // out, so that a NaN which an infinite X makes of those zeros is not added.
   const int NC = (ce - cb + ES - 1) / ES;
-  const int c0 = D != 64 ? cb + part * (ce - cb) / ES : cb + part * NC;
-  const int c1 = ES > 1 && D != 64 ? cb + (part + 1) * (ce - cb) / ES : ce;
+  const int c0 = CUT ? cb + part * (ce - cb) / ES : cb + part * NC;
+  const int c1 = CUT ? cb + (part + 1) * (ce - cb) / ES : ce;
   const int e_end = min(E, c1 * 32);  // columns of W1 (rows of W2) this workgroup reads
   const unsigned RB = (unsigned)part * NSLOT * 128u * D;  // this part's ring
 
@@ -315,7 +318,7 @@ fwd_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* __r
     if constexpr (decltype(SYNC)::value) chunk_end();
   };
   auto last_gemm2 = [&](const St& st) {
-    if (ES > 1 && D != 64 && c0 + NC > c1) return;
+    if (CUT && c0 + NC > c1) return;
     const unsigned base2 = RB + rslot(NC - 1) * SLOT;
 #pragma unroll
     for (int s = 0; s < 2; ++s)
@@ -585,10 +588,10 @@ FwdPlan fwd_plan(int64_t H, int64_t B, int64_t D, int64_t E, int num_cus, size_t
   return p;
 }
 
-template <bool BF16, int D, int ACT, int ES, int OC = 2, int NWP = fwd_waves(D), int DG = D>
+template <bool BF16, int D, int ACT, int ES, int OC = 2, int NWP = fwd_waves(D), int DG = D, bool CUT = (ES > 1)>
 static hipError_t launch_fwd_e(const FwdArgs& a, const FwdPlan& p, int tiles_per_head, hipStream_t st) {
   const size_t lds = (size_t)ES * fwd_nslot(D, OC, ES) * 128u * D;
-  auto k = fwd_kernel<BF16, D, ACT, ES, OC, NWP, DG>;
+  auto k = fwd_kernel<BF16, D, ACT, ES, OC, NWP, DG, CUT>;
   static std::atomic<unsigned long long> lds_set{0};
   hipError_t e = set_lds_once((const void*)k, (int)lds, lds_set);
   if (e != hipSuccess) return e;
@@ -626,8 +629,14 @@ static hipError_t launch_fwd_t(const FwdArgs& a, hipStream_t st) {
   const int BB = 32 * (p.nwp > 0 ? p.nwp : fwd_waves(D));
   const int tiles_per_head = (int)((a.B + BB - 1) / BB);
   if constexpr (D == 64) {
-    if (p.es == 4) return launch_fwd_e<BF16, D, ACT, 4, 2, 2>(a, p, tiles_per_head, st);
-    if (p.es == 2) return launch_fwd_e<BF16, D, ACT, 2>(a, p, tiles_per_head, st);
+    const int64_t nch = (a.E + 31) / 32;
+    const bool cut = p.es > 1 && (nch % p.es != 0 || (p.n_split > 0 && p.nct % p.es != 0));
+    if (p.es == 4)
+      return cut ? launch_fwd_e<BF16, D, ACT, 4, 2, 2, D, true>(a, p, tiles_per_head, st)
+                 : launch_fwd_e<BF16, D, ACT, 4, 2, 2, D, false>(a, p, tiles_per_head, st);
+    if (p.es == 2)
+      return cut ? launch_fwd_e<BF16, D, ACT, 2, 2, 4, D, true>(a, p, tiles_per_head, st)
+                 : launch_fwd_e<BF16, D, ACT, 2, 2, 4, D, false>(a, p, tiles_per_head, st);
     // FMLP_FWD_OCC=2 (read once per process) keeps two waves per SIMD
     static const int occ = env_int("FMLP_FWD_OCC", 3);
     if (occ != 2) return launch_fwd_e<BF16, D, ACT, 1, 3>(a, p, tiles_per_head, st);

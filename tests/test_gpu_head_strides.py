@@ -6,7 +6,10 @@ import pytest
 import torch
 
 import flashmlp_amd as fm
+from flashmlp_amd import _lib
 from oracle.inputs import make_inputs
+from test_gpu_narrow import _generic
+from test_gpu_odd_e import _DT, _p, _rel, _stream
 
 pytestmark = pytest.mark.gpu
 
@@ -70,3 +73,47 @@ def test_no_copy_is_allocated():
     before = torch.cuda.memory_allocated()
     o = fm.flashmlp_fwd(xe, w1, w2, "silu")
     assert torch.cuda.max_memory_allocated() - before < o.numel() * 2 * 1.5  # the output alone
+
+
+def _strided(x, w1, w2, do, act, code, st, ws_bytes=0):
+    """o, dx, dw1, dw2 (fp32 sums) through the strided C entry points with these stride arrays"""
+    L = _lib.lib()
+    (H, B, D), E = x.shape, w1.shape[2]
+    code |= _lib.FMLP_OUT_F32
+    outs = [torch.full(s, float("nan"), device="cuda") for s in ((H, B, D), (H, B, D), (H, D, E), (H, E, D))]
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device="cuda") if ws_bytes else None
+    _lib.check(L.fmlp_fwd_strided(_p(x), _p(w1), _p(w2), _p(outs[0]), H, B, D, E, *st[:3], code, _lib.ACT_CODES[act],
+                                  _stream()), "forward")
+    _lib.check(L.fmlp_bwd_strided(_p(x), _p(w1), _p(w2), _p(do), *(_p(t) for t in outs[1:]), H, B, D, E, *st, code,
+                                  _lib.ACT_CODES[act], _p(ws), ws_bytes, _stream()), "backward")
+    torch.cuda.synchronize()
+    return outs
+
+
+@pytest.mark.parametrize("H,B,D,E", [(2, 96, 64, 288), (2, 300, 64, 96), (2, 96, 64, 160), (3, 4096, 64, 544),
+                                     (2, 96, 128, 288), (2, 96, 128, 96)])
+@pytest.mark.parametrize("what", ["x", "w1"])
+def test_infinities_in_views_stay_where_the_generic_kernels_have_them(H, B, D, E, what):
+    """Views whose heads lie apart, with whole tiles of E (inside a cut one both kernel sets multiply
+    zeros): the chunks that an E part does not have, and the subtiles that a row set does not, must not
+    turn an infinite input's saturated sigmoid into NaN."""
+    dt, act = torch.float16, "sigmoid"
+    print(f"[heads] infinite {what} H={H} B={B} D={D} E={E}", flush=True)
+    x, w1, w2, do = (t.cuda() for t in make_inputs(H, B, D, E, dt, seed=3))
+    w1[w1 == 0] = 0.125  # inf * 0 is the oracle's NaN
+    x[x == 0] = 0.125
+    if what == "x":
+        x[H - 1, 5, 3] = float("inf")
+    else:
+        w1[H - 1, 5, 3] = float("inf")
+    n = _lib.lib().fmlp_bwd_workspace_bytes(H, B, D, E, _DT[dt])
+    gen = _generic(x, w1, w2, do, act, 0)
+    xv = _views(x, 8)
+    st = [_lib.strides(t) for t in (xv, w1, w2, do)]
+    assert gen[0].isfinite().all()
+    for ws in (0, n):
+        got = _strided(xv, w1, w2, do, act, _DT[dt], st, ws)
+        for name, a, r in zip(("o", "dx", "dw1", "dw2"), got, gen):
+            fin = r.isfinite()
+            assert torch.equal(a.isfinite(), fin), (name, ws)
+            assert _rel(a[fin], r[fin]) <= 1e-4, (name, ws)
