@@ -178,6 +178,7 @@ void dense3(int64_t n1, int64_t n2, long long* s) {
   s[1] = (long long)n2;
   s[2] = 1;
 }
+bool same_strides(const int64_t* s, int64_t n1, int64_t n2) { return s[0] == n1 * n2 && s[1] == n2 && s[2] == 1; }
 bool is_dense3(const int64_t* s, int64_t n0, int64_t n1, int64_t n2) {
   return (n0 == 1 || s[0] == n1 * n2) && (n1 == 1 || s[1] == n2) && (n2 == 1 || s[2] == 1);
 }
@@ -476,8 +477,10 @@ int bwd_impl(const void* x, const void* w1, const void* w2, const void* dout, vo
   if (H == 0 || (!want_dx && !want_dw)) return ok();
   const bool dense = sx == nullptr || (is_heads3(sx, H, B, D, (int)es) && is_dense3(sw1, H, D, E) &&
                                        is_dense3(sw2, H, E, D) && is_heads3(sdo, H, B, D, (int)es));
-  // X and dout dense too: the calls whose workspace is required (any other accepts any workspace)
-  const bool all_dense = sx == nullptr || (is_dense3(sx, H, B, D) && is_dense3(sdo, H, B, D));
+  // every stride that of dense tensors, those of dimensions of one element included: the calls whose
+  // workspace is required (any other accepts any workspace)
+  const bool all_dense = sx == nullptr || (same_strides(sx, B, D) && same_strides(sw1, D, E) &&
+                                           same_strides(sw2, E, D) && same_strides(sdo, B, D));
   const bool aligned = aligned16(x) && aligned16(w1) && aligned16(w2) && aligned16(dout) && aligned16(dx) &&
                        aligned16(dw1) && aligned16(dw2);
   hipError_t e = hipSuccess;

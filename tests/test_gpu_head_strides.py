@@ -2,6 +2,8 @@
 every head) are read in place: bit-identical to the same values passed densely, with no copy of
 them allocated; other views are copied as before.
 """
+import ctypes
+
 import pytest
 import torch
 
@@ -88,6 +90,27 @@ def _strided(x, w1, w2, do, act, code, st, ws_bytes=0):
                                   _lib.ACT_CODES[act], _p(ws), ws_bytes, _stream()), "backward")
     torch.cuda.synchronize()
     return outs
+
+
+@pytest.mark.parametrize("B,D,E,which", [(2048, 128, 256, w) for w in range(4)] + [(1, 128, 2048, 0), (1, 128, 2048, 3)])
+def test_one_head_with_any_head_stride_accepts_any_workspace(B, D, E, which):
+    """A lone head (or row) of a view may carry any stride in that dimension; fmlp_bwd_strided takes such
+    a call without a workspace, whatever the dense call's plan needs."""
+    L = _lib.lib()
+    H, dt, act = 1, torch.bfloat16, "silu"
+    x, w1, w2, do = (t.cuda() for t in make_inputs(H, B, D, E, dt, seed=B + E))
+    n = L.fmlp_bwd_workspace_bytes(H, B, D, E, _DT[dt])
+    print(f"[heads] lone head B={B} D={D} E={E} tensor {which} workspace {n}", flush=True)
+    assert n > 0 and L.fmlp_shape_tuned(D, E, _DT[dt]) == 1
+    assert L.fmlp_bwd(_p(x), _p(w1), _p(w2), _p(do), _p(torch.empty_like(x)), _p(torch.empty_like(w1)),
+                      _p(torch.empty_like(w2)), H, B, D, E, _DT[dt], _lib.ACT_CODES[act], None, 0, _stream()) == 4
+    st = [_lib.strides(t) for t in (x, w1, w2, do)]
+    ref = _strided(x, w1, w2, do, act, _DT[dt], st, n)
+    st[which] = (ctypes.c_int64 * 3)(x[0].numel() + 16, D if B > 1 else 3 * D, 1) if which in (0, 3) else \
+        (ctypes.c_int64 * 3)(w1[0].numel() + 16, E if which == 1 else D, 1)
+    got = _strided(x, w1, w2, do, act, _DT[dt], st)
+    for name, a, r in zip(("o", "dx", "dw1", "dw2"), got, ref):
+        assert _rel(a, r) <= 1e-4, name
 
 
 @pytest.mark.parametrize("H,B,D,E", [(2, 96, 64, 288), (2, 300, 64, 96), (2, 96, 64, 160), (3, 4096, 64, 544),
