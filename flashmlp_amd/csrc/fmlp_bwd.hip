@@ -1540,8 +1540,8 @@ dxgs_kernel(const u16* __restrict__ dzt, const u16* __restrict__ W1, void* __res
 // four accumulator tiles and operands of a wave leave room for four waves per SIMD (two
 // workgroups per CU, whose starts and ends overlap). Per 32-column E-chunk: dZ (8 KB, read once) and
 // W1c (16 KB, L2-resident) through a 3-slot LDS ring two chunks ahead, one barrier, and 8 MFMAs
-// per wave from 8 KB of operand reads. The products and their order are dxg_kernel's, and so the
-// bits of dX those of the recomputing programs. Small grids (xs > 1, plan_dw256): a tile's chunks over
+// per wave from 8 KB of operand reads. The products and their order are dxg_kernel's, and so with
+// whole tiles the bits of dX those of the recomputing programs. Small grids (xs > 1, plan_dw256): a tile's chunks over
 // xs workgroups, whose fp32 partial tiles launch_tile_reduce sums in part order.
 // A lone workgroup takes 0.55 us per chunk: H=1 B=33 E=2048 bf16 36.0 -> 5.6 us + 1.6-3 for the sum, H=1 B=1000
 // E=2048 40.4 -> 11.5 + 4 (kernel trace).
@@ -2015,16 +2015,23 @@ Dw256Plan plan_dw256(int64_t H, int64_t B, int64_t E, bool hilo, int dz_mode, in
     double best = 0.8 * kChunkUs * (double)nch;  // by a fifth: the estimate's error, and a launch more on the host
     const long long cap = std::min<long long>(std::min<long long>(2 * R <= N ? N / R : 1, nch / 4), 16);
     const size_t xoff = (p.ws_bytes + 255) / 256 * 256;
+    const auto part_bytes = [&](long long xs) { return (size_t)R * (size_t)xs * (128 * 256 * sizeof(float)); };
     for (long long want = 2; want <= cap; ++want) {
       const long long nct = (nch + want - 1) / want, xs = (nch + nct - 1) / nct;
-      const size_t need = xoff + (size_t)R * (size_t)xs * (128 * 256 * sizeof(float));
       const double t = kChunkUs * (double)nct + 3.0 + (double)(H * B * xs) * (256 * 4.0 / 2.0e6);
-      if (xs < 2 || need > max_ws || t >= best) continue;
+      if (xs < 2 || t >= best) continue;
       best = t;
       p.xg_xs = (int)xs;
       p.xg_nct = (int)nct;
+    }
+    // the split does not depend on the workspace: one too small for it takes whole tiles, whose dX has the
+    // recompute form's bits, not fewer parts with bits of their own
+    if (p.xg_xs > 1 && xoff + part_bytes(p.xg_xs) <= max_ws) {
       p.xg_off = xoff;
-      p.ws_bytes = need;
+      p.ws_bytes = xoff + part_bytes(p.xg_xs);
+    } else {
+      p.xg_xs = 1;
+      p.xg_nct = (int)nch;
     }
   }
   return p;

@@ -61,5 +61,20 @@ def test_tiles_split_over_e(H, B, E, dt, act):
     for flags in (0, _lib.FMLP_DW_HILO):  # dX does not depend on the dW mode; repeats agree
         nf = L.fmlp_bwd_workspace_bytes(H, B, D, E, code | flags)
         assert torch.equal(_bwd(x, w1, w2, do, act, flags, nf, dt)[0], sums[0].to(dt))
-    short = _bwd(x, w1, w2, do, act, f, n - 16, torch.float32)  # fewer parts, or none
+    short = _bwd(x, w1, w2, do, act, f, n - 16, torch.float32)  # whole tiles
     assert ((short[0] - rec[0]).norm() / rec[0].norm()).item() <= 1e-6
+
+
+@pytest.mark.parametrize("H,B,E", [(1, 33, 2048), (2, 300, 1355)])
+def test_a_workspace_too_short_for_every_part_takes_whole_tiles(H, B, E):
+    # dX has the split's bits or the recompute form's, nothing between them
+    L = _lib.lib()
+    D, dt, act = 256, torch.bfloat16, "silu"
+    x, w1, w2, do = (t.cuda() for t in make_inputs(H, B, D, E, dt, seed=B + E))
+    f = _lib.FMLP_OUT_F32
+    n = L.fmlp_bwd_workspace_bytes(H, B, D, E, _DT[dt] | f)
+    rec = _bwd(x, w1, w2, do, act, f | _lib.FMLP_BWD_RECOMPUTE, n, torch.float32)
+    assert not torch.equal(_bwd(x, w1, w2, do, act, f, n, torch.float32)[0], rec[0]), "the case must split its tiles"
+    for short in (n - 16, n - H * -(-B // 128) * 128 * 256 * 4):  # one part of each tile less
+        print(f"[dxg256-short] H={H} B={B} E={E} workspace {short} of {n}", flush=True)
+        assert torch.equal(_bwd(x, w1, w2, do, act, f, short, torch.float32)[0], rec[0])
