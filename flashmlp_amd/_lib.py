@@ -48,6 +48,8 @@ SIGNATURES = {
     "fmlp_fwd_workspace_bytes": (ctypes.c_size_t, [_i64, _i64, _i64, _i64, ctypes.c_int]),
     "fmlp_fwd_ws": (ctypes.c_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, ctypes.c_int, ctypes.c_int, _vp,
                                    ctypes.c_size_t, _vp]),
+    "fmlp_copy_dense": (ctypes.c_int, [ctypes.c_int, ctypes.POINTER(_vp), ctypes.POINTER(_vp), _i64p, _i64p, ctypes.c_int,
+                                       _vp]),
     "fmlp_bwd_workspace_bytes": (ctypes.c_size_t, [_i64, _i64, _i64, _i64, ctypes.c_int]),
     "fmlp_bwd_stores_dz": (ctypes.c_int, [_i64, _i64, _i64, _i64, ctypes.c_int, ctypes.c_int]),
     "fmlp_bwd_plan": (ctypes.c_int, [_i64, _i64, _i64, _i64, ctypes.c_int, ctypes.c_int, _i64p, ctypes.c_int]),

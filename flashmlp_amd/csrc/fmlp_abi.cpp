@@ -372,6 +372,35 @@ FMLP_EXPORT int fmlp_fwd_strided_ws(const void* x, const void* w1, const void* w
                   stream);
 }
 
+FMLP_EXPORT int fmlp_copy_dense(int n, const void* const* src, void* const* dst, const int64_t* sizes,
+                                const int64_t* strides, int elem_bytes, void* stream) {
+  if (n < 0 || n > 4) return fail(FMLP_ERR_INVALID_ARG, "%d tensors: at most 4", n);
+  if (elem_bytes != 2 && elem_bytes != 4) return fail(FMLP_ERR_UNSUPPORTED, "elements of %d bytes: 2 or 4", elem_bytes);
+  if (n > 0 && (src == nullptr || dst == nullptr || sizes == nullptr || strides == nullptr))
+    return fail(FMLP_ERR_INVALID_ARG, "tensor arrays must not be NULL");
+  fmlp::DenseCopies c{};
+  for (int i = 0; i < n; ++i) {
+    const int64_t* z = sizes + 3 * i;
+    int st = check_strides(strides + 3 * i, "tensor");
+    if (st) return st;
+    if (z[0] < 0 || z[1] < 0 || z[2] < 0) return fail(FMLP_ERR_INVALID_ARG, "negative size");
+    if (z[0] == 0 || z[1] == 0 || z[2] == 0) continue;
+    if (z[1] > 0x7fffffffLL / z[0] || z[2] > 0x7fffffffLL / (z[0] * z[1]))
+      return fail(FMLP_ERR_UNSUPPORTED, "a tensor of 2^31 elements or more");
+    if ((st = check_ptr(src[i], "src", true, (size_t)elem_bytes)) || (st = check_ptr(dst[i], "dst", true))) return st;
+    fmlp::DenseCopy& t = c.t[c.n++];
+    t.src = src[i];
+    t.dst = dst[i];
+    t.n1 = (unsigned)z[1];
+    t.n2 = (unsigned)z[2];
+    t.numel = (unsigned)(z[0] * z[1] * z[2]);
+    for (int k = 0; k < 3; ++k) t.s[k] = strides[3 * i + k];
+  }
+  const hipError_t e = fmlp::launch_copy_dense(c, elem_bytes, (hipStream_t)stream);
+  if (e != hipSuccess) return fail(FMLP_ERR_HIP, "copy launch: %s", hipGetErrorString(e));
+  return ok();
+}
+
 FMLP_EXPORT size_t fmlp_bwd_workspace_bytes(int64_t H, int64_t B, int64_t D, int64_t E, int dtype) {
   if (check_shape(H, B, D, E, dtype) != FMLP_OK) return 0;
   const int io = io_of(dtype);

@@ -41,6 +41,20 @@ struct FwdArgs {
   size_t ws_bytes = 0;
 };
 
+// Strided tensors to dense buffers in one launch (fmlp_copy_dense; fmlp_fwd.hip): n of them, numel > 0
+// elements each, first: the tensor's first workgroup (filled in by the launcher).
+struct DenseCopy {
+  const void* src;
+  void* dst;
+  unsigned n1, n2, numel, first;
+  long long s[3];
+};
+struct DenseCopies {
+  DenseCopy t[4];
+  int n;
+};
+hipError_t launch_copy_dense(DenseCopies c, int es, hipStream_t st);
+
 // Forward work split (fwd_plan): es = E parts inside a workgroup (1, or 2 or 4 at D = 64, 4 with
 // nwp = 2 waves per part and 64-row tiles); tiles
 // 0 .. n_main - 1 run whole, the last n_split tiles each as xs workgroups of nct E-chunks whose

@@ -1,7 +1,8 @@
 // _fmlp_fast: the per-call fast path of flashmlp_fwd / flashmlp_bwd (flashmlp_amd/flashmlp.py).
 //
 // A CPython module (METH_FASTCALL) over the C ABI of libflashmlp.so for the common case:
-// inputs on one GPU, dense and 16-byte aligned, a shape with kernels of its own. It allocates the
+// inputs on one GPU, a shape with kernels of its own (views that they do not read in place are copied
+// to dense tensors first). It allocates the
 // outputs and the workspace with ATen on the inputs' device, launches on torch's current HIP
 // stream of that device and returns the C ABI status with the outputs; for any other input it
 // returns None and the Python wrapper takes its general path (which also raises the reference's
@@ -42,9 +43,9 @@ bool rows16(const at::Tensor& t) {
          (t.stride(0) * (int64_t)t.element_size()) % 16 == 0 && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15u) == 0;
 }
 
-// the tensors those kernels take as they are: one GPU, dense, aligned; sets the io
-// dtype code
-bool eligible(PyObject* const* args, int n, const at::Tensor** ts, int* code) {
+// the tensors of a call that those kernels take, as they are or (bit i of *copy) as a dense copy: one GPU,
+// one dtype, strided; sets the io dtype code
+bool eligible(PyObject* const* args, int n, const at::Tensor** ts, int* code, unsigned* copy) {
   for (int i = 0; i < n; ++i) {
     if (!THPVariable_Check(args[i])) return false;
     ts[i] = &THPVariable_Unpack(args[i]);
@@ -53,23 +54,86 @@ bool eligible(PyObject* const* args, int n, const at::Tensor** ts, int* code) {
   if (!x.is_cuda()) return false;
   const int c = io_code(x);
   if (c < 0) return false;
+  *copy = 0;
   for (int i = 0; i < n; ++i) {
     const at::Tensor& t = *ts[i];
-    if (t.scalar_type() != x.scalar_type() || t.device() != x.device() ||
-        !(dense16(t) || ((i == 0 || i == 3) && rows16(t))))
+    if (t.scalar_type() != x.scalar_type() || t.device() != x.device() || t.layout() != at::kStrided || t.dim() != 3)
       return false;
+    if (!dense16(t) && !((i == 0 || i == 3) && rows16(t))) {
+      if (t.is_neg() || t.is_conj()) return false;  // (a lazily negated view: its copy has to apply the sign)
+      *copy |= 1u << i;
+    }
   }
   *code = c;
   return true;
 }
 
-PyObject* wrap_or_none(const at::Tensor& t) {
-  if (!t.defined()) Py_RETURN_NONE;
-  return THPVariable_Wrap(t);
-}
+// A call's inputs as the kernels take them: the caller's tensors, or dense copies held here.
+struct Inputs {
+  const void* p[4];
+  int64_t st[4][3];
+  at::Tensor held[4];
+};
 
 at::Tensor bytes_on(const at::Tensor& like, size_t n) {
   return at::empty({(int64_t)n}, like.options().dtype(at::kByte));
+}
+
+// Elements up to which a call's copies are one launch (fmlp_copy_dense); above, ATen copies each view by
+// itself, which streams rows of large ones faster (bf16 padded rows, this launch / ATen: 2^20 elements 4.4 /
+// 6.2 us, 2^21 4.8 / 6.1, 2^22 7.1 / 6.1, 2^24 19.3 / 13.1).
+constexpr int64_t kFusedElems = (int64_t)1 << 21;
+
+// status of the copies (FMLP_OK); throws c10::OutOfMemoryError when they do not fit
+int take_inputs(const at::Tensor* const* ts, int n, unsigned copy, hipStream_t stream, Inputs* in) {
+  int64_t total = 0;
+  for (int i = 0; i < n; ++i) {
+    const at::Tensor& t = *ts[i];
+    if (copy >> i & 1u) total += t.numel();
+    in->p[i] = t.data_ptr();
+    for (int k = 0; k < 3; ++k) in->st[i][k] = t.stride(k);
+  }
+  if (copy == 0) return FMLP_OK;
+  const bool fused = total <= kFusedElems;
+  const int64_t es = ts[0]->element_size();
+  if (fused) in->held[0] = bytes_on(*ts[0], (size_t)(total * es + 4 * 256));
+  char* next = fused ? (char*)in->held[0].data_ptr() : nullptr;
+  const void* src[4];
+  void* dst[4];
+  int64_t sizes[12], strides[12];
+  int m = 0;
+  for (int i = 0; i < n; ++i) {
+    if (!(copy >> i & 1u)) continue;
+    const at::Tensor& t = *ts[i];
+    if (fused) {
+      src[m] = t.data_ptr();
+      dst[m] = next;
+      for (int k = 0; k < 3; ++k) {
+        sizes[3 * m + k] = t.size(k);
+        strides[3 * m + k] = t.stride(k);
+      }
+      ++m;
+      in->p[i] = next;
+      next += (t.numel() * es + 255) / 256 * 256;
+    } else {
+      in->held[i] = t.is_contiguous() ? t.clone(at::MemoryFormat::Contiguous) : t.contiguous();
+      in->p[i] = in->held[i].data_ptr();
+    }
+    in->st[i][0] = t.size(1) * t.size(2);
+    in->st[i][1] = t.size(2);
+    in->st[i][2] = 1;
+  }
+  return m ? fmlp_copy_dense(m, src, dst, sizes, strides, (int)es, stream) : FMLP_OK;
+}
+
+// a dense output of t's shape
+at::Tensor empty_dense(const at::Tensor& t) {
+  return t.is_contiguous() ? at::empty_like(t) : at::empty(t.sizes(), t.options());
+}
+
+PyObject* wrap_or_none(const at::Tensor& t) {
+  if (!t.defined()) Py_RETURN_NONE;
+  return THPVariable_Wrap(t);
 }
 
 // fwd(x, w1, w2, act) -> (status, o) or None
@@ -81,15 +145,24 @@ PyObject* fast_fwd(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   }
   const at::Tensor* ts[3];
   int code = 0;
-  if (!eligible(args, 3, ts, &code)) Py_RETURN_NONE;
-  const at::Tensor &x = *ts[0], &w1 = *ts[1], &w2 = *ts[2];
+  unsigned copy = 0;
+  if (!eligible(args, 3, ts, &code, &copy)) Py_RETURN_NONE;
+  const at::Tensor &x = *ts[0], &w1 = *ts[1];
   const int act = (int)PyLong_AsLong(args[3]);
   if (act == -1 && PyErr_Occurred()) return nullptr;
   const int64_t H = x.size(0), B = x.size(1), D = x.size(2), E = w1.size(2);
   if (!fmlp_shape_dense(D, E, code)) Py_RETURN_NONE;
   c10::DeviceGuard guard(x.device());
   const hipStream_t stream = c10::hip::getCurrentHIPStream(x.device().index()).stream();
-  at::Tensor o = x.is_contiguous() ? at::empty_like(x) : at::empty(x.sizes(), x.options());
+  Inputs in;
+  try {
+    const int st = take_inputs(ts, 3, copy, stream, &in);
+    if (st != FMLP_OK) return Py_BuildValue("(iO)", st, Py_None);
+  } catch (const c10::OutOfMemoryError&) {
+    if (copy == 0) throw;
+    Py_RETURN_NONE;
+  }
+  at::Tensor o = empty_dense(x);
   size_t n = fmlp_fwd_workspace_bytes(H, B, D, E, code);
   at::Tensor ws;
   if (n) {
@@ -99,9 +172,8 @@ PyObject* fast_fwd(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
       n = 0;
     }
   }
-  const int st = fmlp_fwd_strided_ws(x.data_ptr(), w1.data_ptr(), w2.data_ptr(), o.data_ptr(), H, B, D, E,
-                                     x.strides().data(), w1.strides().data(), w2.strides().data(), code, act,
-                                     n ? ws.data_ptr() : nullptr, n, stream);
+  const int st = fmlp_fwd_strided_ws(in.p[0], in.p[1], in.p[2], o.data_ptr(), H, B, D, E, in.st[0], in.st[1], in.st[2],
+                                     code, act, n ? ws.data_ptr() : nullptr, n, stream);
   return Py_BuildValue("(iN)", st, THPVariable_Wrap(o));
   END_HANDLE_TH_ERRORS
 }
@@ -116,8 +188,9 @@ PyObject* fast_bwd(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   }
   const at::Tensor* ts[4];
   int code = 0;
-  if (!eligible(args, 4, ts, &code)) Py_RETURN_NONE;
-  const at::Tensor &x = *ts[0], &w1 = *ts[1], &w2 = *ts[2], &dout = *ts[3];
+  unsigned copy = 0;
+  if (!eligible(args, 4, ts, &code, &copy)) Py_RETURN_NONE;
+  const at::Tensor &x = *ts[0], &w1 = *ts[1], &w2 = *ts[2];
   const int act = (int)PyLong_AsLong(args[4]);
   if (act == -1 && PyErr_Occurred()) return nullptr;
   int flags = (int)PyLong_AsLong(args[5]);
@@ -128,11 +201,19 @@ PyObject* fast_bwd(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const bool need_dx = (flags & FMLP_BWD_NO_DX) == 0, need_dw = (flags & FMLP_BWD_NO_DW) == 0;
   c10::DeviceGuard guard(x.device());
   const hipStream_t stream = c10::hip::getCurrentHIPStream(x.device().index()).stream();
+  Inputs in;
+  try {
+    const int st = take_inputs(ts, 4, copy, stream, &in);
+    if (st != FMLP_OK) return Py_BuildValue("(iOOO)", st, Py_None, Py_None, Py_None);
+  } catch (const c10::OutOfMemoryError&) {
+    if (copy == 0) throw;
+    Py_RETURN_NONE;
+  }
   at::Tensor dx, dw1, dw2, ws;
-  if (need_dx) dx = x.is_contiguous() ? at::empty_like(x) : at::empty(x.sizes(), x.options());
+  if (need_dx) dx = empty_dense(x);
   if (need_dw) {
-    dw1 = at::empty_like(w1);
-    dw2 = at::empty_like(w2);
+    dw1 = empty_dense(w1);
+    dw2 = empty_dense(w2);
   }
   // the workspace this call's plan needs (one plan lookup, for its own activation)
   auto ws_need = [&](int f) -> size_t {
@@ -159,11 +240,10 @@ PyObject* fast_bwd(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
       }
     }
   }
-  const int st = fmlp_bwd_strided(x.data_ptr(), w1.data_ptr(), w2.data_ptr(), dout.data_ptr(),
-                                  need_dx ? dx.data_ptr() : nullptr, need_dw ? dw1.data_ptr() : nullptr,
-                                  need_dw ? dw2.data_ptr() : nullptr, H, B, D, E, x.strides().data(),
-                                  w1.strides().data(), w2.strides().data(), dout.strides().data(), flags, act,
-                                  n ? ws.data_ptr() : nullptr, n, stream);
+  const int st = fmlp_bwd_strided(in.p[0], in.p[1], in.p[2], in.p[3], need_dx ? dx.data_ptr() : nullptr,
+                                  need_dw ? dw1.data_ptr() : nullptr, need_dw ? dw2.data_ptr() : nullptr, H, B, D, E,
+                                  in.st[0], in.st[1], in.st[2], in.st[3], flags, act, n ? ws.data_ptr() : nullptr, n,
+                                  stream);
   return Py_BuildValue("(iNNN)", st, wrap_or_none(dx), wrap_or_none(dw1), wrap_or_none(dw2));
   END_HANDLE_TH_ERRORS
 }

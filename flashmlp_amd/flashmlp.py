@@ -175,7 +175,7 @@ def flashmlp_fwd(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, activation
     assert E == E2, "Intermediate dimension mismatch"
     assert D == D2, "Output dimension mismatch"
 
-    if _fast is not None:  # one GPU, dense and aligned, a shape with kernels of its own: else None
+    if _fast is not None:  # one GPU, a shape with kernels of its own (views are copied): else None
         r = _fast.fwd(x, w1, w2, _act_code(activation))
         if r is not None:
             if r[0]:

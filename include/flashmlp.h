@@ -171,6 +171,14 @@ int fmlp_fwd_strided_ws(const void* x, const void* w1, const void* w2, void* o, 
                         int64_t E, const int64_t* x_strides, const int64_t* w1_strides, const int64_t* w2_strides,
                         int dtype, int act, void* workspace, size_t workspace_bytes, void* stream);
 
+/* Copies n (at most 4) tensors of three dimensions and any element strides to dense row-major buffers,
+ * all in one launch: tensor i has sizes[3 i ..], strides[3 i ..] (non-negative), elements of elem_bytes
+ * (2 or 4) and fewer than 2^31 of them; dst[i] is 16-byte aligned and overlaps no src. For callers whose
+ * views the kernels for dense tensors do not read in place. No counterpart in the reference, whose
+ * wrapper copies each view by itself (flashmlp.py:453-459,508). */
+int fmlp_copy_dense(int n, const void* const* src, void* const* dst, const int64_t* sizes, const int64_t* strides,
+                    int elem_bytes, void* stream);
+
 /* Bytes of device workspace fmlp_bwd / fmlp_bwd_strided need for these shapes and dtype flags
  * on the current device, whatever the activation (0 when none is needed). Every backward flag
  * can change it (FMLP_DW_HILO, FMLP_BWD_RECOMPUTE and FMLP_BWD_STORE_DZ change the plan,
