@@ -103,6 +103,12 @@ def _alloc_ws(nbytes: int, device: torch.device):
 
 
 @functools.lru_cache(maxsize=1024)
+def _reads_views(D: int, E: int, dtype: int) -> bool:
+    # any workspace accepted, and so views of any strides (in place on the generic kernels)
+    return not _lib.lib().fmlp_shape_tuned(D, E, dtype)
+
+
+@functools.lru_cache(maxsize=1024)
 def _own_kernels(D: int, E: int, dtype: int) -> bool:
     # shapes with kernels of their own, which take dense 16-byte aligned tensors; views of other
     # shapes go to the generic kernels in place
@@ -137,6 +143,17 @@ def _dense_all(*ts: torch.Tensor):
     if all(t.is_contiguous() and t.data_ptr() % 16 == 0 for t in ts):
         return ts
     return tuple(_dense(t) for t in ts)
+
+
+def _copied(in_place: bool, take):
+    """take(): a call's tensors as the kernels for dense tensors want them; None when their copies do not
+    fit on the device and the generic kernels may read the views in place instead (`in_place`)."""
+    try:
+        return take()
+    except torch.OutOfMemoryError:
+        if not in_place:
+            raise
+        return None
 
 
 def _rows(t: torch.Tensor) -> torch.Tensor:
@@ -190,9 +207,10 @@ def flashmlp_fwd(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, activation
         torch.cuda.set_device(dev)
     try:
         stream = _stream_of(dev)
-        if _own_kernels(D, E, dtype):
-            x = _rows(x)
-            w1, w2 = _dense_all(w1, w2)
+        dense = _copied(_reads_views(D, E, dtype), lambda: (_rows(x), *_dense_all(w1, w2))) \
+            if _own_kernels(D, E, dtype) else None
+        if dense is not None:
+            x, w1, w2 = dense
             ws_bytes = _fwd_ws_bytes(dev, H, B, D, E, dtype)
             try:
                 ws = _alloc_ws(ws_bytes, x.device)
@@ -262,9 +280,10 @@ def flashmlp_bwd(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, do: torch.
         torch.cuda.set_device(dev)
     try:
         stream = _stream_of(dev)
-        if _own_kernels(D, E, dtype):
-            x, do = _rows(x), _rows(do)
-            w1, w2 = _dense_all(w1, w2)
+        dense = _copied(_reads_views(D, E, dtype), lambda: (_rows(x), *_dense_all(w1, w2), _rows(do))) \
+            if _own_kernels(D, E, dtype) else None
+        if dense is not None:
+            x, w1, w2, do = dense
             ws_bytes = _ws_bytes(dev, H, B, D, E, flags)
             try:
                 ws = _alloc_ws(ws_bytes, x.device)

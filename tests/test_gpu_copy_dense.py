@@ -2,6 +2,7 @@
 256-piece workgroups and the rows, between sentinel guards; and the wrappers' results for
 views through it (bit-identical to dense calls, one launch for all of a call's views)."""
 import ctypes
+import sys
 
 import pytest
 import torch
@@ -97,3 +98,28 @@ def test_one_launch_for_all_views():
         torch.cuda.synchronize()
     kernels = [e.name for e in prof.events() if "kernel" in e.name.lower() and e.device_type == torch.autograd.DeviceType.CUDA]
     assert len(kernels) == 2 and "copy_dense" in kernels[0], kernels
+
+
+@pytest.mark.parametrize("D,E,dt", [(32, 64, torch.bfloat16), (64, 45, torch.float32), (128, 45, torch.float16),
+                                    (64, 64, torch.bfloat16)])
+def test_views_whose_copies_do_not_fit(monkeypatch, D, E, dt):
+    """Shapes whose views the generic kernels take are read in place then; the others raise, as before."""
+    mod = sys.modules["flashmlp_amd.flashmlp"]
+    H, B = 2, 70
+    x, w1, w2, do = (t.cuda() for t in make_inputs(H, B, D, E, dt, seed=B))
+    xt = x.transpose(0, 1).contiguous().transpose(0, 1)
+    w2p = torch.empty(H, E, D + 3, dtype=dt, device="cuda")[:, :, 1:1 + D].copy_(w2)
+    ref = (fm.flashmlp_fwd(x, w1, w2, "silu"), *fm.flashmlp_bwd(x, w1, w2, do, "silu"))
+
+    def full(t):
+        raise torch.OutOfMemoryError("no room for the copy")
+
+    monkeypatch.setattr(mod, "_fast", None)
+    monkeypatch.setattr(mod, "_dense", full)
+    call = lambda: (fm.flashmlp_fwd(xt, w1, w2p, "silu"), *fm.flashmlp_bwd(xt, w1, w2p, do, "silu"))
+    if _lib.lib().fmlp_shape_tuned(D, E, {torch.bfloat16: 1, torch.float16: 0, torch.float32: 2}[dt]):
+        with pytest.raises(torch.OutOfMemoryError):
+            call()
+        return
+    for a, b in zip(call(), ref):  # other kernels: sums in another order, results rounded to dt
+        assert ((a - b).float().norm() / b.float().norm()).item() <= {torch.float32: 1e-6}.get(dt, 2.0 ** -8)
