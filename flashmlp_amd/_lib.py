@@ -82,7 +82,9 @@ def lib() -> ctypes.CDLL:
                     f"{LIB_PATH} is not built; run `python -m flashmlp_amd.build` (hipcc, gfx950)")
             handle = ctypes.CDLL(str(LIB_PATH))
             for name, (res, args) in SIGNATURES.items():
-                fn = getattr(handle, name)
+                fn = getattr(handle, name, None)
+                if fn is None:  # entry points were added within an ABI version
+                    raise FlashMLPLibraryError(f"{LIB_PATH} has no {name}: rebuild it (`python -m flashmlp_amd.build`)")
                 fn.restype = res
                 fn.argtypes = args
             if handle.fmlp_abi_version() != ABI_VERSION:

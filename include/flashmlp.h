@@ -39,7 +39,9 @@ extern "C" {
 #define FMLP_ABI_VERSION 4  /* 2: FMLP_BWD_NO_DX / FMLP_BWD_NO_DW; 3: fmlp_fwd_ws, fmlp_bwd_plan;
                               4: FMLP_BWD_NO_DX runs the full call's dW plan, FMLP_BWD_NO_DW
                               the full recompute launch's dX programs (a workspace where it
-                              splits ragged dX tiles) */
+                              splits ragged dX tiles). Raised where an entry point that was
+                              there changes; added within 4, with no change to the others:
+                              fmlp_shape_dense, fmlp_fwd_strided_ws, fmlp_copy_dense */
 
 typedef enum {
   FMLP_OK = 0,

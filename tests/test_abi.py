@@ -191,3 +191,16 @@ def test_ceiling_library_exports_its_entry_point():
     assert "fmlp_ceiling_mfma" in exported and "fmlp_ceiling_mix" in exported
     assert "fmlp_ceiling_act_mix" in exported
     ctypes.CDLL(str(lib))  # loads without a GPU
+
+
+def test_a_library_without_an_entry_point_asks_for_a_rebuild(tmp_path, monkeypatch):
+    """A library built before an entry point was added: the rebuild message, not an AttributeError."""
+    src = tmp_path / "old.c"
+    src.write_text("int fmlp_abi_version(void) { return %d; }\n" % _lib.ABI_VERSION)
+    old = tmp_path / "libflashmlp.so"
+    subprocess.run(["gcc", "-shared", "-fPIC", str(src), "-o", str(old)], check=True)
+    monkeypatch.setattr(_lib, "LIB_PATH", old)
+    monkeypatch.setattr(_lib, "_lib", None)
+    with pytest.raises(_lib.FlashMLPLibraryError, match="rebuild"):
+        _lib.lib()
+    assert _lib._lib is None
