@@ -67,9 +67,9 @@ def test_shape_support(L):
     assert L.fmlp_shape_supported(1, 1, 64, 8, 1) == 1
     assert L.fmlp_shape_supported(2, 8, 96, 64, 1) == 0   # D not a power of two
     assert L.fmlp_shape_supported(2, 8, 512, 64, 1) == 0  # D above 256
-    for D in (16, 32, 256):                                # the generic kernels' D
+    for D in (16, 32, 256):                                # beside fmlp_shape_tuned's D
         assert L.fmlp_shape_supported(2, 8, D, 64, 1) == 1
-    assert L.fmlp_shape_supported(2, 8, 64, 12, 1) == 1   # any E (generic kernels when E % 8 != 0)
+    assert L.fmlp_shape_supported(2, 8, 64, 12, 1) == 1   # any E
     assert L.fmlp_shape_supported(2, 8, 64, 0, 1) == 0    # E = 0
     assert L.fmlp_shape_supported(2, 8, 64, 64, 2) == 1   # fp32 io
     assert L.fmlp_shape_supported(2, 8, 64, 64, 3) == 0   # no such dtype
@@ -161,7 +161,7 @@ def test_backward_argument_validation(L):
 
 def test_workspace_query_is_zero_for_invalid_shapes(L):
     assert L.fmlp_bwd_workspace_bytes(2, 8, 96, 64, 1) == 0
-    # the backward-form query answers 0 for rejected arguments (and for the generic kernels)
+    # the backward-form query answers 0 for rejected arguments (and for fp32)
     assert L.fmlp_bwd_stores_dz(2, 8, 96, 64, 1, 1) == 0
     assert L.fmlp_bwd_stores_dz(2, 8, 64, 64, 1, -1) == 0
     assert L.fmlp_bwd_stores_dz(2, 8, 64, 64, 1 | _lib.FMLP_BWD_RECOMPUTE | _lib.FMLP_BWD_STORE_DZ, 1) == 0

@@ -263,7 +263,7 @@ def test_fast_path_equals_general_path(monkeypatch, H, B, D, E, dt, act):
 @pytest.mark.parametrize("H,B,D,E,dt,act", [
     (2, 4096, 128, 512, torch.bfloat16, "silu"),       # tuned kernels, B split of the dW programs
     (8, 4097, 64, 2048, torch.float16, "sigmoid"),     # tuned kernels, B and dX-tile tails
-    (3, 300, 32, 45, torch.float16, "leaky_relu"),     # generic kernels
+    (3, 300, 32, 45, torch.float16, "leaky_relu"),     # narrow heads, W1 through its padded copy
     (1, 4096, 128, 1024, torch.bfloat16, "silu"),      # stored dZ, dW programs split unlike the recompute form's
 ], ids=["bf16-D128", "fp16-D64-tail", "fp16-D32-generic", "bf16-D128-stored-dz"])
 def test_function_computes_only_the_gradients_autograd_needs(H, B, D, E, dt, act):

@@ -4,8 +4,8 @@ atomically), and ctypes releases the GIL during a call, so threads on their own 
 library at the same time. No kernel waits on another workgroup, so kernels of different
 streams may overlap on the device in any way.
 
-Four threads, each on its own stream, run forward + backward on a shape of their own (the
-tuned D = 128 and D = 64 kernels, the generic kernels in fp32, the D = 256 programs) several
+Five threads, each on its own stream, run forward + backward on a shape of their own (the
+tuned D = 128 and D = 64 kernels, the fp32 kernels, the D = 256 programs, the generic kernels) several
 times, starting on shapes no other test plans, so the plans are computed concurrently too.
 Afterwards each shape runs once more serially on the default stream: every output of every
 thread must be bitwise equal to it (same plan, deterministic kernels).
@@ -24,6 +24,7 @@ CASES = [
     (6, 1517, 64, 520, torch.float16, "sigmoid"),
     (3, 777, 32, 200, torch.float32, "leaky_relu"),
     (2, 1203, 256, 264, torch.bfloat16, "silu"),
+    (2, 911, 256, 72, torch.float32, "silu"),
 ]
 ITERS = 5
 

@@ -1,5 +1,7 @@
-"""Parity of the generic kernels (fmlp_gen.hip): the shapes, dtypes and layouts the tuned
-kernels do not take, against the CPU oracle.
+"""Parity of the shapes, dtypes and layouts outside fmlp_shape_tuned, through the public API, against
+the CPU oracle. Dense tensors of these shapes run on kernels of their own (fmlp_shape_dense) except
+fp32 at D = 256; the generic kernels (fmlp_gen.hip), which gave this file its name, are pinned through
+the calls that reach them in tests/test_gpu_generic_views.py.
 
   * D in {16, 32, 256} (the reference's D is any power of two >= 16, flashmlp.py:66,186),
     E not a multiple of 8, and B tails, at fp16 / bf16 with the bars of test_gpu_parity
@@ -7,9 +9,9 @@ kernels do not take, against the CPU oracle.
     the cast-point emulation and normwise 1e-2 against fp32);
   * fp32 io (the reference's io dtype is x's, flashmlp.py:87): every output is an fp32 sum,
     held to the north star's 1e-4 relative (normwise) against the fp32 oracle;
-  * strided inputs read in place (sliced, transposed and stride-0 views): bit-identical to the
+  * strided inputs (sliced, transposed and stride-0 views): bit-identical to the
     same values passed densely;
-  * the fp32-output flag and the hi/lo dW mode on the generic path.
+  * the fp32-output flag and the hi/lo dW mode.
 """
 import ctypes
 import sys
@@ -74,7 +76,7 @@ def test_generic_16bit(D, dt, act):
 
 
 def test_generic_tuned_d_with_odd_e():
-    # D = 128 bf16 with E % 8 != 0 leaves the tuned kernels for the generic ones
+    # D = 128 bf16 with E % 8 != 0: W1 through its padded copy
     (x, w1, w2, do), (o, dx, dw1, dw2) = _run(3, 130, 128, 13, torch.bfloat16, "silu", seed=4)
     ro, rdx, _, _ = reference.autograd_grads(x, w1, w2, do, "silu")
     _, edw1, edw2 = emulate.emu_bwd(x, w1, w2, do, "silu", torch.bfloat16)
@@ -107,8 +109,7 @@ def test_fp32_cfg1_shape():
 
 @pytest.mark.parametrize("D,dt", [(32, torch.bfloat16), (256, torch.float16), (64, torch.float32)])
 def test_strided_views_are_read_in_place(D, dt):
-    # both calls on the generic kernels: at D = 256 an E that is no multiple of 8 keeps the dense
-    # forward off the tuned kernel (which takes dense D = 256 inputs with E % 8 == 0)
+    # through the wrappers, which copy these views for the kernels for dense tensors
     H, B, E = 3, 70, (44 if D == 256 else 40)
     x, w1, w2, do = (t.cuda() for t in make_inputs(H, B, D, E, dt, seed=8))
     o_ref = fm.flashmlp_fwd(x, w1, w2, "silu")
@@ -138,7 +139,7 @@ def test_strided_views_are_read_in_place(D, dt):
 
 
 def test_fp32_outputs_on_generic_path():
-    # FMLP_OUT_F32: the generic kernels' unrounded fp32 sums against the emulation's
+    # FMLP_OUT_F32 at D = 32: the unrounded fp32 sums against the emulation's
     L = _lib.lib()
     H, B, D, E = 2, 90, 32, 72
     x, w1, w2, do = make_inputs(H, B, D, E, torch.bfloat16, seed=12)
@@ -207,8 +208,8 @@ def _bwd_strided(x, w1, w2, do, act, ws_bytes):
 @pytest.mark.parametrize("D,dt,act", [(32, torch.bfloat16, "silu"), (256, torch.float16, "sigmoid"),
                                       (64, torch.float32, "leaky_relu")], ids=["D32-bf16", "D256-fp16", "D64-fp32"])
 def test_generic_dw_b_split(D, dt, act):
-    """The generic dW programs split B over workgroups when the workspace allows (fp32 partials,
-    then a reduction in split order): with the queried workspace the results match the oracle at
+    """Dense strides through the strided entry point: the dW programs split B over workgroups when the
+    workspace allows (fp32 partials, then a reduction in split order): with the queried workspace the results match the oracle at
     the usual bars, and the unsplit run (no workspace) within the summation-order difference."""
     H, B, E = 2, 3000, 136
     x, w1, w2, do = make_inputs(H, B, D, E, dt, seed=81)

@@ -9,7 +9,7 @@ inputs and the same call is run eagerly on separate tensors, with synchronisatio
 every replay's outputs must be bitwise equal to the eager call's (the kernels are deterministic).
 Cases: D = 64 fp16 with a B-split workspace (recompute form), a ragged D = 64 forward whose
 split tiles use the forward's workspace (cfg5's shape), the stored-dZ backward at cfg4's shape,
-and the generic kernels (D = 32). The reference has no graph support to compare with.
+the D = 32 programs, and the generic kernels (fp32 at D = 256). The reference has no graph support to compare with.
 """
 import sys
 
@@ -25,7 +25,8 @@ CASES = [
     ("d128_bf16_stored_dz", 32, 16384, 128, 1024, torch.bfloat16, "silu", {}),
     ("d128_bf16_recompute_accurate", 4, 2048, 128, 512, torch.bfloat16, "leaky_relu",
      {"recompute": True, "accurate_dw": True}),
-    ("d32_generic", 3, 300, 32, 72, torch.bfloat16, "sigmoid", {}),
+    ("d32_generic", 3, 300, 32, 72, torch.bfloat16, "sigmoid", {}),  # (kernels of its own, despite the name)
+    ("d256_fp32_generic", 2, 1100, 256, 72, torch.float32, "silu", {}),
 ]
 REPLAYS = 4
 

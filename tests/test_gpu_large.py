@@ -13,8 +13,8 @@ test_gpu_parity.py:
   * dW1, dW2 elementwise against the emulation over S, normwise against fp32.
 Cases: D = 64 fp16 sigmoid and D = 128 bf16 SiLU with B past 2^24 (recompute form: one head's
 dZ image would exceed 2 GB, so the plan cannot store it); a four-head D = 128 shape forced into
-the stored-dZ form (FMLP_BWD_STORE_DZ), whose dZ workspace also passes 2^32 bytes; fp32 io on the
-generic kernels (normwise 1e-4 against fp32, the north star's bar for fp32 sums); and X as a
+the stored-dZ form (FMLP_BWD_STORE_DZ), whose dZ workspace also passes 2^32 bytes; fp32 io at
+D = 32 (normwise 1e-4 against fp32, the north star's bar for fp32 sums); and X as a
 transposed view of a (B, H, D) tensor through fmlp_fwd_strided / fmlp_bwd_strided (generic
 kernels reading the view in place, row stride H D).
 """
@@ -38,6 +38,7 @@ CASES = [
     ("d64_fp16_sigmoid", 2, (1 << 24) + 129, 64, 128, torch.float16, "sigmoid", "api"),
     ("d128_bf16_silu", 2, (1 << 24) + 129, 128, 256, torch.bfloat16, "silu", "api"),
     ("d128_bf16_silu_stored_dz", 4, (1 << 22) + 65, 128, 128, torch.bfloat16, "silu", "stored_dz"),
+    # (the fp32 kernels, despite the name)
     ("d32_fp32_leaky_generic", 2, (1 << 25) + 33, 32, 64, torch.float32, "leaky_relu", "api"),
     ("d64_fp16_silu_strided_x", 2, (1 << 24) + 129, 64, 64, torch.float16, "silu", "strided"),
 ]

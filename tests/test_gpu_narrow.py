@@ -1,6 +1,6 @@
 """D = 16 and 32 on the fused programs (32-column tiles; at D = 16 their upper half is zeros).
 
-Against the generic kernels, which the same values reach as a strided view of X: the unrounded
+Against the generic kernels, which the same values reach with W2 as a view of padded rows: the unrounded
 fp32 sums (FMLP_OUT_F32) within 1e-4 normwise, the bar of the other fp32-sum tests. Sizes at the
 edges of the tiles (32 columns of E, 64 / 128 rows, 32-row subtiles and the B split of the dW
 programs, the forward's E split and its whole grids), with guards around every output.
@@ -26,20 +26,18 @@ CASES = [
 
 
 def _generic(x, w1, w2, do, act, flags):
-    """forward and backward on the generic kernels: X as a transposed copy viewed back"""
+    """forward and backward on the generic kernels: W2 with padded rows, which the others do not read"""
     L = _lib.lib()
     H, B, D = x.shape
     E = w1.shape[2]
-    xv = x.transpose(1, 2).contiguous().transpose(1, 2)
-    if B == 1:  # a single row needs a padded pitch to be a view
-        xv = torch.empty(H, 2, D + 8, dtype=x.dtype, device="cuda")[:, :1, :D].copy_(x)
-    assert not xv.is_contiguous()
+    w2v = torch.empty(H, E, D + 8, dtype=x.dtype, device="cuda")[:, :, :D].copy_(w2)
+    assert E > 1  # (a single row's pitch is no layout of its own)
     code = _DT[x.dtype] | _lib.FMLP_OUT_F32
     outs = [torch.empty(s, device="cuda") for s in ((H, B, D), (H, B, D), (H, D, E), (H, E, D))]
-    st = [_lib.strides(t) for t in (xv, w1, w2, do)]
-    _lib.check(L.fmlp_fwd_strided(_p(xv), _p(w1), _p(w2), _p(outs[0]), H, B, D, E, *st[:3], code, _lib.ACT_CODES[act],
+    st = [_lib.strides(t) for t in (x, w1, w2v, do)]
+    _lib.check(L.fmlp_fwd_strided(_p(x), _p(w1), _p(w2v), _p(outs[0]), H, B, D, E, *st[:3], code, _lib.ACT_CODES[act],
                                   _stream()), "forward")
-    _lib.check(L.fmlp_bwd_strided(_p(xv), _p(w1), _p(w2), _p(do), *(_p(t) for t in outs[1:]), H, B, D, E, *st,
+    _lib.check(L.fmlp_bwd_strided(_p(x), _p(w1), _p(w2v), _p(do), *(_p(t) for t in outs[1:]), H, B, D, E, *st,
                                   code | flags, _lib.ACT_CODES[act], None, 0, _stream()), "backward")
     torch.cuda.synchronize()
     return outs

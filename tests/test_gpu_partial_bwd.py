@@ -87,7 +87,7 @@ CASES = [
     # H, B, D, E, dtype, act, seed, x transposed (a strided view: generic kernels)
     (2, 4096, 128, 512, torch.bfloat16, "silu", 71, False),      # tuned kernels, B split
     (8, 4097, 64, 2048, torch.float16, "sigmoid", 72, False),    # tuned kernels, tails
-    (3, 300, 32, 45, torch.float16, "leaky_relu", 73, False),    # generic kernels (D = 32)
+    (3, 300, 32, 45, torch.float16, "leaky_relu", 73, False),    # narrow heads, W1 padded (D = 32)
     (2, 260, 64, 136, torch.bfloat16, "silu", 74, True),         # generic kernels (strided X)
     (1, 4096, 128, 1024, torch.bfloat16, "silu", 75, False),     # stored dZ, another B split
     (1, 4096, 64, 2048, torch.float16, "sigmoid", 76, False),    # stored dZ, 128- vs 64-column dW
