@@ -108,8 +108,7 @@ size_t elem_bytes(int io) { return io == FMLP_DTYPE_F32 ? 4 : 2; }
 bool tuned_shape(int64_t D, int64_t E, int io) {
   return (io == FMLP_DTYPE_F16 || io == FMLP_DTYPE_BF16) && (D == 64 || D == 128) && E % 8 == 0;
 }
-// the tuned forward also takes D = 256 (one wave per SIMD), and so do the backward's D = 256 dX
-// and dW programs (launch_dx256, launch_dw256), with the generic kernels' workspace rule
+// the shapes fmlp_bwd_plan reports a plan for: those above and D = 256 with E % 8 == 0
 bool fwd_tuned_shape(int64_t D, int64_t E, int io) {
   return tuned_shape(D, E, io) || ((io == FMLP_DTYPE_F16 || io == FMLP_DTYPE_BF16) && D == 256 && E % 8 == 0);
 }
@@ -439,7 +438,7 @@ FMLP_EXPORT int fmlp_bwd_plan(int64_t H, int64_t B, int64_t D, int64_t E, int dt
   int st = check_shape(H, B, D, E, dtype);
   if (st) return st;
   if ((st = check_act(act))) return st;
-  if (!fwd_tuned_shape(D, E, io_of(dtype))) return fail(FMLP_ERR_UNSUPPORTED, "the generic kernels have no such plan");
+  if (!fwd_tuned_shape(D, E, io_of(dtype))) return fail(FMLP_ERR_UNSUPPORTED, "no plan is reported outside 16-bit D = 64, 128 and 256 with E %% 8 == 0");
   if (n_info > 0 && info == nullptr) return fail(FMLP_ERR_INVALID_ARG, "info is NULL");
   int cus = 0;
   if ((st = num_cus_current(&cus))) return st;
@@ -481,8 +480,8 @@ FMLP_EXPORT int fmlp_bwd_stores_dz(int64_t H, int64_t B, int64_t D, int64_t E, i
 
 namespace {
 
-// The backward of every entry point: argument checks, then the tuned kernels (dense, aligned,
-// tuned shape; fp32 partials in `ws`, or in the static scratch when `noalloc`) or the
+// The backward of every entry point: argument checks, then the kernels for dense tensors (aligned, X and
+// dout with any head stride; fp32 partials in `ws`, or in the static scratch when `noalloc`) or the
 // generic kernels.
 int bwd_impl(const void* x, const void* w1, const void* w2, const void* dout, void* dx, void* dw1, void* dw2,
              int64_t H, int64_t B, int64_t D, int64_t E, const int64_t* sx, const int64_t* sw1, const int64_t* sw2,

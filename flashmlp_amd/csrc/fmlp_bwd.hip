@@ -776,7 +776,7 @@ dx2_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* __r
                               (E + 31) >> 5, nullptr);
 }
 
-// dX programs at D = 256 (the tuned backward's dX only; its dW runs on the generic kernels):
+// dX programs at D = 256 (the recompute form; dw256_kernel has its dW programs):
 // 4 waves of 32 rows, one per SIMD (the X and dO rows and the dX accumulators take ~320
 // registers of the 512).
 template <bool BF16, int ACT>
@@ -870,7 +870,7 @@ dw256_kernel(const u16* __restrict__ X, const u16* __restrict__ W1, const u16* _
   issue(1);
 
   // ---- weight operands (once) ----
-  // W1 rows d, columns e_prog .. + 127 -> staging tile (zeros past E; E % 8 == 0)
+  // W1 rows d, columns e_prog .. + 127 -> staging tile (zeros past E: rows of ldw, whole 16-byte vectors)
 #pragma unroll 4
   for (int k = 0; k < 256 * 16 / 256; ++k) {
     const int p = tid + 256 * k, d = p >> 4, u = p & 15;
@@ -1089,7 +1089,7 @@ template <bool BF16>
 __global__ void __launch_bounds__(256)
 dw_reduce_kernel(const float* __restrict__ ws, void* __restrict__ dW1, void* __restrict__ dW2, int H, int E, int D,
                  int nS, int outf32) {
-  const size_t per = (size_t)H * E * D;  // a multiple of 8 (E % 8 == 0)
+  const size_t per = (size_t)H * E * D;  // a multiple of 16 (D)
   const size_t n4 = per / 4;
   const size_t stride = (size_t)gridDim.x * blockDim.x;
   for (size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x; q < 2 * n4; q += stride) {
@@ -1960,6 +1960,9 @@ BwdPlan plan_bwd(int64_t H, int64_t B, int64_t D, int64_t E, int act, bool hilo,
 // B split of the D = 256 dW programs: the nS (1, 2, 4, ...) with the least estimated time,
 // rounds of programs over the CUs times a program's time (a fixed part and one per 32-row
 // subtile) plus, for nS > 1, the summing launch and the partials' traffic (written, then read).
+// The constants date from the programs that stored no dZ and are low on small grids: kernel traces of the
+// present ones give 17.9 us for 2 subtiles, 43-45 for 16 and 92-97 for 32 on a full device, that is 14-15 us of
+// fixed time and about 2 us a subtile, where the estimate says 6, 20 and 36.
 // FMLP_DW256_NS (read once per process) forces nS where its workspace fits.
 Dw256Plan plan_dw256(int64_t H, int64_t B, int64_t E, bool hilo, int dz_mode, int num_cus, size_t max_ws) {
   constexpr double kFixedUs = 4.0, kSubUs = 1.0, kSubHiloUs = 1.4;

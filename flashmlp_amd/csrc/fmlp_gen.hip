@@ -2,8 +2,8 @@
 // (fmlp_fwd.hip, fmlp_bwd.hip) do not take.
 //
 //   * D in {16, 32, 64, 128, 256} (the reference's D is a power of two >= 16: tl.arange(0, D),
-//     flashmlp.py:66,186), any E >= 1, any B (dense 16-bit tensors with D >= 64 come here only when
-//     the call has no workspace for the tuned kernels' copy of W1, E % 8 != 0);
+//     flashmlp.py:66,186), any E >= 1, any B (dense aligned tensors come here only in fp32 at D = 256 and,
+//     where W1's rows are not 16-byte vectors, when the call has no workspace for its padded copy);
 //   * io dtype fp16, bf16 or fp32 (the reference's io dtype is x's, flashmlp.py:87,183,265,367);
 //     16-bit io uses v_mfma_f32_32x32x16_{f16,bf16}, fp32 io v_mfma_f32_32x32x2_f32;
 //   * inputs X, W1, W2, dO with arbitrary element strides (views, no copies); outputs are

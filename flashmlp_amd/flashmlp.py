@@ -28,10 +28,11 @@ Differences from the reference, all deliberate:
     use its default reduced input precision); other dtypes raise TypeError;
   * strided inputs are accepted: shapes with kernels of their own (fmlp_shape_dense: 16-bit
     io, and fp32 with D <= 128) read an x or do of dense rows in place, whatever the distance of its
-    heads (an x expanded to every head, say), and copy other views to dense tensors, as the
-    reference's reshape / contiguous does (flashmlp.py:453-459,508); every other shape reads the
-    views in place (generic kernels), where the reference would copy them or fail its contiguity
-    assertions.
+    heads (an x expanded to every head, say), and copy other views to dense tensors, all in one
+    launch, as the reference's reshape / contiguous does one by one (flashmlp.py:453-459,508); every
+    other shape (and, outside fmlp_shape_tuned, a call whose copies do not fit on the device) reads
+    the views in place (generic kernels), where the reference would copy them or fail its
+    contiguity assertions.
 """
 from __future__ import annotations
 
@@ -237,7 +238,8 @@ def flashmlp_bwd(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, do: torch.
     """FlashMLP backward pass (reference: flashmlp.py:480-538).
 
     Recomputes Z = x @ w1 and h = act(Z) instead of reading stored activations.
-    Returns (dx, dw1, dw2) shaped like (x, w1, w2). For large shapes the library stores dZ in
+    Returns (dx, dw1, dw2) shaped like (x, w1, w2). For large shapes, and at D = 256 for all,
+    the library stores dZ in
     a temporary workspace (H x ceil(E/128)*128 x ceil(B/256)*256 io elements) and computes dx
     from it; recompute=True keeps the reference's recompute-only form, whose extra memory is
     at most the fp32 dW partials, and it is also taken when the stored-dZ workspace cannot be

@@ -10,10 +10,10 @@
  * (the *_strided entry points take X, W1, W2, dO with arbitrary element strides). Element
  * type of every tensor is the io dtype (fp16, bf16 or fp32, as the reference's io dtype is
  * x's, flashmlp.py:87). All pointers are device pointers on the current HIP device, aligned
- * to their element size. Two kernel sets sit behind the entry points: the tuned gfx950
- * kernels for 16-bit io, D in {64, 128}, E % 8 == 0 on dense 16-byte aligned tensors
- * (fmlp_shape_tuned) with their like for other D, fp32 io and other E (fmlp_shape_dense), and
- * generic kernels for every other supported shape, dtype and layout.
+ * to their element size. Two kernel sets sit behind the entry points: gfx950 kernels
+ * for dense 16-byte aligned tensors (fmlp_shape_dense: 16-bit io at every D and E, fp32 at
+ * D <= 128; X and dout also with any head stride), and generic kernels for every other
+ * supported shape, dtype and layout.
  * The library never allocates: the caller passes every buffer, including the backward
  * workspace.
  *
@@ -72,7 +72,8 @@ typedef enum { FMLP_DTYPE_F16 = 0, FMLP_DTYPE_BF16 = 1, FMLP_DTYPE_F32 = 2 } fml
 /* OR-ed into the dtype argument of fmlp_bwd / fmlp_bwd_strided / fmlp_bwd_noalloc /
  * fmlp_bwd_workspace_bytes (rejected by fmlp_fwd): keep the reference's recompute-only
  * backward (flashmlp.py:341-421), whose workspace is at most the fp32 dW partials of a B split,
- * instead of the stored-dZ form the library picks for large shapes (see fmlp_bwd). No
+ * instead of the stored-dZ form the library picks for large shapes, and at D = 256 for all
+ * (see fmlp_bwd). No
  * counterpart in the reference: for callers that need the backward's memory to stay
  * O(weights). Results agree with the stored-dZ form within rounding (the same cast points). */
 #define FMLP_BWD_RECOMPUTE 0x400
@@ -119,12 +120,10 @@ int fmlp_act_from_name(const char* name);
  * dtype fp16, bf16 or fp32 with optional flags. */
 int fmlp_shape_supported(int64_t H, int64_t B, int64_t D, int64_t E, int dtype);
 
-/* 1 when the tuned kernels take these shapes (16-bit io, D in {64, 128}, E % 8 == 0) on dense,
- * 16-byte aligned tensors; other supported shapes, dtypes and layouts run on the generic
- * kernels, except that D = 256 (16-bit io, E % 8 == 0, dense, aligned) also has kernels of
- * its own: the tuned forward and the backward's D = 256 dX and dW programs, which keep the
- * generic kernels' workspace rule. No counterpart in the reference (its Triton kernels are
- * autotuned per shape). */
+/* 1 for the shapes (16-bit io, D in {64, 128}, E % 8 == 0) whose backward requires its queried
+ * workspace on dense tensors (fmlp_bwd_workspace_bytes); every other shape accepts any. Which
+ * shapes have kernels of their own is fmlp_shape_dense's answer. No counterpart in the
+ * reference (its Triton kernels are autotuned per shape). */
 int fmlp_shape_tuned(int64_t D, int64_t E, int dtype);
 
 /* 1 when dense, 16-byte aligned tensors of these shapes run on kernels other than the generic ones:
@@ -153,7 +152,10 @@ size_t fmlp_fwd_workspace_bytes(int64_t H, int64_t B, int64_t D, int64_t E, int 
  * ragged B just past a multiple of the CU count; at D >= 128 also a grid of few tiles) splits
  * those tiles over E across workgroups.
  * The parts' fp32 partials go through the workspace and a second launch sums them in a fixed
- * order. With a smaller workspace or NULL it is fmlp_fwd. The workspace is scratch for the
+ * order. Where W1's rows are not 16-byte vectors (E % 8 != 0; fp32: E % 4 != 0) its start holds
+ * their padded copy. With a smaller workspace or NULL it is fmlp_fwd, but a workspace that holds
+ * the padded copy alone still takes the kernels for dense tensors (without the split; fmlp_fwd, which
+ * has no room for it, the generic kernels). The workspace is scratch for the
  * duration of the call on `stream`. */
 int fmlp_fwd_ws(const void* x, const void* w1, const void* w2, void* o, int64_t H, int64_t B, int64_t D,
                 int64_t E, int dtype, int act, void* workspace, size_t workspace_bytes, void* stream);
@@ -207,8 +209,9 @@ int fmlp_bwd_stores_dz(int64_t H, int64_t B, int64_t D, int64_t E, int dtype, in
  * launches (the dW programs alone, or the dX programs alone over whole tiles) and the workspace
  * it needs. Also for dense 16-bit D = 256 with E % 8 == 0 (the D = 256 dX and dW programs, one
  * launch each, or dX from the stored dZ; the split and the form as with an unlimited workspace,
- * which such calls take only as far as their workspace holds). Returns FMLP_OK, or FMLP_ERR_UNSUPPORTED for shapes
- * the generic kernels take. No counterpart in the reference: a diagnostic for tests and
+ * which such calls take only as far as their workspace holds). Returns FMLP_OK, or
+ * FMLP_ERR_UNSUPPORTED for every other shape (D < 64, E % 8 != 0 and fp32 have plans too, which are not
+ * reported; their workspace is fmlp_bwd_workspace_bytes'). No counterpart in the reference: a diagnostic for tests and
  * benches. */
 int fmlp_bwd_plan(int64_t H, int64_t B, int64_t D, int64_t E, int dtype, int act, int64_t* info, int n_info);
 
@@ -220,7 +223,8 @@ int fmlp_bwd_plan(int64_t H, int64_t B, int64_t D, int64_t E, int dtype, int act
  * recompute Z and dH (one launch), and a stored-dZ form for large shapes, whose dW programs
  * also write dZ (in the io dtype: the value the dX product takes) to the workspace and dx is a
  * GEMM over it (two launches, 10u instead of 14u of matrix work, u = H B D E, at
- * H ceil(E/128) 128 ceil(B/256) 256 io elements of workspace). FMLP_BWD_RECOMPUTE keeps the
+ * H ceil(E/128) 128 ceil(B/256) 256 io elements of workspace). At D = 256 the second is taken
+ * at every size, whenever the workspace has room. FMLP_BWD_RECOMPUTE keeps the
  * first. dx, dw1, dw2 are fully overwritten. `workspace` may be NULL when
  * fmlp_bwd_workspace_bytes() is 0.
  */
