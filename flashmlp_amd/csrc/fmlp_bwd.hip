@@ -649,14 +649,11 @@ __device__ __forceinline__ void dw2_body(const u16* __restrict__ X, const u16* _
     }
     if constexpr (DZ) {
       // dzT[s] holds rows 16 s + 4 g + 0..3 and 16 s + 8 + 4 g + 0..3 of column e0 + l32: positions
-      // 16 s + 8 g .. + 7 under sig, one 16-byte store each; subtiles past the program's rows
-      // (the odd last one of a B range) store nothing (an empty resource). The block base and
-      // that test are wave-uniform, so they live in the resource (scalar registers) and each
-      // lane's offset is a constant.
-      const bool live = rbase < b_hi;
+      // 16 s + 8 g .. + 7 under sig, one 16-byte store each. The block base is wave-uniform, so it
+      // lives in the resource (scalar registers) and each lane's offset is a constant.
       const unsigned blk = ((unsigned)(rbase >> 8) * (unsigned)(Ep >> 5) + (unsigned)(e0 >> 5)) * 8u +
                            (unsigned)((rbase & 255) >> 5);
-      const Rsrc rb = make_rsrc(dzh + (size_t)blk * 1024u, live ? 2048 : 0);
+      const Rsrc rb = make_rsrc(dzh + (size_t)blk * 1024u, 2048);
 #pragma unroll
       // non-temporal: dZ is read once, by dxg_kernel, so its lines should not stay in the
       // device's caches (measured at cfg4: backward -20 us, step +1.4 %)
