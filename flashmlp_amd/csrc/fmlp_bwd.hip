@@ -24,10 +24,59 @@ namespace fmlp {
 constexpr int DW_ET = 128;           // E columns per dW program (32 per wave column group)
 constexpr int DW_BT = 32;            // rows per streamed subtile
 
+// dW1 of one head, [D][E] at `out`: rows d = 32 nt + l32; a lane holds columns e0 + 8 i4 + 4 g .. + 3 of each in
+// a1[nt][4 i4 ..]. VEC (E % 4 == 0): those four are one aligned vector. The bases are wave-uniform, the lanes' byte
+// offsets within 32 rows stay below 2^32 (dense_shape: D E 2 < 2^31).
+template <bool BF16, int NTN, bool F32, bool VEC>
+__device__ __forceinline__ void dw1_store(const f32x16 (&a1)[NTN], char* __restrict__ out, int E, int e0, int g,
+                                          int l32) {
+  constexpr unsigned ES = F32 ? 4 : 2;
+  const unsigned vo = ((unsigned)l32 * (unsigned)E + 4u * g) * ES;
+#pragma unroll
+  for (int i4 = 0; i4 < 4; ++i4) {
+    const int eb = e0 + 8 * i4 + 4 * g;
+    if constexpr (VEC) {
+      if (eb < E) {
+#pragma unroll
+        for (int nt = 0; nt < NTN; ++nt) {
+          const Rsrc r = make_rsrc(out + ((size_t)(nt * 32) * E + e0) * ES, -1);
+          if constexpr (F32)
+            __builtin_amdgcn_raw_buffer_store_b128(
+                u32x4{__float_as_uint(a1[nt][4 * i4]), __float_as_uint(a1[nt][4 * i4 + 1]),
+                      __float_as_uint(a1[nt][4 * i4 + 2]), __float_as_uint(a1[nt][4 * i4 + 3])},
+                r, (int)(vo + 8 * i4 * ES), 0, 0);
+          else
+            __builtin_amdgcn_raw_buffer_store_b64(
+                u32x2{pack2<BF16>(a1[nt][4 * i4], a1[nt][4 * i4 + 1]), pack2<BF16>(a1[nt][4 * i4 + 2], a1[nt][4 * i4 + 3])},
+                r, (int)(vo + 8 * i4 * ES), 0, 0);
+        }
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (eb + j < E) {
+#pragma unroll
+          for (int nt = 0; nt < NTN; ++nt) {
+            const Rsrc r = make_rsrc(out + ((size_t)(nt * 32) * E + e0) * ES, -1);
+            if constexpr (F32)
+              __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(a1[nt][4 * i4 + j]), r, (int)(vo + (8 * i4 + j) * ES), 0, 0);
+            else
+              __builtin_amdgcn_raw_buffer_store_b16(from_f32<BF16>(a1[nt][4 * i4 + j]), r, (int)(vo + (8 * i4 + j) * ES), 0, 0);
+          }
+        }
+      }
+    }
+  }
+}
+
 // dW epilogue. C layout of the accumulators: lane = column d
 // (32 nt + l32), rows e = e0 + 8 (i / 4) + 4 g + (i % 4). nS == 1 writes dW1, dW2 in the io
 // dtype (fp32 when outf32); otherwise fp32 partials in the outputs' layouts, ws2[s][h][e][d]
 // and ws1[s][h][d][e], which dw_reduce_kernel sums elementwise.
+// At D = 256 the outputs go out through buffer stores: with a 64-bit address per element of each of the four kinds of
+// output the programs spilled registers (dW alone at H=48 B=28 E=88 bf16 12.9 us, so 10.85; the step at H=8 B=4096
+// E=1024 166.0 and 163.7). At D <= 128 nothing spills and they are slower (backward at H=300 B=100 D=64 E=64 15.5 us,
+// so 15.8; H=1 B=16 D=128 E=64 8.0 and 8.3), as are partials at every D (that step at nS > 1 +0.9 %).
 // DG < D = 32: the tensors have DG columns d.
 template <bool BF16, int D, int DG = D>
 __device__ __forceinline__ void dw_store(const f32x16 (&a1)[D / 32], const f32x16 (&a2)[D / 32], void* __restrict__ dW1,
@@ -35,7 +84,17 @@ __device__ __forceinline__ void dw_store(const f32x16 (&a1)[D / 32], const f32x1
                                          int s, int nS, int e0, int g, int l32, int outf32) {
   constexpr int NTN = D / 32;
   if (DG < D && l32 >= DG) return;
-  if (nS == 1 && outf32) {
+  if (D == 256 && nS == 1) {
+    store_rows<BF16, D, DG>(a2, dW2, (size_t)h * E * DG, E, e0, g, l32, outf32);
+    char* o1 = (char*)dW1 + (size_t)h * DG * E * (outf32 ? 4 : 2);
+    if (outf32) {
+      if ((E & 3) == 0) dw1_store<BF16, NTN, true, true>(a1, o1, E, e0, g, l32);
+      else dw1_store<BF16, NTN, true, false>(a1, o1, E, e0, g, l32);
+    } else {
+      if ((E & 3) == 0) dw1_store<BF16, NTN, false, true>(a1, o1, E, e0, g, l32);
+      else dw1_store<BF16, NTN, false, false>(a1, o1, E, e0, g, l32);
+    }
+  } else if (nS == 1 && outf32) {
     float* dW2h = (float*)dW2 + (size_t)h * E * DG;
     float* dW1h = (float*)dW1 + (size_t)h * DG * E;
 #pragma unroll

@@ -13,6 +13,7 @@ import pytest
 import torch
 
 from flashmlp_amd import _lib
+from oracle import emulate
 from oracle.inputs import make_inputs
 
 pytestmark = pytest.mark.gpu
@@ -160,3 +161,28 @@ def test_infinite_weights_stay_where_the_generic_kernels_have_them(H, B, D, E):
                 assert torch.equal(a.isfinite(), fin), (hex(flags), name)
                 # (HILO carries h and dZ with twice the bits: the io type's rounding apart)
                 assert _rel(a[fin], r[fin]) <= (5e-3 if flags & _lib.FMLP_DW_HILO else 1e-4), (hex(flags), name)
+
+
+@pytest.mark.parametrize("E", [1, 45, 100, 88, 130])
+def test_d256_one_row_range(E):
+    """D = 256 and at most 32 rows: one program per E tile writes dW1 and dW2 themselves (no partials), as
+    vectors where E % 4 == 0 and else element by element. The unrounded sums against the generic kernels,
+    the io-dtype outputs bitwise the rounding of those sums, guards untouched."""
+    H, B, D, dt, act = 3, 28, 256, torch.bfloat16, "silu"
+    print(f"[odd E] one row range H={H} B={B} D={D} E={E}", flush=True)
+    L = _lib.lib()
+    x, w1, w2, do = (t.cuda() for t in make_inputs(H, B, D, E, dt, seed=E))
+    f32 = _lib.FMLP_OUT_F32
+    # (E % 8 == 0 needs no workspace for kernels of its own: the oracle below bounds that call as well)
+    gen = _bwd(x, w1, w2, do, act, f32, 0, torch.float32)
+    for flags in (0, _lib.FMLP_BWD_RECOMPUTE, _lib.FMLP_BWD_NO_DX):
+        n = L.fmlp_bwd_workspace_bytes(H, B, D, E, _DT[dt] | f32 | flags)
+        own = _bwd(x, w1, w2, do, act, f32 | flags, n, torch.float32)
+        io = _bwd(x, w1, w2, do, act, flags, n, dt)
+        for name, a, r, o in zip(("dx", "dw1", "dw2"), own, gen, io):
+            if a is not None:
+                assert _rel(a, r) <= 1e-4, (hex(flags), name)
+                assert torch.equal(o, a.to(dt)), (hex(flags), name)
+    ref = emulate.emu_bwd(*(t.cpu() for t in (x, w1, w2, do)), act, dt, round_out=False)
+    for name, a, r in zip(("dx", "dw1", "dw2"), gen, ref):
+        assert _rel(a.cpu(), r) <= 1e-4, name
